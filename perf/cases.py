@@ -19,7 +19,6 @@ Kinds of case:
 * ``affine``: logdet of A + tB for a general B (one recurrence per t).
 * ``gauss``: Golub-Kahn on a rectangular sparse Gaussian matrix.
 * ``dense``: a dense symmetric matrix.
-* ``batch``: many matrices of uneven size in one ``slq_batch`` call.
 * ``train``: training of the learned surrogate (full-batch Adam steps).
 """
 
@@ -30,7 +29,6 @@ import scipy.sparse
 import torch
 
 import imate_amd
-from imate_amd.batch import slq_batch
 from imate_amd.linear_operator import AffineMatrixFunction, Matrix
 from imate_amd.sample_matrices import CorrelationFamily
 from imate_amd.surrogate import LogdetSurrogate, init_params
@@ -89,10 +87,9 @@ def listed():
         {'name': 'gauss_65k_16k', 'kind': 'gauss', 'rows': 65536,
          'n': 16384, 'k': 164, 'm': 30, 'low': 64, 'high': 64,
          'dtype': 'float64'},
-        # many problems of uneven size in one call
-        {'name': 'batch_12', 'kind': 'batch', 'count': 12, 'nmin': 1000,
-         'nmax': 40000, 'k': 40, 'm': 30, 'low': 64, 'high': 64,
-         'dtype': 'float64'},
+        # a dense covariance matrix, odd size
+        {'name': 'dense_6k', 'kind': 'dense', 'n': 6001, 'm': 30, 'low': 64,
+         'high': 64, 'dtype': 'float64'},
         # training of the surrogate over (length scale, t)
         {'name': 'train_2000', 'kind': 'train', 'points': 2000, 'steps': 100},
     ]
@@ -104,8 +101,7 @@ def _log_int(rng, a, b):
 
 def draw(rng):
     kind = rng.choice(['sparse', 'sparse', 'sparse', 'sparse', 'toeplitz',
-                       'shifts', 'affine', 'gauss', 'batch', 'dense',
-                       'train'])
+                       'shifts', 'affine', 'gauss', 'dense', 'train'])
     samples = rng.choice([24, 50, 64, 100, 128])
     m = rng.randint(10, 45)
     if kind == 'sparse':
@@ -141,10 +137,6 @@ def draw(rng):
     if kind == 'gauss':
         return {'kind': kind, 'rows': _log_int(rng, 4000, 70000),
                 'n': _log_int(rng, 1000, 16000), 'k': rng.randint(20, 160),
-                'm': m, 'low': 64, 'high': 64, 'dtype': 'float64'}
-    if kind == 'batch':
-        return {'kind': kind, 'count': rng.randint(3, 12), 'nmin': 1000,
-                'nmax': _log_int(rng, 5000, 40000), 'k': rng.randint(20, 50),
                 'm': m, 'low': 64, 'high': 64, 'dtype': 'float64'}
     if kind == 'dense':
         return {'kind': kind, 'n': _log_int(rng, 200, 5000), 'm': m,
@@ -275,13 +267,6 @@ def _params(case):
     return numpy.logspace(-2, 1, case['q'])
 
 
-def _sizes(case):
-    """Sizes of a batch: log-uniform steps from nmin to nmax, made odd."""
-    s = numpy.exp(numpy.linspace(math.log(case['nmin']),
-                                 math.log(case['nmax']), case['count']))
-    return [int(x) | 1 for x in s]
-
-
 def _inputs(case, seed):
     """The case's matrices on the GPU: CSR triples or a dense tensor."""
     gen = _generator(seed)
@@ -295,9 +280,6 @@ def _inputs(case, seed):
         return [_gauss(case['rows'], case['n'], case['k'], gen)]
     if kind == 'dense':
         return [_dense(case['n'], gen)]
-    if kind == 'batch':
-        return [_correlation(_points(n, gen), case['k'])
-                for n in _sizes(case)]
     return [_correlation(_points(case['n'], gen), case['k'])]
 
 
@@ -325,12 +307,6 @@ def prepare(case, seed):
     dt = case['dtype']
     if kind == 'dense':
         state['A'] = Matrix(ins[0].cpu().numpy())
-    elif kind == 'batch':
-        state['A'] = [Matrix(_scipy(c, (n, n), dt))
-                      for c, n in zip(ins, _sizes(case))]
-        for M in state['A']:
-            M.get_linear_operator(gpu=True)
-        return state
     elif kind == 'gauss':
         state['A'] = Matrix(_scipy(ins[0], (case['rows'], case['n']), dt))
     else:
@@ -354,12 +330,6 @@ def run(state):
         s = state['surrogate']
         s.train(state['data'], steps=(case['steps'],), lr=(3e-3,))
         return {'params': s.params, 'losses': s.losses}
-    if kind == 'batch':
-        trace, info = slq_batch(state['A'], func='log',
-                                lanczos_degree=case['m'],
-                                num_samples=case['high'], seed=state['seed'])
-        return {'trace': trace, 'error': info['error'],
-                'samples': info['samples']}
     func = FUNCS[case.get('func', 'logdet')]
     gram = kind == 'gauss' or case.get('gram', False)
     fixed = case['low'] == case['high']
@@ -391,38 +361,34 @@ def work(case):
     blocks = -(-case['high'] // 64)
     vb = 4 if case['dtype'] == 'float32' or \
         case.get('precision') == 'mixed' else 8
-    sizes = _sizes(case) if kind == 'batch' else [case['n']]
-    total = {'bytes': 0.0, 'flops': 0.0}
-    for n in sizes:
-        rows = case.get('rows', n)
-        if kind == 'toeplitz':
-            nnz = 3.0 * n
-        elif kind == 'dense':
-            nnz = float(n) * n
-        elif kind == 'affine':
-            nnz = float(n) * (case['k'] + case['kb'])
-        elif kind == 'gauss':
-            nnz = float(rows) * case['k']
-        else:
-            nnz = float(n) * case['k']
-        entry = vb if kind == 'dense' else vb + 4
-        gram = kind == 'gauss' or case.get('gram', False)
-        runs = case['q'] if kind == 'affine' else 1
-        sides = 2 if gram else 1
-        vec = (n + rows) if gram else n
-        step_b = sides * nnz * entry + 3.0 * vec * 64 * vb
-        step_f = sides * 2.0 * nnz * 64
-        reo = case.get('ortho', 0)
-        steps = m * blocks * runs
-        total['bytes'] += steps * step_b
-        total['flops'] += steps * step_f
-        if reo:
-            depth = sum(j if reo < 0 else min(j, reo)
-                        for j in range(1, m + 1)) * blocks
-            total['bytes'] += 2.0 * depth * vec * 64 * vb
-            total['flops'] += 4.0 * depth * vec * 64
-        if case.get('handed') == 'array':
-            total['bytes'] += nnz * entry
+    n = case['n']
+    rows = case.get('rows', n)
+    if kind == 'toeplitz':
+        nnz = 3.0 * n
+    elif kind == 'dense':
+        nnz = float(n) * n
+    elif kind == 'affine':
+        nnz = float(n) * (case['k'] + case['kb'])
+    elif kind == 'gauss':
+        nnz = float(rows) * case['k']
+    else:
+        nnz = float(n) * case['k']
+    entry = vb if kind == 'dense' else vb + 4
+    gram = kind == 'gauss' or case.get('gram', False)
+    runs = case['q'] if kind == 'affine' else 1
+    sides = 2 if gram else 1
+    vec = (n + rows) if gram else n
+    steps = m * blocks * runs
+    total = {'bytes': steps * (sides * nnz * entry + 3.0 * vec * 64 * vb),
+             'flops': steps * sides * 2.0 * nnz * 64}
+    reo = case.get('ortho', 0)
+    if reo:
+        depth = sum(j if reo < 0 else min(j, reo)
+                    for j in range(1, m + 1)) * blocks
+        total['bytes'] += 2.0 * depth * vec * 64 * vb
+        total['flops'] += 4.0 * depth * vec * 64
+    if case.get('handed') == 'array':
+        total['bytes'] += nnz * entry
     return total
 
 
@@ -604,16 +570,6 @@ def exact(case, seed):
     sd = int(seed) % (1 << 30)
     if case['dtype'] == 'float32':
         ins = [(a, b, c.float().double()) for a, b, c in ins]
-    if kind == 'batch':
-        tr, er, sa = [], [], []
-        for M, n in zip(ins, _sizes(case)):
-            S = _samples(_matvec(M, (n, n)), n, case, sd, 'logdet', 1, [0.0])
-            t, e, s, _ = _statistics(S[:, 0], case['low'], True)
-            tr.append(t)
-            er.append(e)
-            sa.append(s)
-        return {'trace': numpy.array(tr), 'error': numpy.array(er),
-                'samples': numpy.array(sa)}
     n = case['n']
     func, p = case.get('func', 'logdet'), case.get('p', 1)
     fixed = case['low'] == case['high']
