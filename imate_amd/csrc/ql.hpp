@@ -1,7 +1,7 @@
-// Device and host implicit-QL eigensolve and Gauss quadrature of a Lanczos
-// tridiagonal or Golub-Kahn bidiagonal, and the matrix functions, in FP64.
-// Included by quadrature.hip (one probe per GPU thread) and by host_slq.cpp
-// (the CPU path), so both run the same arithmetic.
+// Implicit-QL eigensolve and Gauss quadrature of a Lanczos tridiagonal or
+// Golub-Kahn bidiagonal, and the matrix functions, in FP64. Included by
+// host_slq.cpp (the CPU path's solver) and by quadrature.hip, which runs it
+// for the matrices past its divide-and-conquer solver's size.
 #pragma once
 
 #include <cfloat>

@@ -11,51 +11,191 @@
 // the Ritz values of A + t_0 I shifted by t_j - t_0 (c_trace_estimator.cpp:
 // 564-594, c_affine_matrix_function.cpp get_eigenvalue).
 //
-// Here each thread owns one probe and runs the implicit QL algorithm with
-// Wilkinson-type shifts (Bowdler, Martin, Reinsch & Wilkinson 1968; the
-// EISPACK tql2 scheme) on its tridiagonal, accumulating only the first row of
-// the eigenvector matrix (Golub & Welsch 1969): every plane rotation of QL is
-// applied to that row alone, O(k) per rotation. The bidiagonal case is solved
-// as the 2k x 2k Golub-Kahan tridiagonal with zero diagonal and off-diagonal
-// (alpha_0, beta_0, alpha_1, ..., alpha_{k-1}), whose eigenvalues are
-// +-sigma_i; the eigenvector of +sigma_i is (v_0, u_0, v_1, u_1, ...)/sqrt(2),
-// so tau_i^2 = 2 z_0^2. The k largest eigenvalues are taken.
+// Here a workgroup owns one probe and solves its tridiagonal by
+// divide-and-conquer (dc.hpp), carrying only the first and last rows of the
+// eigenvectors of each block. The bidiagonal case is solved as the 2k x 2k
+// Golub-Kahan tridiagonal with zero diagonal and off-diagonal (alpha_0,
+// beta_0, alpha_1, ..., alpha_{k-1}), whose eigenvalues are +-sigma_i; the
+// eigenvector of +sigma_i is (v_0, u_0, v_1, u_1, ...)/sqrt(2), so tau_i^2 =
+// 2 z_0^2. The k largest eigenvalues are taken. Matrices past kDcMaxRows
+// rows (their work arrays would not fit the LDS) run the implicit QL of
+// ql.hpp, the host path's solver, one probe per workgroup.
 //
-// Per-thread arrays live in LDS, interleaved by thread.
+// What bounds it: latency. One probe's QL is a serial chain of about
+// 0.65 m^2 plane rotations of some hundred dependent FP64 operations each
+// (measured 266 us at m = 20, 525 at 30, 1840 at 60, the same for one probe
+// or 64), while divide-and-conquer is log2(m) merges whose roots are
+// independent threads: 41, 54 and 77 us. The matrix function at the
+// nodes is spread over the threads too: by node for a few inquiries, by
+// inquiry for many (256 inquiries at m = 30 took 2.9 ms in one thread per
+// probe).
 
 #include <cfloat>
 #include <cmath>
 
 #include "slq_internal.hpp"
 #include "ql.hpp"
+#include "dc.hpp"
 
 namespace slq {
 
 namespace {
 
-// Probes per workgroup: one. Each probe's QL is a chain of dependent FP64
-// operations; a wavefront per probe (64 of them, on as many compute units)
-// runs no lane in lockstep with another probe's different iteration counts:
-// measured 434 against 522 us at lanczos_degree 30 and 1.62 against 2.04 ms
-// at 60 for 16 probes per workgroup (8 and 4 per workgroup: no better).
-constexpr int kQuadThreads = 1;
+// Rows up to which the divide-and-conquer work arrays are taken: 92 bytes a
+// row, 92 KB of the CU's 160 KB of LDS.
+constexpr int kDcMaxRows = 1024;
+// Inquiries up to which the threads share the nodes of one inquiry.
+constexpr int kFewInquiries = 8;
 
-__global__ __launch_bounds__(64) void quadrature_kernel(QuadArgs a)
+// Lane l's value from the lane that Ctrl names (row operations within 16
+// lanes; every lane of the row is read, so all of its lanes must be active).
+template <int Ctrl>
+__device__ __forceinline__ int dpp(int x)
+{
+    return __builtin_amdgcn_update_dpp(0, x, Ctrl, 0xf, 0xf, true);
+}
+
+template <int Ctrl>
+__device__ __forceinline__ double dpp(double x)
+{
+    const uint64_t u = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = (uint32_t) dpp<Ctrl>((int) (uint32_t) u);
+    const uint32_t hi = (uint32_t) dpp<Ctrl>((int) (uint32_t) (u >> 32));
+    return __builtin_bit_cast(double, ((uint64_t) hi << 32) | lo);
+}
+
+struct Workgroup {
+    int tid, nt;
+    __device__ __forceinline__ void sync() const { __syncthreads(); }
+    // Sum / product over P = 1, 2, 4, 8 or 16 neighbouring lanes, the same
+    // value in each: lane ^ 1, ^ 2 (quad permutes), then the mirrored half
+    // row and row, whose lanes already agree within quads and halves.
+    template <int P, typename T>
+    __device__ __forceinline__ T sum(T x) const
+    {
+        if constexpr (P > 1) x += dpp<0xB1>(x);
+        if constexpr (P > 2) x += dpp<0x4E>(x);
+        if constexpr (P > 4) x += dpp<0x141>(x);
+        if constexpr (P > 8) x += dpp<0x140>(x);
+        return x;
+    }
+    template <int P>
+    __device__ __forceinline__ double prod(double x) const
+    {
+        if constexpr (P > 1) x *= dpp<0xB1>(x);
+        if constexpr (P > 2) x *= dpp<0x4E>(x);
+        if constexpr (P > 4) x *= dpp<0x141>(x);
+        if constexpr (P > 8) x *= dpp<0x140>(x);
+        return x;
+    }
+};
+
+template <int NT, int P>
+__global__ __launch_bounds__(NT) void quadrature_dc_kernel(QuadArgs a)
 {
     extern __shared__ double sh[];
-    const int t = threadIdx.x;
-    const int p = blockIdx.x * kQuadThreads + t;
+    const int p = blockIdx.x;
+    const Workgroup g{(int) threadIdx.x, NT};
+    const int k = a.sizes[p] > 0 ? a.sizes[p] : a.m;
+    const int K = a.gram ? 2 * k : k;
+    const DcWork w = dc_carve(sh, K);
+    const double* al = a.alpha + p;
+    const double* be = a.beta + p;
+    for (int i = g.tid; i < k; i += NT)
+    {
+        const double ai = al[(int64_t) i * kBlock];
+        const double bi = i < k - 1 ? be[(int64_t) i * kBlock] : 0.0;
+        if (a.gram)
+        {
+            w.d[2 * i] = 0.0;
+            w.d[2 * i + 1] = 0.0;
+            w.e[2 * i] = ai;
+            w.e[2 * i + 1] = bi;
+        }
+        else
+        {
+            w.d[i] = ai;
+            w.e[i] = bi;
+        }
+    }
+    g.sync();
+    const bool ok = dc_first_row<P>(g, w, K);
+    // nodes and weights in order: ascending, or the k largest singular
+    // values descending
+    double* th = w.ds;
+    double* tau = w.zs;
+    if (ok)
+        for (int i = g.tid; i < K; i += NT)
+        {
+            const double di = w.d[i];
+            int r = 0;
+            for (int j = 0; j < K; ++j)
+            {
+                const double dj = w.d[j];
+                r += ((a.gram ? dj > di : dj < di) || (dj == di && j < i)) ? 1 : 0;
+            }
+            if (r < k)
+            {
+                th[r] = a.gram ? di * di : di;
+                tau[r] = a.gram ? sqrt(2.0) * w.f[i] : w.f[i];
+            }
+        }
+    g.sync();
+    if (a.theta_out)
+        for (int i = g.tid; i < a.m; i += NT)
+        {
+            a.theta_out[(size_t) p * a.m + i] = ok && i < k ? th[i] : (i < k ? NAN : 0.0);
+            a.tau_out[(size_t) p * a.m + i] = ok && i < k ? tau[i] : (i < k ? NAN : 0.0);
+        }
+    const int jn = a.shift ? a.q : 1;
+    const double t0 = a.shift ? a.params[0] : 0.0;
+    double* out = a.samples + (size_t) p * a.q_stride;
+    auto term = [&](int i, double tj) {
+        const double x = a.shift ? (th[i] - t0) + tj : th[i];
+        // a node of zero weight adds nothing, whatever f is there
+        const double t = tau[i];
+        return t == 0.0 ? 0.0 : t * t * ffunc(a.func, a.fp, fpow(x, a.exponent));
+    };
+    if (jn > kFewInquiries)
+    {
+        for (int j = g.tid; j < jn; j += NT)
+        {
+            const double tj = a.params[j];
+            double sum = 0.0;
+            if (ok)
+                for (int i = 0; i < k; ++i) sum += term(i, tj);
+            out[j] = ok ? a.n * sum : NAN;
+        }
+        return;
+    }
+    for (int j = 0; j < jn; ++j)
+    {
+        const double tj = a.shift ? a.params[j] : 0.0;
+        double sum = 0.0;
+        if (ok)
+            for (int i = g.tid; i < k; i += NT) sum += term(i, tj);
+        for (int s = 1; s < kWave; s <<= 1) sum += __shfl_xor(sum, s);
+        if (NT > kWave)
+        {
+            double* red = w.fs;
+            if (g.tid % kWave == 0) red[g.tid / kWave] = sum;
+            g.sync();
+            sum = 0.0;
+            for (int v = 0; v < NT / kWave; ++v) sum += red[v];
+            g.sync();
+        }
+        if (g.tid == 0) out[a.shift ? j : a.j_out] = ok ? a.n * sum : NAN;
+    }
+}
+
+// One probe per workgroup and thread, for matrices past kDcMaxRows rows.
+__global__ __launch_bounds__(64) void quadrature_ql_kernel(QuadArgs a)
+{
+    extern __shared__ double sh[];
+    const int p = blockIdx.x;
     const int K2 = a.gram ? 2 * a.m : a.m;
-    double* d = sh;
-    double* e = sh + (size_t) K2 * kQuadThreads;
-    double* z = sh + (size_t) 2 * K2 * kQuadThreads;
-    const int S = kQuadThreads;
-    d += t;
-    e += t;
-    z += t;
-    if (p >= a.count) return;
-    quadrature_one(a, a.alpha + p, a.beta + p, kBlock, a.sizes[p], d, e, z, S,
-                   a.samples + (size_t) p * a.q_stride,
+    quadrature_one(a, a.alpha + p, a.beta + p, kBlock, a.sizes[p], sh, sh + K2,
+                   sh + (size_t) 2 * K2, 1, a.samples + (size_t) p * a.q_stride,
                    a.theta_out ? a.theta_out + (size_t) p * a.m : nullptr,
                    a.tau_out ? a.tau_out + (size_t) p * a.m : nullptr);
 }
@@ -89,17 +229,35 @@ int run_quadrature(hipStream_t s, const double* alpha, const double* beta,
     a.theta_out = theta_dev;
     a.tau_out = tau_dev;
     const int K2 = gram ? 2 * m : m;
-    const size_t lds = sizeof(double) * 3 * (size_t) K2 * kQuadThreads;
+    if (K2 <= kDcMaxRows)
+    {
+        const size_t lds = (size_t) K2 * (kDcDoubles * sizeof(double) + kDcInts * sizeof(int));
+        // 8 threads a row while 512 threads (256 up to 32 rows, for cheaper
+        // barriers: 41 against 45 us at m = 20, 54 against 62 at 30) cover
+        // them, then fewer: 77 us at 60 rows and 166 at 120 (gram, m = 60)
+        // against 81 and 216 with 256 threads
+        auto kern = quadrature_dc_kernel<512, 1>;
+        if (K2 <= 32) kern = quadrature_dc_kernel<256, 8>;
+        else if (K2 <= 64) kern = quadrature_dc_kernel<512, 8>;
+        else if (K2 <= 128) kern = quadrature_dc_kernel<512, 4>;
+        const int nt = K2 <= 32 ? 256 : 512;
+        if (lds > 64 * 1024)
+            SLQ_CHECK(hipFuncSetAttribute((const void*) kern,
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
+        hipLaunchKernelGGL(kern, dim3(count), dim3(nt), lds, s, a);
+        SLQ_CHECK(hipGetLastError());
+        return SLQ_OK;
+    }
+    const size_t lds = sizeof(double) * 3 * (size_t) K2;
     if (lds > 160 * 1024)
     {
         set_error("lanczos_degree %d too large for the device eigensolver", m);
         return SLQ_E_ARG;
     }
-    const int grid = (count + kQuadThreads - 1) / kQuadThreads;
     if (lds > 64 * 1024)
-        SLQ_CHECK(hipFuncSetAttribute((const void*) quadrature_kernel,
+        SLQ_CHECK(hipFuncSetAttribute((const void*) quadrature_ql_kernel,
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int) lds));
-    hipLaunchKernelGGL(quadrature_kernel, dim3(grid), dim3(kQuadThreads), lds, s, a);
+    hipLaunchKernelGGL(quadrature_ql_kernel, dim3(count), dim3(1), lds, s, a);
     SLQ_CHECK(hipGetLastError());
     return SLQ_OK;
 }

@@ -397,7 +397,8 @@ int slq_copy_bandwidth(int64_t bytes, int32_t iters, double* ms_per_launch);
  * one multiply of the operator per block and step, rows split over
  * num_threads worker threads with reductions summed in a fixed order (the
  * result does not depend on the thread count). Same probes as slq_estimate
- * (thread-0 stream), same eigensolve and quadrature code as the device path.
+ * (thread-0 stream) and the same quadrature as the device path, with an
+ * implicit-QL eigensolve (the device solves by divide-and-conquer).
  * No HIP call: usable on a machine without a GPU. Host handles copy the
  * caller's arrays. */
 
