@@ -59,7 +59,7 @@ int hip_status(hipError_t e, const char* what, const char* file, int line)
 
 // ---------------------------------------------------------------- storage
 
-static void free_tiles(DevTiles& t)
+void free_tiles(DevTiles& t)
 {
     if (t.ptr) (void) hipFree(t.ptr);
     if (t.cols) (void) hipFree(t.cols);
@@ -109,19 +109,6 @@ int Workspace::reserve(size_t need)
 
 // ---------------------------------------------------------------- tiles
 
-// Position of the value (slab, row r) in the tile value array. R = 8: slab
-// by slab, R values each. R = 16 (matrix-core layout): a group of four
-// slabs is one MFMA A operand, lane l = 16 (slab % 4) + r; the two groups of
-// each eight slabs are interleaved per lane ([slab / 8][lane][2]) so that a
-// lane loads both of its A values with one access.
-size_t tile_slot(int R, int64_t slab, int r)
-{
-    if (R != 16) return (size_t) slab * R + r;
-    const int64_t pair = slab >> 3, half = (slab >> 2) & 1;
-    const int lane = 16 * (int) (slab & 3) + r;
-    return (size_t) pair * 128 + (size_t) lane * 2 + (size_t) half;
-}
-
 int build_tiles(int64_t nrows, int64_t ncols, const int64_t* indptr,
                 const int32_t* indices, const void* data, int dtype, int R,
                 double min_density, DevTiles& out, std::vector<int32_t>* src_host)
@@ -167,10 +154,9 @@ int build_tiles(int64_t nrows, int64_t ncols, const int64_t* indptr,
         for (int64_t row = t * R; row < r1; ++row)
         {
             const int r = (int) (row - t * R);
-            const int32_t* p = cb;
             for (int64_t k = indptr[row]; k < indptr[row + 1]; ++k)
             {
-                p = std::lower_bound(p, ce, indices[k]);
+                const int32_t* p = std::lower_bound(cb, ce, indices[k]);
                 const size_t slot = tile_slot(R, p - cols.data(), r);
                 if (!data)
                     ;
@@ -213,6 +199,38 @@ int build_tiles(int64_t nrows, int64_t ncols, const int64_t* indptr,
         else src_host->clear();
     }
     return SLQ_OK;
+}
+
+// Non-zeros up to which a matrix given in host memory is tiled there: the
+// host takes about 27 ns a non-zero (0.8 ms at 30,000), the device build
+// 0.12 ms for its launches, allocations and copies even of a tiny matrix.
+constexpr int64_t kHostTileNnz = 4096;
+
+// Tiled form of a device CSR whose column order is known (strict): on the
+// device, else on the host from a copy.
+static int tiles_of(hipStream_t s, const DevCSR& c, int R, DevTiles& out)
+{
+    if (c.strict)
+    {
+        TileStatus st;
+        SLQ_TRY(device_tiles(s, c, nullptr, R, 0.25, out, nullptr, nullptr, st));
+        if (st.built) return SLQ_OK;
+    }
+    const size_t vb = c.dtype == SLQ_F64 ? 8 : 4;
+    std::vector<int64_t> ip(c.nrows + 1);
+    std::vector<int32_t> ix(c.nnz > 0 ? c.nnz : 1);
+    std::vector<char> dv(vb * (c.nnz > 0 ? c.nnz : 1));
+    SLQ_CHECK(hipStreamSynchronize(s));
+    SLQ_CHECK(hipMemcpy(ip.data(), c.indptr, sizeof(int64_t) * (c.nrows + 1),
+                        hipMemcpyDeviceToHost));
+    if (c.nnz > 0)
+    {
+        SLQ_CHECK(hipMemcpy(ix.data(), c.indices, sizeof(int32_t) * c.nnz,
+                            hipMemcpyDeviceToHost));
+        SLQ_CHECK(hipMemcpy(dv.data(), c.data, vb * c.nnz, hipMemcpyDeviceToHost));
+    }
+    return build_tiles(c.nrows, c.ncols, ip.data(), ix.data(), dv.data(), c.dtype, R, 0.25,
+                       out);
 }
 
 PairTiles::~PairTiles()
@@ -273,10 +291,69 @@ bool union_pattern(int64_t nrows, const std::vector<int64_t>& ipa,
     return true;
 }
 
+// The pair tiles on the host, from device copies of both patterns (rows in
+// any order).
+int host_pair_tiles(slq_op* op, const DevCSR& ca, const DevCSR& cb, int64_t n, int R,
+                    PairTiles& ab)
+{
+    SLQ_CHECK(hipStreamSynchronize(op->stream));   // transposes built on it
+    std::vector<int64_t> ipa(n + 1), ipb(n + 1), ipu;
+    std::vector<int32_t> ixa(ca.nnz > 0 ? ca.nnz : 1), ixb(cb.nnz > 0 ? cb.nnz : 1), ixu,
+        ka, kb;
+    SLQ_CHECK(hipMemcpy(ipa.data(), ca.indptr, sizeof(int64_t) * (n + 1),
+                        hipMemcpyDeviceToHost));
+    SLQ_CHECK(hipMemcpy(ipb.data(), cb.indptr, sizeof(int64_t) * (n + 1),
+                        hipMemcpyDeviceToHost));
+    if (ca.nnz > 0)
+        SLQ_CHECK(hipMemcpy(ixa.data(), ca.indices, sizeof(int32_t) * ca.nnz,
+                            hipMemcpyDeviceToHost));
+    if (cb.nnz > 0)
+        SLQ_CHECK(hipMemcpy(ixb.data(), cb.indices, sizeof(int32_t) * cb.nnz,
+                            hipMemcpyDeviceToHost));
+    if (!union_pattern(n, ipa, ixa, ipb, ixb, ipu, ixu, ka, kb)) return SLQ_OK;
+    std::vector<int32_t> src;
+    DevTiles t;
+    SLQ_TRY(build_tiles(n, ca.ncols, ipu.data(), ixu.data(), nullptr, ca.dtype, R, 0.25, t,
+                        &src));
+    if (t.R == 0) return SLQ_OK;
+    if (src.empty())
+    {
+        free_tiles(t);
+        return SLQ_OK;
+    }
+    if (t.src)
+    {
+        (void) hipFree(t.src);
+        t.src = nullptr;
+    }
+    // slot -> union entry -> position in A's / B's values
+    std::vector<int32_t> sa(src.size()), sb(src.size());
+    for (size_t i = 0; i < src.size(); ++i)
+    {
+        sa[i] = src[i] >= 0 ? ka[src[i]] : -1;
+        sb[i] = src[i] >= 0 ? kb[src[i]] : -1;
+    }
+    hipError_t e;
+    if ((e = hipMalloc(&ab.src_a, sizeof(int32_t) * sa.size())) != hipSuccess ||
+        (e = hipMalloc(&ab.src_b, sizeof(int32_t) * sb.size())) != hipSuccess ||
+        (e = hipMemcpy(ab.src_a, sa.data(), sizeof(int32_t) * sa.size(),
+                       hipMemcpyHostToDevice)) != hipSuccess ||
+        (e = hipMemcpy(ab.src_b, sb.data(), sizeof(int32_t) * sb.size(),
+                       hipMemcpyHostToDevice)) != hipSuccess)
+    {
+        free_tiles(t);
+        if (ab.src_a) (void) hipFree(ab.src_a);
+        if (ab.src_b) (void) hipFree(ab.src_b);
+        ab.src_a = ab.src_b = nullptr;
+        return hip_status(e, "pair tile upload", __FILE__, __LINE__);
+    }
+    ab.tiles = t;
+    return SLQ_OK;
+}
+
 }  // namespace
 
-// Tiled form of A + tB (R of A's tiles), built once per affine operator on
-// the host from device copies of both patterns. Leaves op->ab.tiles.R = 0
+// Tiled form of A + tB (R of A's tiles), built once per affine operator. Leaves op->ab.tiles.R = 0
 // (the two-stream CSR SpMM) when A has no tiled form, a pattern repeats a
 // column or the union is too sparse for tiles.
 int ensure_pair_tiles(slq_op* op, bool need_f32, bool trans)
@@ -297,65 +374,21 @@ int ensure_pair_tiles(slq_op* op, bool need_f32, bool trans)
         const DevCSR& ca = trans ? A.trans : A.csr;
         const DevCSR& cb = trans ? B.trans : B.csr;
         const int64_t n = ca.nrows;
-        SLQ_CHECK(hipStreamSynchronize(op->stream));   // transposes built on it
-        std::vector<int64_t> ipa(n + 1), ipb(n + 1), ipu;
-        std::vector<int32_t> ixa(ca.nnz > 0 ? ca.nnz : 1), ixb(cb.nnz > 0 ? cb.nnz : 1), ixu,
-            ka, kb;
-        SLQ_CHECK(hipMemcpy(ipa.data(), ca.indptr, sizeof(int64_t) * (n + 1),
-                            hipMemcpyDeviceToHost));
-        SLQ_CHECK(hipMemcpy(ipb.data(), cb.indptr, sizeof(int64_t) * (n + 1),
-                            hipMemcpyDeviceToHost));
-        if (ca.nnz > 0)
-            SLQ_CHECK(hipMemcpy(ixa.data(), ca.indices, sizeof(int32_t) * ca.nnz,
-                                hipMemcpyDeviceToHost));
-        if (cb.nnz > 0)
-            SLQ_CHECK(hipMemcpy(ixb.data(), cb.indices, sizeof(int32_t) * cb.nnz,
-                                hipMemcpyDeviceToHost));
-        if (!union_pattern(n, ipa, ixa, ipb, ixb, ipu, ixu, ka, kb)) return SLQ_OK;
-        std::vector<int32_t> src;
-        DevTiles t;
-        SLQ_TRY(build_tiles(n, ca.ncols, ipu.data(), ixu.data(), nullptr, ca.dtype, R, 0.25, t,
-                            &src));
-        if (t.R == 0) return SLQ_OK;
-        if (src.empty())
+        bool built = false;
+        if (ca.strict && cb.strict)
         {
-            free_tiles(t);
-            return SLQ_OK;
+            TileStatus st;
+            SLQ_TRY(device_tiles(op->stream, ca, &cb, R, 0.25, ab.tiles, &ab.src_a, &ab.src_b,
+                                 st));
+            built = st.built;
         }
-        if (t.src)
-        {
-            (void) hipFree(t.src);
-            t.src = nullptr;
-        }
-        // slot -> union entry -> position in A's / B's values
-        std::vector<int32_t> sa(src.size()), sb(src.size());
-        for (size_t i = 0; i < src.size(); ++i)
-        {
-            sa[i] = src[i] >= 0 ? ka[src[i]] : -1;
-            sb[i] = src[i] >= 0 ? kb[src[i]] : -1;
-        }
-        hipError_t e;
-        if ((e = hipMalloc(&ab.src_a, sizeof(int32_t) * sa.size())) != hipSuccess ||
-            (e = hipMalloc(&ab.src_b, sizeof(int32_t) * sb.size())) != hipSuccess ||
-            (e = hipMemcpy(ab.src_a, sa.data(), sizeof(int32_t) * sa.size(),
-                           hipMemcpyHostToDevice)) != hipSuccess ||
-            (e = hipMemcpy(ab.src_b, sb.data(), sizeof(int32_t) * sb.size(),
-                           hipMemcpyHostToDevice)) != hipSuccess)
-        {
-            free_tiles(t);
-            if (ab.src_a) (void) hipFree(ab.src_a);
-            if (ab.src_b) (void) hipFree(ab.src_b);
-            ab.src_a = ab.src_b = nullptr;
-            return hip_status(e, "pair tile upload", __FILE__, __LINE__);
-        }
-        ab.tiles = t;
+        if (!built) SLQ_TRY(host_pair_tiles(op, ca, cb, n, R, ab));
     }
     if (need_f32 && ab.tiles.R > 0 && op->A->csr.dtype == SLQ_F64 && !ab.tiles.vals_f32)
         SLQ_CHECK(hipMalloc(&ab.tiles.vals_f32,
                             sizeof(float) * (size_t) (ab.tiles.nslabs * ab.tiles.R)));
     return SLQ_OK;
 }
-
 // ---------------------------------------------------------------- profiling
 
 void prof_begin(slq_op* op, hipEvent_t* ev)
@@ -610,6 +643,7 @@ static int build_transpose_chunked(hipStream_t s, const DevCSR& A, DevCSR& T)
     T.nnz = nnz;
     T.dtype = A.dtype;
     T.sorted = true;   // each chunk is sorted stably by column: rows ascend
+    T.strict = A.strict;
     SLQ_CHECK(hipMalloc(&T.indptr, sizeof(int64_t) * (T.nrows + 1)));
     SLQ_CHECK(hipMalloc(&T.indices, sizeof(int32_t) * nnz));
     SLQ_CHECK(hipMalloc(&T.data, vb * nnz));
@@ -757,6 +791,7 @@ int build_transpose(hipStream_t s, const DevCSR& A, DevCSR& T)
     T.nnz = nnz;
     T.dtype = A.dtype;
     T.sorted = true;   // stable sort by column: the rows of A ascend
+    T.strict = A.strict;
     SLQ_CHECK(hipMalloc(&T.indptr, sizeof(int64_t) * (T.nrows + 1)));
     SLQ_CHECK(hipMalloc(&T.indices, sizeof(int32_t) * (nnz > 0 ? nnz : 1)));
     SLQ_CHECK(hipMalloc(&T.data, vb * (nnz > 0 ? nnz : 1)));
@@ -1085,23 +1120,8 @@ int prepare(slq_op* op, int gram, int precision)
         }
         if (!op->A->trans_tiles_tried && op->A->tiles.R > 0)
         {
-            // tiled form of A^T, built on the host from the device transpose
             op->A->trans_tiles_tried = true;
-            const DevCSR& T = op->A->trans;
-            const size_t vb = T.dtype == SLQ_F64 ? 8 : 4;
-            std::vector<int64_t> ip(T.nrows + 1);
-            std::vector<int32_t> ix(T.nnz > 0 ? T.nnz : 1);
-            std::vector<char> dv(vb * (T.nnz > 0 ? T.nnz : 1));
-            SLQ_CHECK(hipMemcpy(ip.data(), T.indptr, sizeof(int64_t) * (T.nrows + 1),
-                                hipMemcpyDeviceToHost));
-            if (T.nnz > 0)
-            {
-                SLQ_CHECK(hipMemcpy(ix.data(), T.indices, sizeof(int32_t) * T.nnz,
-                                    hipMemcpyDeviceToHost));
-                SLQ_CHECK(hipMemcpy(dv.data(), T.data, vb * T.nnz, hipMemcpyDeviceToHost));
-            }
-            SLQ_TRY(build_tiles(T.nrows, T.ncols, ip.data(), ix.data(), dv.data(), T.dtype,
-                                op->A->tiles.R, 0.25, op->A->trans_tiles));
+            SLQ_TRY(tiles_of(op->stream, op->A->trans, op->A->tiles.R, op->A->trans_tiles));
         }
         if (op->kind == OP_AFFINE_B && !op->B->has_trans)
         {
@@ -1724,23 +1744,29 @@ int slq_op_create_csr(int64_t nrows, int64_t ncols, int64_t nnz,
         return SLQ_E_ARG;
     }
     // Every kernel gathers X[column]: reject pointers or columns out of range
-    // here rather than let a kernel read outside its buffers.
+    // here rather than let a kernel read outside its buffers. The columns are
+    // looked over on the device; on the host only where that is not done, or
+    // to name the column it found.
     for (int64_t r = 0; r < nrows; ++r)
         if (indptr[r + 1] < indptr[r])
         {
             set_error("slq_op_create_csr: indptr decreases at row %lld", (long long) r);
             return SLQ_E_ARG;
         }
-    for (int64_t k = 0; k < nnz; ++k)
-        if (indices[k] < 0 || (int64_t) indices[k] >= ncols)
-        {
-            set_error("slq_op_create_csr: column index %d out of range at %lld",
-                      indices[k], (long long) k);
-            return SLQ_E_ARG;
-        }
+    auto check_columns = [&]() -> int {
+        for (int64_t k = 0; k < nnz; ++k)
+            if (indices[k] < 0 || (int64_t) indices[k] >= ncols)
+            {
+                set_error("slq_op_create_csr: column index %d out of range at %lld",
+                          indices[k], (long long) k);
+                return SLQ_E_ARG;
+            }
+        return SLQ_OK;
+    };
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1)
     {
+        SLQ_TRY(check_columns());
         set_error("no HIP device found");
         return SLQ_E_NODEVICE;
     }
@@ -1757,16 +1783,9 @@ int slq_op_create_csr(int64_t nrows, int64_t ncols, int64_t nnz,
     c.ncols = ncols;
     c.nnz = nnz;
     c.dtype = dtype;
-    c.sorted = true;
-    for (int64_t r = 0; r < nrows && c.sorted; ++r)
-        for (int64_t k = indptr[r] + 1; k < indptr[r + 1]; ++k)
-            if (indices[k] < indices[k - 1])
-            {
-                c.sorted = false;
-                break;
-            }
     const size_t vb = dtype == SLQ_F64 ? 8 : 4;
     auto fail = [&](int code) {
+        if (op->stream) (void) hipStreamDestroy(op->stream);
         delete op;
         return code;
     };
@@ -1788,10 +1807,32 @@ int slq_op_create_csr(int64_t nrows, int64_t ncols, int64_t nnz,
         // 0 (CSR only)
         const char* env = std::getenv("SLQ_TILE_ROWS");
         const int R = env ? std::atoi(env) : 16;
-        if (R == 8 || R == 16)
+        TileStatus st;
+        st.want_tiles = R == 8 || R == 16;
+        int r = SLQ_OK;
+        if (nnz > kHostTileNnz)
+            r = device_tiles(op->stream, c, nullptr, R, 0.25, op->A->tiles, nullptr, nullptr,
+                             st);
+        if (r == SLQ_OK && (!st.checked || st.bad_column)) r = check_columns();
+        if (r != SLQ_OK) return fail(r);
+        if (st.checked)
         {
-            int r = build_tiles(nrows, ncols, indptr, indices, data, dtype, R, 0.25,
-                                op->A->tiles);
+            c.sorted = st.sorted;
+            c.strict = st.strict;
+        }
+        else
+        {
+            c.sorted = c.strict = true;
+            for (int64_t i = 0; i < nrows && c.sorted; ++i)
+                for (int64_t k = indptr[i] + 1; k < indptr[i + 1]; ++k)
+                {
+                    if (indices[k] < indices[k - 1]) c.sorted = false;
+                    if (indices[k] <= indices[k - 1]) c.strict = false;
+                }
+        }
+        if (st.want_tiles && !st.built)
+        {
+            r = build_tiles(nrows, ncols, indptr, indices, data, dtype, R, 0.25, op->A->tiles);
             if (r != SLQ_OK) return fail(r);
         }
     }
@@ -1938,7 +1979,7 @@ int slq_op_create_sparse_gaussian(int64_t nrows, int64_t ncols, int32_t per_row,
     c.ncols = ncols;
     c.nnz = nrows * per_row;
     c.dtype = dtype;
-    c.sorted = true;   // one entry per column stratum, strata in order
+    c.sorted = c.strict = true;   // one entry per column stratum, strata in order
     const size_t vb = dtype == SLQ_F64 ? 8 : 4;
     auto fail = [&](int code) {
         delete op;

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <cstring>
 #include <memory>
 #include <vector>
 
@@ -62,6 +63,7 @@ struct DevCSR {
     int32_t* indices = nullptr;
     void* data = nullptr;
     bool sorted = false;   // column indices non-decreasing within every row
+    bool strict = false;   // sorted, and no row repeats a column
 };
 
 // Row-tiled "column slab" form of a CSR matrix for the SpMM. Rows are grouped
@@ -121,11 +123,44 @@ struct MatrixStore {
     ~MatrixStore();
 };
 
-// Host construction of the tiled form (R in {8, 16}); returns R = 0 in
-// `out` when fewer than `min_density` of the slab entries would be non-zero.
-// With R = 16 every tile's slab count is padded to a multiple of eight (zero
-// slabs repeating the tile's last column) and the values are laid out as the
-// matrix-core SpMM's operands (tile_slot in capi.hip).
+// Position of the value (slab, row r) in the tile value array. R = 8: slab
+// by slab, R values each. R = 16 (matrix-core layout): a group of four
+// slabs is one MFMA A operand, lane l = 16 (slab % 4) + r; the two groups of
+// each eight slabs are interleaved per lane ([slab / 8][lane][2]) so that a
+// lane loads both of its A values with one access.
+__host__ __device__ inline size_t tile_slot(int R, int64_t slab, int r)
+{
+    if (R != 16) return (size_t) slab * R + r;
+    const int64_t pair = slab >> 3, half = (slab >> 2) & 1;
+    const int lane = 16 * (int) (slab & 3) + r;
+    return (size_t) pair * 128 + (size_t) lane * 2 + (size_t) half;
+}
+
+void free_tiles(DevTiles& t);
+
+// Construction of the tiled form (R in {8, 16}); R = 0 in `out` when fewer
+// than `min_density` of the slab entries would be non-zero. With R = 16
+// every tile's slab count is padded to a multiple of eight (zero slabs
+// repeating the tile's last column) and the values are laid out as the
+// matrix-core SpMM's operands (tile_slot).
+//
+// device_tiles builds it on the device for matrices whose rows are sorted
+// without repeats and of at most 2^31 - 1 entries: of `a`, or with `b` of
+// the union of both patterns (values left zero; *src_a and *src_b receive
+// the slot -> CSR position maps of the two in place of out.src). st.checked
+// tells whether the columns were looked at and st.built whether the form was
+// decided; otherwise (unsorted rows, too many entries, no memory for the
+// temporaries) the caller builds on the host.
+struct TileStatus {
+    bool want_tiles = true;    // false: only look the columns over
+    bool checked = false;
+    bool built = false;
+    bool bad_column = false;   // a column index out of range
+    bool sorted = false, strict = false;
+};
+int device_tiles(hipStream_t s, const DevCSR& a, const DevCSR* b, int R, double min_density,
+                 DevTiles& out, int32_t** src_a, int32_t** src_b, TileStatus& st);
+// On the host, for rows in any order; repeated columns are summed.
 // `data` may be null (values left zero); `src_host`, when given, receives
 // the host copy of the slot -> CSR position map (empty if not kept).
 int build_tiles(int64_t nrows, int64_t ncols, const int64_t* indptr,
