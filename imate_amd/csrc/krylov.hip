@@ -33,6 +33,7 @@
 // kernel boundary orders the two). The result is bitwise reproducible run
 // to run.
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -1321,7 +1322,12 @@ __global__ __launch_bounds__(kThreads) void dense_spmm_kernel(SpmmArgs<T> a,
 }
 
 // Adds the ksplit partial products of each row in split order and finishes
-// the rows as dense_spmm_kernel does without a split.
+// the rows as dense_spmm_kernel does without a split. Four rows a wavefront,
+// 32 a workgroup: with the product kernel's 128 rows a workgroup an n = 6001
+// matrix kept 47 of the 256 CUs busy (20.9 us with 11 splits; 6.6 us with the
+// 5 of today).
+constexpr int kDenseReduceRows = 4 * kWavesPerWG;
+
 template <typename T, bool NT>
 __global__ __launch_bounds__(kThreads) void dense_reduce_kernel(SpmmArgs<T> a,
                                                                 const T* __restrict__ X,
@@ -1345,39 +1351,51 @@ __global__ __launch_bounds__(kThreads) void dense_reduce_kernel(SpmmArgs<T> a,
     }
     const T tt = (T) a.t;
     double red[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int64_t rb = blockIdx.x; rb * 128 < a.nrows; rb += gridDim.x)
+    for (int64_t rb = blockIdx.x; rb * kDenseReduceRows < a.nrows; rb += gridDim.x)
     {
-        const int64_t r0 = rb * 128 + wave * 16;
-#pragma unroll
-        for (int m = 0; m < 4; ++m)
+        const int64_t row = rb * kDenseReduceRows + wave * 4 + kq;
+        if (row >= a.nrows) continue;
+        T y[4] = {T(0), T(0), T(0), T(0)};
+        for (int sp = 0; sp < ksplit; ++sp)
         {
-            const int64_t row = r0 + (Mfma16<T>::kRowStride == 4 ? kq + 4 * m : 4 * kq + m);
-            if (row >= a.nrows) continue;
-            T y[4] = {T(0), T(0), T(0), T(0)};
-            for (int sp = 0; sp < ksplit; ++sp)
-            {
-                T v[4];
-                Lanes<T>::load(scratch + ((int64_t) sp * a.nrows + row) * kBlock, i0, v);
+            T v[4];
+            Lanes<T>::load(scratch + ((int64_t) sp * a.nrows + row) * kBlock, i0, v);
 #pragma unroll
-                for (int q = 0; q < 4; ++q) y[q] += v[q];
-            }
-            spmm_epilogue4<T, NT>(a, row, i0, y, sq, tt, sub_c, sub_s, X, Y, Vout, Sub, red);
+            for (int q = 0; q < 4; ++q) y[q] += v[q];
         }
+        spmm_epilogue4<T, NT>(a, row, i0, y, sq, tt, sub_c, sub_s, X, Y, Vout, Sub, red);
     }
     if (a.red_mode) dense_red_partial<T>(a, red, wave, kq, i0, lane);
 }
 
-// Column splits of the dense SpMM for an nrows x ncols operand: enough work
-// items (row blocks x splits) for ~512 workgroups, at most one split per
-// 64-column chunk and 64 in all.
+// Column splits of the dense SpMM for an nrows x ncols operand: at most
+// enough for ~512 work items (row blocks x splits), one per 64-column chunk
+// and 64 in all, and of those the count with the least time in rounds of
+// resident workgroups: the kernel's 222 VGPRs (142 in FP32) let one workgroup
+// stay on a CU, 256 at a time. n = 6001 (47 row blocks) took 11 splits, 517
+// items in three rounds of which the last was nearly empty: 127 us a
+// product; 5 splits are one round of 235: 106 us.
 int dense_ksplit(int64_t nrows, int64_t ncols)
 {
+    const int64_t resident = 256;
     const int64_t rblocks = (nrows + 127) / 128;
     const int64_t nchunk = (ncols + kDenseKC - 1) / kDenseKC;
-    int64_t k = (512 + rblocks - 1) / rblocks;
-    if (k > nchunk) k = nchunk;
-    if (k > 64) k = 64;
-    return k < 1 ? 1 : (int) k;
+    int64_t cap = (512 + rblocks - 1) / rblocks;
+    if (cap > nchunk) cap = nchunk;
+    if (cap > 64) cap = 64;
+    int64_t best = 1, least = INT64_MAX;
+    for (int64_t k = 1; k <= cap; ++k)
+    {
+        // an item's start and end cost about two chunks
+        const int64_t rounds = (rblocks * k + resident - 1) / resident;
+        const int64_t cost = rounds * ((nchunk + k - 1) / k + 2);
+        if (cost < least)
+        {
+            least = cost;
+            best = k;
+        }
+    }
+    return (int) best;
 }
 
 // Sum of the per-tile partial rows in tile order, in two launches (the
@@ -1929,9 +1947,8 @@ int64_t sched_tiles(const slq_op* op)
     {
         // rows of 64 values of the dense SpMM's split scratch, either way
         const int64_t nr = A.csr.nrows, nc = A.csr.ncols;
-        const int64_t a = dense_ksplit(nr, nc) > 1 ? dense_ksplit(nr, nc) * nr : 0;
-        const int64_t b = dense_ksplit(nc, nr) > 1 ? dense_ksplit(nc, nr) * nc : 0;
-        return a > b ? a : b;
+        auto rows = [](int64_t n, int ks) { return ks > 1 ? ks * n : 0; };
+        return std::max(rows(nr, dense_ksplit(nr, nc)), rows(nc, dense_ksplit(nc, nr)));
     }
     if (A.tiles.R == 0) return 0;
     const int64_t R = A.tiles.R;
@@ -2160,7 +2177,8 @@ void launch_spmm_nt(slq_op* op, const SpmmArgs<T>& s, const SpmmIO<T>& io, const
         int rg = grid;
         if (ks > 1)
         {
-            rg = (int) (rblocks < kMaxGrid ? rblocks : kMaxGrid);
+            const int64_t units = (s.nrows + kDenseReduceRows - 1) / kDenseReduceRows;
+            rg = (int) (units < kMaxGrid ? units : kMaxGrid);
             hipLaunchKernelGGL((dense_reduce_kernel<T, NT>), dim3(rg), dim3(kThreads), 0,
                                op->stream, s, io.X, io.Y, io.Vout, io.Sub, ks,
                                (const T*) scratch);
