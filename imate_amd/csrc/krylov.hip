@@ -381,7 +381,7 @@ __global__ __launch_bounds__(kThreads) void spmm_kernel(SpmmArgs<T> a,
 // non-zero gathers a random operand row, and rows drawn from a table larger
 // than the L2 arrive at about half the rate of rows drawn from an
 // L2-resident table (measured: 14-15 vs 27.7 G rows/s for 512 B rows). A
-// wavefront owns kBlkRows rows and sweeps the columns in blocks of `cb`; the
+// wavefront owns RW rows and sweeps the columns in blocks of `cb`; the
 // waves of a workgroup pass the blocks together (a barrier every `sync`
 // blocks), the workgroups are as large as allowed (16 wavefronts, one per
 // CU) and the grid holds only as many as fit on the chip, so all of them
@@ -395,9 +395,7 @@ __global__ __launch_bounds__(kThreads) void spmm_kernel(SpmmArgs<T> a,
 // window (columns ascend), found with a ballot. Per row the products are
 // added in CSR order with the same fma chain as row_gather, so the result
 // equals spmm_kernel's bit for bit.
-constexpr int kBlkRows = 8;
-
-template <typename T, bool NT, int WPG>
+template <typename T, bool NT, int WPG, int RW>
 __global__ __launch_bounds__(WPG * kWave) void csr_blocked_kernel(SpmmArgs<T> a,
                                                                   const T* __restrict__ X,
                                                                   T* __restrict__ Y,
@@ -407,7 +405,7 @@ __global__ __launch_bounds__(WPG * kWave) void csr_blocked_kernel(SpmmArgs<T> a,
 {
     const int lane = threadIdx.x % kWave;
     const int wave = wave_id();
-    const int64_t ngroups = (a.nrows + kBlkRows - 1) / kBlkRows;
+    const int64_t ngroups = (a.nrows + RW - 1) / RW;
     const Sweep sw = sweep_wpg<WPG>(ngroups, wave);
     const T s = a.xscale ? (T) a.xscale[lane] : T(1);
     const T tt = (T) a.t;
@@ -424,10 +422,10 @@ __global__ __launch_bounds__(WPG * kWave) void csr_blocked_kernel(SpmmArgs<T> a,
     for (int64_t round = 0; round < rounds; ++round)
     {
         const int64_t gi = sw.first + round * sw.stride;
-        const int64_t r0 = gi < sw.end ? gi * kBlkRows : a.nrows;
-        int64_t cur[kBlkRows], end[kBlkRows];
-        int wc[kBlkRows], wpos[kBlkRows], wcnt[kBlkRows];
-        T wv[kBlkRows], acc[kBlkRows];
+        const int64_t r0 = gi < sw.end ? gi * RW : a.nrows;
+        int64_t cur[RW], end[RW];
+        int wc[RW], wpos[RW], wcnt[RW];
+        T wv[RW], acc[RW];
         auto load_window = [&](int k) {
             const int64_t rem = end[k] - cur[k];
             wcnt[k] = rem < kWave ? (int) rem : kWave;
@@ -441,7 +439,7 @@ __global__ __launch_bounds__(WPG * kWave) void csr_blocked_kernel(SpmmArgs<T> a,
             }
         };
 #pragma unroll
-        for (int k = 0; k < kBlkRows; ++k)
+        for (int k = 0; k < RW; ++k)
         {
             const bool in = r0 + k < a.nrows;
             cur[k] = in ? a.indptr[r0 + k] : 0;
@@ -453,7 +451,7 @@ __global__ __launch_bounds__(WPG * kWave) void csr_blocked_kernel(SpmmArgs<T> a,
         {
             const int64_t cend = (b + 1) * (int64_t) cb;
 #pragma unroll
-            for (int k = 0; k < kBlkRows; ++k)
+            for (int k = 0; k < RW; ++k)
             {
                 while (wcnt[k] > 0)
                 {
@@ -495,7 +493,7 @@ __global__ __launch_bounds__(WPG * kWave) void csr_blocked_kernel(SpmmArgs<T> a,
             if ((b + 1) % sync == 0 || b + 1 == nb) __syncthreads();
         }
 #pragma unroll
-        for (int k = 0; k < kBlkRows; ++k)
+        for (int k = 0; k < RW; ++k)
             if (r0 + k < a.nrows)
                 spmm_epilogue<T, NT>(a, r0 + k, lane, acc[k], s, tt, sub_c, sub_s, X, Y, Vout,
                                      Sub, red);
@@ -2036,18 +2034,48 @@ int nt_default()
 // Column block of the blocked CSR SpMM, or 0 for the row-per-wavefront
 // kernel: blocked when the rows are sorted, long (>= 128 non-zeros on
 // average) and the gathered operand is well beyond the L2 (> 16 MiB), and
-// no second (B) stream. SLQ_CSR_BLOCK_COLS sets the block (0 disables).
+// no second (B) stream. Operands up to 128 MiB (half the Infinity Cache,
+// which then serves the L2's misses) take blocks of 4 MiB: at 16384 rows of
+// 656 non-zeros over 65536 columns 388 us against 396 / 418 / 458 with 2, 1
+// and 0.5 MiB and 453 for the row kernel; larger ones 1024 columns.
+// SLQ_CSR_BLOCK_COLS sets the block (0 disables).
+constexpr double kCachedOperand = 128.0 * (1 << 20);
+
 template <typename T>
 int csr_blocked_cols(const SpmmArgs<T>& s)
 {
-    static int cb = [] {
+    static const int env = [] {
         const char* e = std::getenv("SLQ_CSR_BLOCK_COLS");
-        return e ? std::atoi(e) : 1024;
+        return e ? std::atoi(e) : -1;
     }();
-    if (cb <= 0 || !s.sorted || s.shift_mode == 2 || s.nrows <= 0) return 0;
-    if ((double) s.ncols * kBlock * sizeof(T) <= 16.0 * (1 << 20)) return 0;
+    if (env == 0 || !s.sorted || s.shift_mode == 2 || s.nrows <= 0) return 0;
+    const double operand = (double) s.ncols * kBlock * sizeof(T);
+    if (operand <= 16.0 * (1 << 20)) return 0;
     if (s.avg_row_nnz < 128.0) return 0;
-    return cb;
+    if (env > 0) return env;
+    return operand <= kCachedOperand ? (4 << 20) / (int) (kBlock * sizeof(T)) : 1024;
+}
+
+// Rows per wavefront of the blocked CSR SpMM, 8 or 4, or 0 for the row
+// kernel. Every wavefront sweeps all columns once per group of rows, so the
+// groups should fill whole rounds of the resident wavefronts (16 on each of
+// 256 CUs): 16384 rows in groups of 8 left half of the CUs idle (881 us;
+// groups of 4: 458 us at the same block). When neither count fills 85 % of
+// its rounds the row kernel, whose rows are independent, is the faster one
+// while the operand stays in the Infinity Cache.
+template <typename T>
+int csr_blocked_rows(const SpmmArgs<T>& s)
+{
+    auto used = [&](int rows) {
+        const int64_t resident = 256 * 16;
+        const int64_t groups = (s.nrows + rows - 1) / rows;
+        const int64_t rounds = (groups + resident - 1) / resident;
+        return (double) groups / (double) (rounds * resident);
+    };
+    if (used(8) >= 0.85) return 8;
+    if (used(4) >= 0.85) return 4;
+    if ((double) s.ncols * kBlock * sizeof(T) <= kCachedOperand) return 0;
+    return used(8) >= used(4) ? 8 : 4;
 }
 
 template <typename T>
@@ -2226,9 +2254,10 @@ void launch_spmm_nt(slq_op* op, const SpmmArgs<T>& s, const SpmmIO<T>& io, const
             }
         }
     }
-    else if (csr_blocked_cols(s) > 0)
+    else if (csr_blocked_cols(s) > 0 && csr_blocked_rows(s) > 0)
     {
-        const int64_t ngroups = (s.nrows + kBlkRows - 1) / kBlkRows;
+        const int rw = csr_blocked_rows(s);
+        const int64_t ngroups = (s.nrows + rw - 1) / rw;
         int grid = grid_for(ngroups, op->spmm_grid);
         // no more workgroups than fit on the chip at once, so that all of
         // them start the column sweep together
@@ -2238,15 +2267,21 @@ void launch_spmm_nt(slq_op* op, const SpmmArgs<T>& s, const SpmmIO<T>& io, const
             const char* e = std::getenv("SLQ_BLK_WAVES");
             return e && std::atoi(e) == 8 ? 8 : 16;
         }();
-        auto kern = wpg == 16 ? csr_blocked_kernel<T, NT, 16> : csr_blocked_kernel<T, NT, 8>;
+        auto kern = wpg == 16 ? (rw == 8 ? csr_blocked_kernel<T, NT, 16, 8>
+                                         : csr_blocked_kernel<T, NT, 16, 4>)
+                              : (rw == 8 ? csr_blocked_kernel<T, NT, 8, 8>
+                                         : csr_blocked_kernel<T, NT, 8, 4>);
         const int threads = wpg * kWave;
         if (wpg == 16) grid = (int) std::max<int64_t>(kXcds, ((grid / 2) / kXcds) * kXcds);
+        // (the 8-row kernel holds the more registers)
         static const int resident = [&] {
             int per_cu = 0, cus = 0, dev = 0;
+            auto most = wpg == 16 ? csr_blocked_kernel<T, NT, 16, 8>
+                                  : csr_blocked_kernel<T, NT, 8, 8>;
             if (hipGetDevice(&dev) != hipSuccess ||
                 hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=
                     hipSuccess ||
-                hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, threads, 0) !=
+                hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, most, threads, 0) !=
                     hipSuccess)
                 return 0;
             return ((per_cu * cus) / kXcds) * kXcds;

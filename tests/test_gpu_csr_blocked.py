@@ -1,0 +1,52 @@
+"""Products with long rows over many columns, at the row counts where the
+column-blocked SpMM takes 8 or 4 rows a wavefront and where the row kernel
+serves (a few rows below and above each line), against scipy in FP64."""
+
+import ctypes
+
+import numpy
+import pytest
+import scipy.sparse
+
+from imate_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+def _strata(nrows, ncols, k, seed, dtype):
+    rng = numpy.random.default_rng(seed)
+    s = numpy.arange(k + 1) * ncols // k
+    u = rng.random((nrows, k))
+    cols = (s[:-1] + (u * (s[1:] - s[:-1])).astype(numpy.int64)).ravel()
+    vals = rng.standard_normal(nrows * k).astype(dtype)
+    ip = numpy.arange(nrows + 1, dtype=numpy.int64) * k
+    return scipy.sparse.csr_matrix((vals, cols.astype(numpy.int32), ip),
+                                   shape=(nrows, ncols))
+
+
+# 4096 resident wavefronts: 85 % of a round is 27853 rows in groups of 8 and
+# 13927 in groups of 4; two rounds of 8 from 55706
+@pytest.mark.parametrize('nrows', [3001, 13900, 13931, 16389, 27860, 33001])
+@pytest.mark.parametrize('dtype', [numpy.float64, numpy.float32])
+def test_product(gpu_lib, nrows, dtype):
+    ncols = 32900 if dtype == numpy.float64 else 65700
+    A = _strata(nrows, ncols, 129, nrows, dtype)
+    ip = A.indptr.astype(numpy.int64)
+    h = ctypes.c_void_p()
+    _lib.check(gpu_lib.slq_op_create_csr(
+        nrows, ncols, A.nnz, _lib.ptr(ip), _lib.ptr(A.indices),
+        _lib.ptr(A.data), _lib.dtype_code(dtype), ctypes.byref(h)), 'create')
+    try:
+        X = numpy.random.default_rng(1).standard_normal(
+            (ncols, 64)).astype(dtype)
+        Y = numpy.empty((nrows, 64), dtype=dtype)
+        _lib.check(gpu_lib.slq_op_spmm(h, 0.0, 64, 0, _lib.ptr(X),
+                                       _lib.ptr(Y)), 'slq_op_spmm')
+        ref = A.astype(numpy.float64) @ X.astype(numpy.float64)
+        # 129 products summed in order: 129 eps of the sum of moduli
+        tol = 129 * numpy.finfo(dtype).eps
+        bound = tol * (abs(A).astype(numpy.float64) @
+                       numpy.abs(X.astype(numpy.float64)))
+        assert numpy.all(numpy.abs(Y - ref) <= bound)
+    finally:
+        gpu_lib.slq_op_destroy(h)
