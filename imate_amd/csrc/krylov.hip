@@ -1584,13 +1584,28 @@ __global__ __launch_bounds__(kTotalWaves * kWave) void norm_total_kernel(
 
 // ------------------------------------------------ Gram-Schmidt (CGS2)
 
-// Classical Gram-Schmidt, twice, against the K newest basis vectors of each
-// probe (basis layout [slot][row][64]; vector k of a pass is slot last - k):
-// h1 = V^T r, r -= V h1, h2 = V^T r, r -= V h2, |r|. Every probe has its own
-// basis, so each product is a GEMV per probe (0.5 flop per byte): the
-// kernels are HBM streams, written for loads in flight: a wavefront takes
-// one row per iteration and issues the loads of kGsChunk basis vectors at
-// once.
+// Classical Gram-Schmidt against the K newest basis vectors of each probe
+// (basis layout [slot][row][64]; vector k of a pass is slot last - k), a
+// second time where the first cancelled: h = V^T r, r -= V h, |r|, and again
+// when |h| is not small against |r| for some probe of the block
+// (gs_norm_kernel). "Twice is enough" (Parlett & Kahan; Daniel, Gragg,
+// Kaufman & Stewart, Math. Comp. 30, 1976): one pass leaves V^T r at the
+// rounding level unless the subtraction cancels most of r, and after the
+// three-term recurrence it does so only near a breakdown. The second pass's
+// kernels are queued either way; its product kernel also decides, and the
+// other returns at once when there is nothing to do. (An empty launch costs
+// 4-5 us, as much as a pass over a few thousand rows: so the second pass is
+// two launches, whose totals the last workgroup to finish adds up.)
+// Every probe has its own basis, so each product is a GEMV per probe (0.5
+// flop per byte): the kernels are HBM streams, written for loads in flight:
+// a wavefront takes one row per iteration and issues the loads of kGsChunk
+// basis vectors at once. Two
+// passes over the basis a step instead of the three of a pass that always
+// runs twice (the middle two fused): n = 65536, m = 60, 128 probes 98.5 ->
+// 67.4 ms in FP64 and 59.4 -> 39.3 ms with FP32 vectors; the passes run at
+// 5.1 (products) and 4.9 TB/s (subtractions). Sweeping the subtraction's rows
+// backwards, to meet what the product pass left in the Infinity Cache, was
+// 7 % faster in FP32 and 7 % slower in FP64, and is not done.
 constexpr int kGsChunk = 32;     // basis vectors per pass over the rows
 
 // Element stride between the stored basis vectors of a re-orthogonalised
@@ -1605,7 +1620,19 @@ struct GsArgs {
     int K;
     const double* h;         // [K][64] coefficients (gs_sub_kernel)
     double* partial_k;       // [G][K][64] (gs_dots_kernel)
-    int do_norm;             // gs_sub_kernel: partial rows of |r|^2 in rb
+    // gs_dots_kernel with UPD: r = w - alpha v (v the newest vector) first
+    const double* alpha;
+    // the second pass (gs_again_kernel, gs_sub_kernel<T, true>)
+    int* again;              // 1 where it runs
+    unsigned int* ticket;    // workgroups done, zero between launches
+    double* h_out;           // h, to be replaced by the second pass's
+    int first_rows;          // partial rows of the first pass's |r|^2
+    int twice;               // always run it
+    int j;
+    double tol_sqrt_n;
+    double* norm_out;
+    double* scale_out;
+    int32_t* sizes;
     RedBuf rb;
 };
 
@@ -1614,10 +1641,10 @@ struct GsArgs {
 // again as the last (a cache hit), so every load is unconditional and all C
 // are in flight at once; chunks are cut to C = 8, 16 or 32 to keep the
 // repeats few.
-template <typename T, int C>
-__device__ __forceinline__ void dots_rows(const T* __restrict__ base, const T* __restrict__ R,
+template <typename T, int C, bool UPD>
+__device__ __forceinline__ void dots_rows(const T* __restrict__ base, T* __restrict__ R,
                                           int64_t stride, int kn, const Sweep& sw, int lane,
-                                          double (&acc)[kGsChunk])
+                                          double al, double (&acc)[kGsChunk])
 {
     for (int64_t row = sw.first; row < sw.end; row += sw.stride)
     {
@@ -1625,7 +1652,14 @@ __device__ __forceinline__ void dots_rows(const T* __restrict__ base, const T* _
         T v[C];
 #pragma unroll
         for (int g = 0; g < C; ++g) v[g] = base[o - (int64_t) (g < kn ? g : kn - 1) * stride];
-        const double r = (double) R[o];
+        T rt = R[o];
+        if constexpr (UPD)
+        {
+            // the Lanczos update, rounded as lanczos_update_kernel rounds it
+            rt = (T) ((double) rt - al * (double) v[0]);
+            R[o] = rt;
+        }
+        const double r = (double) rt;
 #pragma unroll
         for (int g = 0; g < C; ++g) acc[g] += r * (double) v[g];
     }
@@ -1654,16 +1688,18 @@ __device__ __forceinline__ double sub_rows(const T* __restrict__ base, T* __rest
     return red;
 }
 
-// partial_k[g][k] = sum over the rows of workgroup g of basis_k * r.
-template <typename T>
-__global__ __launch_bounds__(kThreads) void gs_dots_kernel(GsArgs a, const T* __restrict__ R,
-                                                           const T* __restrict__ basis)
+// partial_k[g][k] = sum over the rows of workgroup g of basis_k * r, with
+// UPD after the update r = w - alpha v_j.
+template <typename T, bool UPD>
+__device__ __forceinline__ void gs_dots(const GsArgs& a, T* __restrict__ R,
+                                        const T* __restrict__ basis)
 {
     __shared__ double red[kWavesPerWG][8][kWave];
     const int lane = threadIdx.x % kWave;
     const int wave = wave_id();
     const Sweep sw = sweep_linear(a.nrows, wave);
     const int64_t stride = a.slot;
+    const double al = UPD ? a.alpha[lane] : 0.0;
     for (int k0 = 0; k0 < a.K; k0 += kGsChunk)
     {
         const int kn = (a.K - k0) < kGsChunk ? (a.K - k0) : kGsChunk;
@@ -1671,9 +1707,18 @@ __global__ __launch_bounds__(kThreads) void gs_dots_kernel(GsArgs a, const T* __
         double acc[kGsChunk];
 #pragma unroll
         for (int g = 0; g < kGsChunk; ++g) acc[g] = 0.0;
-        if (kn > 16) dots_rows<T, 32>(base, R, stride, kn, sw, lane, acc);
-        else if (kn > 8) dots_rows<T, 16>(base, R, stride, kn, sw, lane, acc);
-        else dots_rows<T, 8>(base, R, stride, kn, sw, lane, acc);
+        if (UPD && k0 == 0)
+        {
+            if (kn > 16) dots_rows<T, 32, UPD>(base, R, stride, kn, sw, lane, al, acc);
+            else if (kn > 8) dots_rows<T, 16, UPD>(base, R, stride, kn, sw, lane, al, acc);
+            else dots_rows<T, 8, UPD>(base, R, stride, kn, sw, lane, al, acc);
+        }
+        else
+        {
+            if (kn > 16) dots_rows<T, 32, false>(base, R, stride, kn, sw, lane, al, acc);
+            else if (kn > 8) dots_rows<T, 16, false>(base, R, stride, kn, sw, lane, al, acc);
+            else dots_rows<T, 8, false>(base, R, stride, kn, sw, lane, al, acc);
+        }
         // workgroup sums, eight vectors at a time through LDS
 #pragma unroll
         for (int g0 = 0; g0 < kGsChunk; g0 += 8)
@@ -1694,12 +1739,107 @@ __global__ __launch_bounds__(kThreads) void gs_dots_kernel(GsArgs a, const T* __
     }
 }
 
-// r -= sum_k h_k basis_k (in k order), optionally with the partial rows of
-// |r|^2 for norm_total_kernel.
+template <typename T, bool UPD>
+__global__ __launch_bounds__(kThreads) void gs_dots_kernel(GsArgs a, T* __restrict__ R,
+                                                           const T* __restrict__ basis)
+{
+    gs_dots<T, UPD>(a, R, basis);
+}
+
+// True in every thread of the last workgroup of the grid to get here, whose
+// later reads see what the others wrote before (the counter is then zero
+// again).
+__device__ __forceinline__ bool last_workgroup(unsigned int* ticket)
+{
+    __shared__ bool last;
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0)
+    {
+        last = atomicAdd(ticket, 1u) == gridDim.x - 1;
+        if (last) atomicExch(ticket, 0u);
+    }
+    __syncthreads();
+    __threadfence();
+    return last;
+}
+
+// Sum of rows[g][lane] over g in [0, G) by the workgroup's wavefronts, in a
+// fixed order, the same in every wavefront.
+__device__ __forceinline__ double wg_total(const double* __restrict__ rows, int G, int lane,
+                                           int wave)
+{
+    __shared__ double red[kWavesPerWG][kWave];
+    double s = 0.0;
+    int g = wave;
+    for (; g + 7 * kWavesPerWG < G; g += 8 * kWavesPerWG)
+    {
+        double v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = rows[(int64_t) (g + u * kWavesPerWG) * kWave + lane];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) s += v[u];
+    }
+    for (; g < G; g += kWavesPerWG) s += rows[(int64_t) g * kWave + lane];
+    __syncthreads();
+    red[wave][lane] = s;
+    __syncthreads();
+    double t = 0.0;
+#pragma unroll
+    for (int w = 0; w < kWavesPerWG; ++w) t += red[w][lane];
+    return t;
+}
+
+// After the first pass: |r|^2 from its partial rows, by every workgroup.
+// Unless |h| > 0.1 |r| for some probe (below that r lost at most 0.5 % of its
+// length; a NaN asks for nothing, it would stay one) the norm is final and
+// *again = 0; else, and always with `twice`, *again = 1 and this is the
+// second pass's product h = V^T r, whose totals the last workgroup stores.
+constexpr double kCancelSquared = 1e-2;
+
 template <typename T>
+__global__ __launch_bounds__(kThreads) void gs_again_kernel(GsArgs a, T* __restrict__ R,
+                                                            const T* __restrict__ basis)
+{
+    const int lane = threadIdx.x % kWave;
+    const int wave = wave_id();
+    __shared__ double hs[kWavesPerWG][kWave];
+    double hh = 0.0;
+    for (int k = wave; k < a.K; k += kWavesPerWG)
+    {
+        const double v = a.h[(int64_t) k * kWave + lane];
+        hh += v * v;
+    }
+    hs[wave][lane] = hh;
+    const double t = wg_total(a.rb.partial, a.first_rows, lane, wave);
+    double sum = 0.0;
+#pragma unroll
+    for (int w = 0; w < kWavesPerWG; ++w) sum += hs[w][lane];
+    const bool more = a.twice || __any(sum > kCancelSquared * t);
+    if (blockIdx.x == 0 && wave == 0)
+    {
+        if (lane == 0) *a.again = more ? 1 : 0;
+        if (!more) finish_norm(t, lane, a.j, a.tol_sqrt_n, a.norm_out, a.scale_out, a.sizes);
+    }
+    if (!more) return;
+    gs_dots<T, false>(a, R, basis);
+    if (!last_workgroup(a.ticket)) return;
+    const int G = gridDim.x;
+    for (int k = wave; k < a.K; k += kWavesPerWG)
+    {
+        double s = 0.0;
+        for (int g = 0; g < G; ++g) s += a.partial_k[((int64_t) g * a.K + k) * kWave + lane];
+        a.h_out[(int64_t) k * kWave + lane] = s;
+    }
+}
+
+// r -= sum_k h_k basis_k, with the partial rows of |r|^2; in the second pass
+// (SECOND) where that runs, and the last workgroup finishes the norm.
+template <typename T, bool SECOND>
 __global__ __launch_bounds__(kThreads) void gs_sub_kernel(GsArgs a, T* __restrict__ R,
                                                           const T* __restrict__ basis)
 {
+    if (SECOND && *a.again == 0) return;
     __shared__ double hs[kGsChunk][kWave];
     const int lane = threadIdx.x % kWave;
     const int wave = wave_id();
@@ -1718,7 +1858,7 @@ __global__ __launch_bounds__(kThreads) void gs_sub_kernel(GsArgs a, T* __restric
     for (int k0 = 0; k0 < a.K; k0 += kGsChunk)
     {
         const int kn = (a.K - k0) < kGsChunk ? (a.K - k0) : kGsChunk;
-        const bool norm = a.do_norm && k0 + kGsChunk >= a.K;
+        const bool norm = k0 + kGsChunk >= a.K;
         __syncthreads();
         for (int i = threadIdx.x; i < kGsChunk * kWave; i += blockDim.x)
             hs[i / kWave][i % kWave] = i < kn * kWave ? a.h[(int64_t) k0 * kWave + i] : 0.0;
@@ -1728,75 +1868,13 @@ __global__ __launch_bounds__(kThreads) void gs_sub_kernel(GsArgs a, T* __restric
         else if (kn > 8) red = sub_rows<T, 16>(base, R, stride, kn, sw, lane, hs, norm);
         else red = sub_rows<T, 8>(base, R, stride, kn, sw, lane, hs, norm);
     }
-    if (a.do_norm) wg_partial(red, a.rb);
-}
-
-// The first subtraction and the second product of CGS2 in one pass over the
-// basis: per row r' = r - sum_k h1_k v_k (k order, all K <= C vectors held
-// in registers), stored, and partial_k[g][k] = sum over the rows of
-// workgroup g of v_k r'. Per row this is the arithmetic of gs_sub_kernel
-// followed by gs_dots_kernel (for K > kGsChunk without the rounding of r to
-// T between chunks), with one read of the basis instead of two.
-// C <= 32 runs in 512-thread workgroups (two wavefronts per SIMD: at C =
-// 32 the values, the sums and the addresses take 252 VGPRs); C = 64 in
-// 256-thread workgroups, one wavefront per SIMD with up to 512 VGPRs.
-template <typename T, int C, int WPG>
-__global__ __launch_bounds__(WPG * kWave) void gs_subdots_kernel(GsArgs a, T* __restrict__ R,
-                                                                 const T* __restrict__ basis)
-{
-    __shared__ double hs[C][kWave];
-    __shared__ double red[WPG][8][kWave];
-    const int lane = threadIdx.x % kWave;
-    const int wave = wave_id();
-    Sweep sw;
-    sw.first = (int64_t) blockIdx.x * WPG + wave;
-    sw.stride = (int64_t) gridDim.x * WPG;
-    sw.end = a.nrows;
-    const int64_t stride = a.slot;
-    const int kn = a.K;
-    for (int i = threadIdx.x; i < C * kWave; i += blockDim.x)
-        hs[i / kWave][i % kWave] = i < kn * kWave ? a.h[i] : 0.0;
-    __syncthreads();
-    const T* __restrict__ base = basis + (int64_t) a.last * stride;
-    double acc[C];
-#pragma unroll
-    for (int g = 0; g < C; ++g) acc[g] = 0.0;
-#pragma unroll 1
-    for (int64_t row = sw.first; row < sw.end; row += sw.stride)
+    wg_partial(red, a.rb);
+    if constexpr (SECOND)
     {
-        // re-read hs from LDS every row rather than hold C coefficients in
-        // registers beside the C values and C sums
-        asm volatile("" ::: "memory");
-        const int64_t o = row * kBlock + lane;
-        T v[C];
-#pragma unroll
-        for (int g = 0; g < C; ++g) v[g] = base[o - (int64_t) (g < kn ? g : kn - 1) * stride];
-        double r = (double) R[o];
-#pragma unroll
-        for (int g = 0; g < C; ++g) r -= hs[g][lane] * (double) v[g];
-        const T rt = (T) r;
-        R[o] = rt;
-        const double rd = (double) rt;
-#pragma unroll
-        for (int g = 0; g < C; ++g) acc[g] += rd * (double) v[g];
-    }
-    // workgroup sums, eight vectors at a time through LDS
-#pragma unroll
-    for (int g0 = 0; g0 < C; g0 += 8)
-    {
-        if (g0 >= kn) break;
-#pragma unroll
-        for (int g = 0; g < 8; ++g) red[wave][g][lane] = acc[g0 + g];
-        __syncthreads();
-        for (int q = wave; q < 8; q += WPG)
-            if (g0 + q < kn)
-            {
-                double t = 0.0;
-#pragma unroll
-                for (int w = 0; w < WPG; ++w) t += red[w][q][lane];
-                a.partial_k[((int64_t) blockIdx.x * a.K + g0 + q) * kWave + lane] = t;
-            }
-        __syncthreads();
+        if (!last_workgroup(a.ticket)) return;
+        const double t = wg_total(a.rb.partial, gridDim.x, lane, wave);
+        if (wave == 0)
+            finish_norm(t, lane, a.j, a.tol_sqrt_n, a.norm_out, a.scale_out, a.sizes);
     }
 }
 
@@ -1969,10 +2047,13 @@ bool redbuf_ok(const RedBuf& rb)
     return rb.partial && rb.tickets;
 }
 
-void zero_counters(hipStream_t s, const RedBuf& rb)
+void zero_counters(hipStream_t s, const RedBuf& rb, int* gs_words = nullptr, int n = 0)
 {
     hipLaunchKernelGGL(zero_u32_kernel, dim3(kTicketWords / 64), dim3(64), 0, s, rb.tickets,
                        kTicketWords);
+    if (gs_words)
+        hipLaunchKernelGGL(zero_u32_kernel, dim3((n + 63) / 64), dim3(64), 0, s,
+                           (unsigned int*) gs_words, n);
 }
 
 size_t redbuf_bytes(int64_t tiles)
@@ -2356,20 +2437,28 @@ int launch_update(slq_op* op, const UpdateArgs& u, T* R, const T* Vj, const T* V
 // K partial rows.
 int gs_grid(int64_t rows, int cap) { return stream_grid(rows, cap); }
 
-// The fused subtraction + product pass is on unless SLQ_FUSED_GS=0 (read per
-// call, so a process can time both).
-bool fused_gs_enabled()
+// Words of the re-orthogonalisation's flags: [0] second pass, [kGsTicket] the
+// workgroup counter of its kernels.
+constexpr int kGsTicket = 32;
+constexpr int kGsWords = 64;
+
+// The second Gram-Schmidt pass runs only where the first cancelled, unless
+// SLQ_FUSED_GS=0 asks for it always (read per call, so a process can compare
+// the two).
+bool gs_twice()
 {
     const char* e = std::getenv("SLQ_FUSED_GS");
-    return !(e && std::atoi(e) == 0);
+    return e && std::atoi(e) == 0;
 }
 
-// CGS2 of r against the K newest basis vectors (slots last, last-1, ...);
-// the final pass finishes the norm (beta_j, or alpha_j for Golub-Kahn u).
+// Gram-Schmidt of r against the K newest basis vectors (slots last, last -
+// 1, ...), with the norm (beta_j, or alpha_j for Golub-Kahn u). `alpha`, when
+// given, is the Lanczos update's coefficient: R holds w and the newest vector
+// is v_j.
 template <typename T>
 int reorthogonalize(slq_op* op, int64_t nrows, T* R, const T* basis, size_t slot,
-                    int last, int K, double* h1, double* h2, double* partial_k,
-                    const RedBuf& rb, double* norm_out, double* scale_out,
+                    int last, int K, const double* alpha, double* h, int* again,
+                    double* partial_k, const RedBuf& rb, double* norm_out, double* scale_out,
                     int32_t* sizes, int j, double tol_sqrt_n)
 {
     const int G = gs_grid(nrows, op->stream_grid);
@@ -2381,50 +2470,39 @@ int reorthogonalize(slq_op* op, int64_t nrows, T* R, const T* basis, size_t slot
     g.K = K;
     g.partial_k = partial_k;
     g.rb = rb;
+    g.h = h;
+    g.h_out = h;
+    g.alpha = alpha;
+    g.again = again;
+    g.ticket = (unsigned int*) again + kGsTicket;
+    g.first_rows = G;
+    g.twice = gs_twice() ? 1 : 0;
+    g.j = j;
+    g.tol_sqrt_n = tol_sqrt_n;
+    g.norm_out = norm_out;
+    g.scale_out = scale_out;
+    g.sizes = sizes;
+    const dim3 tg(kTotalWaves * kWave), grid(G), wg(kThreads);
     if (K > 0)
     {
-        // h1 = V^T r; r -= V h1; h2 = V^T r; then r -= V h2 below
-        const dim3 tg(kTotalWaves * kWave);
-        hipLaunchKernelGGL(gs_dots_kernel<T>, dim3(G), dim3(kThreads), 0, op->stream, g, R,
-                           basis);
-        hipLaunchKernelGGL(reduce_partials_kernel, dim3(K), tg, 0, op->stream, partial_k, G,
-                           K, h1);
-        g.h = h1;
-        // r -= V h1 and h2 = V^T r in one pass while the K vectors of a row
-        // fit in registers without spilling (K <= 64), else two passes
-        if (K <= 64 && fused_gs_enabled())
-        {
-            if (K > 32)
-                hipLaunchKernelGGL((gs_subdots_kernel<T, 64, 4>), dim3(G), dim3(4 * kWave), 0,
-                                   op->stream, g, R, basis);
-            else if (K > 16)
-                hipLaunchKernelGGL((gs_subdots_kernel<T, 32, kWavesPerWG>), dim3(G),
-                                   dim3(kThreads), 0, op->stream, g, R, basis);
-            else if (K > 8)
-                hipLaunchKernelGGL((gs_subdots_kernel<T, 16, kWavesPerWG>), dim3(G),
-                                   dim3(kThreads), 0, op->stream, g, R, basis);
-            else
-                hipLaunchKernelGGL((gs_subdots_kernel<T, 8, kWavesPerWG>), dim3(G),
-                                   dim3(kThreads), 0, op->stream, g, R, basis);
-        }
+        if (alpha)
+            hipLaunchKernelGGL((gs_dots_kernel<T, true>), grid, wg, 0, op->stream, g, R, basis);
         else
-        {
-            hipLaunchKernelGGL(gs_sub_kernel<T>, dim3(G), dim3(kThreads), 0, op->stream, g, R,
+            hipLaunchKernelGGL((gs_dots_kernel<T, false>), grid, wg, 0, op->stream, g, R,
                                basis);
-            hipLaunchKernelGGL(gs_dots_kernel<T>, dim3(G), dim3(kThreads), 0, op->stream, g,
-                               R, basis);
-        }
-        hipLaunchKernelGGL(reduce_partials_kernel, dim3(K), tg, 0, op->stream, partial_k, G,
-                           K, h2);
-        SLQ_CHECK(hipGetLastError());
-        g.h = h2;
+        hipLaunchKernelGGL(reduce_partials_kernel, dim3(K), tg, 0, op->stream,
+                           (const double*) partial_k, G, K, h);
     }
-    g.do_norm = 1;
-    hipLaunchKernelGGL(gs_sub_kernel<T>, dim3(G), dim3(kThreads), 0, op->stream, g, R, basis);
-    SLQ_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(norm_total_kernel, dim3(1), dim3(kTotalWaves * kWave), 0, op->stream,
-                       (const double*) rb.partial, G, j, tol_sqrt_n, norm_out, scale_out,
-                       sizes);
+    hipLaunchKernelGGL((gs_sub_kernel<T, false>), grid, wg, 0, op->stream, g, R, basis);
+    if (K == 0)
+        hipLaunchKernelGGL(norm_total_kernel, dim3(1), tg, 0, op->stream,
+                           (const double*) rb.partial, G, j, tol_sqrt_n, norm_out, scale_out,
+                           sizes);
+    else
+    {
+        hipLaunchKernelGGL(gs_again_kernel<T>, grid, wg, 0, op->stream, g, R, basis);
+        hipLaunchKernelGGL((gs_sub_kernel<T, true>), grid, wg, 0, op->stream, g, R, basis);
+    }
     SLQ_CHECK(hipGetLastError());
     return SLQ_OK;
 }
@@ -2560,22 +2638,22 @@ int lanczos(const RecurrenceArgs& ra, Bump& bump)
     double* scale = bump.take<double>(kBlock);
     double* ones = bump.take<double>(kBlock);   // scale of the stored basis
     const RedBuf rb = take_redbuf(bump, sched_tiles(op));
-    double* h1 = nullptr;
-    double* h2 = nullptr;
+    double* h = nullptr;
+    int* again = nullptr;
     double* partial_k = nullptr;
     if (reorth)
     {
-        h1 = bump.take<double>((size_t) (m + 1) * kBlock);
-        h2 = bump.take<double>((size_t) (m + 1) * kBlock);
+        h = bump.take<double>((size_t) (m + 1) * kBlock);
+        again = bump.take<int>(kGsWords);
         partial_k = bump.take<double>((size_t) kMaxGrid * (m + 1) * kBlock);
     }
     if (!P || !Q || !V || !scale || !ones || !redbuf_ok(rb) ||
-        (reorth && (!h1 || !h2 || !partial_k)))
+        (reorth && (!h || !again || !partial_k)))
     {
         set_error("internal: Lanczos workspace too small");
         return SLQ_E_OOM;
     }
-    zero_counters(op->stream, rb);
+    zero_counters(op->stream, rb, again, kGsWords);
     hipLaunchKernelGGL(set_ones_kernel, dim3(1), dim3(kBlock), 0, op->stream, ones);
     const bool beta_in_spmm = spmm_beta_enabled();
     // initial_beta = |probe| = sqrt(n) exactly for a Rademacher probe
@@ -2619,27 +2697,25 @@ int lanczos(const RecurrenceArgs& ra, Bump& bump)
         }
         SLQ_TRY(launch_spmm<T>(op, s, io, tl));
 
-        UpdateArgs u;
-        std::memset(&u, 0, sizeof(u));
-        u.nrows = n;
-        u.alpha = ra.alpha + (size_t) j * kBlock;
-        u.beta = j > 0 && !fused ? ra.beta + (size_t) (j - 1) * kBlock : nullptr;
-        u.do_norm = reorth ? 0 : 1;
-        u.rb = rb;
-        u.beta_out = ra.beta + (size_t) j * kBlock;
-        u.scale_out = scale;
-        u.sizes = ra.sizes;
-        u.j = j;
-        u.tol_sqrt_n = tol_sqrt_n;
-        SLQ_TRY(launch_update<T>(op, u, W, Vj, fused ? nullptr : Vjm1));
-
-        if (reorth)
+        // r = w - alpha_j v_j in the product pass of the re-orthogonalisation,
+        // whose newest basis vector is v_j; with the beta term still to
+        // subtract (SLQ_SPMM_BETA=0) in the update kernel
+        const double* alpha = ra.alpha + (size_t) j * kBlock;
+        if (j > 0 && !fused)
         {
-            const int num_ortho = j < buffer ? j + 1 : buffer;
-            SLQ_TRY(reorthogonalize<T>(op, n, W, V, vst, j, num_ortho, h1, h2, partial_k, rb,
-                                       ra.beta + (size_t) j * kBlock, scale, ra.sizes, j,
-                                       tol_sqrt_n));
+            UpdateArgs u;
+            std::memset(&u, 0, sizeof(u));
+            u.nrows = n;
+            u.alpha = alpha;
+            u.beta = ra.beta + (size_t) (j - 1) * kBlock;
+            u.j = j;
+            SLQ_TRY(launch_update<T>(op, u, W, Vj, Vjm1));
+            alpha = nullptr;
         }
+        const int num_ortho = j < buffer ? j + 1 : buffer;
+        SLQ_TRY(reorthogonalize<T>(op, n, W, V, vst, j, num_ortho, alpha, h, again, partial_k,
+                                   rb, ra.beta + (size_t) j * kBlock, scale, ra.sizes, j,
+                                   tol_sqrt_n));
         src = W;
     }
     return SLQ_OK;
@@ -2674,22 +2750,22 @@ int golub_kahn(const RecurrenceArgs& ra, Bump& bump)
     double* sv = bump.take<double>((size_t) (m + 1) * kBlock);   // 1/beta_{j-1}
     const RedBuf rb = take_redbuf(bump, sched_tiles(op));
     int32_t* usizes = bump.take<int32_t>(kBlock);
-    double* h1 = nullptr;
-    double* h2 = nullptr;
+    double* h = nullptr;
+    int* again = nullptr;
     double* partial_k = nullptr;
     if (reorth)
     {
-        h1 = bump.take<double>((size_t) (m + 1) * kBlock);
-        h2 = bump.take<double>((size_t) (m + 1) * kBlock);
+        h = bump.take<double>((size_t) (m + 1) * kBlock);
+        again = bump.take<int>(kGsWords);
         partial_k = bump.take<double>((size_t) kMaxGrid * (m + 1) * kBlock);
     }
     if (!U || !V || !su || !sv || !redbuf_ok(rb) || !usizes ||
-        (reorth && (!h1 || !h2 || !partial_k)))
+        (reorth && (!h || !again || !partial_k)))
     {
         set_error("internal: Golub-Kahn workspace too small");
         return SLQ_E_OOM;
     }
-    zero_counters(op->stream, rb);
+    zero_counters(op->stream, rb, again, kGsWords);
     // v_0 = probe / |probe|, |probe| = sqrt(ncols) exactly
     const double s0 = 1.0 / std::sqrt((double) nc);
     hipLaunchKernelGGL(init_block_kernel, dim3(1), dim3(kBlock), 0, op->stream,
@@ -2747,7 +2823,7 @@ int golub_kahn(const RecurrenceArgs& ra, Bump& bump)
         {
             const int num_ortho = j < buffer ? j : buffer - 1;
             SLQ_TRY(reorthogonalize<T>(op, nr, uslot(j), U, ust, j - 1, j > 0 ? num_ortho : 0,
-                                       h1, h2, partial_k, rb, ra.alpha + (size_t) j * kBlock,
+                                       nullptr, h, again, partial_k, rb, ra.alpha + (size_t) j * kBlock,
                                        su + (size_t) j * kBlock, usizes, j, -1.0));
             SLQ_TRY(normalize_in_place<T>(op, uslot(j), nr, su + (size_t) j * kBlock));
         }
@@ -2778,7 +2854,7 @@ int golub_kahn(const RecurrenceArgs& ra, Bump& bump)
         if (reorth)
         {
             const int num_ortho = j < buffer ? j : buffer - 1;
-            SLQ_TRY(reorthogonalize<T>(op, nc, vslot(j + 1), V, vst, j, num_ortho, h1, h2,
+            SLQ_TRY(reorthogonalize<T>(op, nc, vslot(j + 1), V, vst, j, num_ortho, nullptr, h, again,
                                        partial_k, rb, ra.beta + (size_t) j * kBlock,
                                        sv + (size_t) (j + 1) * kBlock, ra.sizes, j,
                                        tol_sqrt_n));
@@ -2830,7 +2906,7 @@ size_t recurrence_scratch_bytes(const slq_op* op, int gram, int m, int ortho,
     if (reorth)
     {
         add(sizeof(double) * (m + 1) * kBlock);
-        add(sizeof(double) * (m + 1) * kBlock);
+        add(sizeof(int) * kGsWords);
         add(sizeof(double) * (size_t) kMaxGrid * (m + 1) * kBlock);
     }
     return b + 4096;
