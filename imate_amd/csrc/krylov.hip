@@ -1601,9 +1601,9 @@ __global__ __launch_bounds__(kTotalWaves * kWave) void norm_total_kernel(
 // a wavefront takes one row per iteration and issues the loads of kGsChunk
 // basis vectors at once. Two
 // passes over the basis a step instead of the three of a pass that always
-// runs twice (the middle two fused): n = 65536, m = 60, 128 probes 98.5 ->
-// 67.4 ms in FP64 and 59.4 -> 39.3 ms with FP32 vectors; the passes run at
-// 5.1 (products) and 4.9 TB/s (subtractions). Sweeping the subtraction's rows
+// runs twice (the middle two fused, as FP32 vectors still take them):
+// n = 65536, m = 60, 128 probes 98.5 -> 67.4 ms; the passes run at 5.1
+// (products) and 4.9 TB/s (subtractions). Sweeping the subtraction's rows
 // backwards, to meet what the product pass left in the Infinity Cache, was
 // 7 % faster in FP32 and 7 % slower in FP64, and is not done.
 constexpr int kGsChunk = 32;     // basis vectors per pass over the rows
@@ -1627,7 +1627,6 @@ struct GsArgs {
     unsigned int* ticket;    // workgroups done, zero between launches
     double* h_out;           // h, to be replaced by the second pass's
     int first_rows;          // partial rows of the first pass's |r|^2
-    int twice;               // always run it
     int j;
     double tol_sqrt_n;
     double* norm_out;
@@ -1793,8 +1792,8 @@ __device__ __forceinline__ double wg_total(const double* __restrict__ rows, int 
 // After the first pass: |r|^2 from its partial rows, by every workgroup.
 // Unless |h| > 0.1 |r| for some probe (below that r lost at most 0.5 % of its
 // length; a NaN asks for nothing, it would stay one) the norm is final and
-// *again = 0; else, and always with `twice`, *again = 1 and this is the
-// second pass's product h = V^T r, whose totals the last workgroup stores.
+// *again = 0; else *again = 1 and this is the second pass's product h = V^T r,
+// whose totals the last workgroup stores.
 constexpr double kCancelSquared = 1e-2;
 
 template <typename T>
@@ -1815,7 +1814,7 @@ __global__ __launch_bounds__(kThreads) void gs_again_kernel(GsArgs a, T* __restr
     double sum = 0.0;
 #pragma unroll
     for (int w = 0; w < kWavesPerWG; ++w) sum += hs[w][lane];
-    const bool more = a.twice || __any(sum > kCancelSquared * t);
+    const bool more = __any(sum > kCancelSquared * t);
     if (blockIdx.x == 0 && wave == 0)
     {
         if (lane == 0) *a.again = more ? 1 : 0;
@@ -1875,6 +1874,75 @@ __global__ __launch_bounds__(kThreads) void gs_sub_kernel(GsArgs a, T* __restric
         const double t = wg_total(a.rb.partial, gridDim.x, lane, wave);
         if (wave == 0)
             finish_norm(t, lane, a.j, a.tol_sqrt_n, a.norm_out, a.scale_out, a.sizes);
+    }
+}
+
+// The first subtraction and the second product of the classical form that
+// always runs twice, in one pass over the basis: per row r' = r - sum_k h1_k v_k (k order, all K <= C vectors held
+// in registers), stored, and partial_k[g][k] = sum over the rows of
+// workgroup g of v_k r'. Per row this is the arithmetic of gs_sub_kernel
+// followed by gs_dots_kernel (for K > kGsChunk without the rounding of r to
+// T between chunks), with one read of the basis instead of two.
+// C <= 32 runs in 512-thread workgroups (two wavefronts per SIMD: at C =
+// 32 the values, the sums and the addresses take 252 VGPRs); C = 64 in
+// 256-thread workgroups, one wavefront per SIMD with up to 512 VGPRs.
+template <typename T, int C, int WPG>
+__global__ __launch_bounds__(WPG * kWave) void gs_subdots_kernel(GsArgs a, T* __restrict__ R,
+                                                                 const T* __restrict__ basis)
+{
+    __shared__ double hs[C][kWave];
+    __shared__ double red[WPG][8][kWave];
+    const int lane = threadIdx.x % kWave;
+    const int wave = wave_id();
+    Sweep sw;
+    sw.first = (int64_t) blockIdx.x * WPG + wave;
+    sw.stride = (int64_t) gridDim.x * WPG;
+    sw.end = a.nrows;
+    const int64_t stride = a.slot;
+    const int kn = a.K;
+    for (int i = threadIdx.x; i < C * kWave; i += blockDim.x)
+        hs[i / kWave][i % kWave] = i < kn * kWave ? a.h[i] : 0.0;
+    __syncthreads();
+    const T* __restrict__ base = basis + (int64_t) a.last * stride;
+    double acc[C];
+#pragma unroll
+    for (int g = 0; g < C; ++g) acc[g] = 0.0;
+#pragma unroll 1
+    for (int64_t row = sw.first; row < sw.end; row += sw.stride)
+    {
+        // re-read hs from LDS every row rather than hold C coefficients in
+        // registers beside the C values and C sums
+        asm volatile("" ::: "memory");
+        const int64_t o = row * kBlock + lane;
+        T v[C];
+#pragma unroll
+        for (int g = 0; g < C; ++g) v[g] = base[o - (int64_t) (g < kn ? g : kn - 1) * stride];
+        double r = (double) R[o];
+#pragma unroll
+        for (int g = 0; g < C; ++g) r -= hs[g][lane] * (double) v[g];
+        const T rt = (T) r;
+        R[o] = rt;
+        const double rd = (double) rt;
+#pragma unroll
+        for (int g = 0; g < C; ++g) acc[g] += rd * (double) v[g];
+    }
+    // workgroup sums, eight vectors at a time through LDS
+#pragma unroll
+    for (int g0 = 0; g0 < C; g0 += 8)
+    {
+        if (g0 >= kn) break;
+#pragma unroll
+        for (int g = 0; g < 8; ++g) red[wave][g][lane] = acc[g0 + g];
+        __syncthreads();
+        for (int q = wave; q < 8; q += WPG)
+            if (g0 + q < kn)
+            {
+                double t = 0.0;
+#pragma unroll
+                for (int w = 0; w < WPG; ++w) t += red[w][q][lane];
+                a.partial_k[((int64_t) blockIdx.x * a.K + g0 + q) * kWave + lane] = t;
+            }
+        __syncthreads();
     }
 }
 
@@ -2442,10 +2510,9 @@ int gs_grid(int64_t rows, int cap) { return stream_grid(rows, cap); }
 constexpr int kGsTicket = 32;
 constexpr int kGsWords = 64;
 
-// The second Gram-Schmidt pass runs only where the first cancelled, unless
-// SLQ_FUSED_GS=0 asks for it always (read per call, so a process can compare
-// the two).
-bool gs_twice()
+// SLQ_FUSED_GS=0: every product and subtraction of two passes by itself
+// (read per call, so a process can compare).
+bool gs_plain()
 {
     const char* e = std::getenv("SLQ_FUSED_GS");
     return e && std::atoi(e) == 0;
@@ -2476,30 +2543,77 @@ int reorthogonalize(slq_op* op, int64_t nrows, T* R, const T* basis, size_t slot
     g.again = again;
     g.ticket = (unsigned int*) again + kGsTicket;
     g.first_rows = G;
-    g.twice = gs_twice() ? 1 : 0;
     g.j = j;
     g.tol_sqrt_n = tol_sqrt_n;
     g.norm_out = norm_out;
     g.scale_out = scale_out;
     g.sizes = sizes;
     const dim3 tg(kTotalWaves * kWave), grid(G), wg(kThreads);
-    if (K > 0)
-    {
-        if (alpha)
+    auto dots = [&](bool update) {
+        if (update)
             hipLaunchKernelGGL((gs_dots_kernel<T, true>), grid, wg, 0, op->stream, g, R, basis);
         else
             hipLaunchKernelGGL((gs_dots_kernel<T, false>), grid, wg, 0, op->stream, g, R,
                                basis);
+    };
+    auto reduce = [&]() {
         hipLaunchKernelGGL(reduce_partials_kernel, dim3(K), tg, 0, op->stream,
                            (const double*) partial_k, G, K, h);
-    }
-    hipLaunchKernelGGL((gs_sub_kernel<T, false>), grid, wg, 0, op->stream, g, R, basis);
-    if (K == 0)
+    };
+    auto sub = [&]() {
+        hipLaunchKernelGGL((gs_sub_kernel<T, false>), grid, wg, 0, op->stream, g, R, basis);
+    };
+    auto norm = [&]() {
         hipLaunchKernelGGL(norm_total_kernel, dim3(1), tg, 0, op->stream,
                            (const double*) rb.partial, G, j, tol_sqrt_n, norm_out, scale_out,
                            sizes);
+    };
+    // FP32 vectors always take both passes: the error of their results is
+    // that of the vectors' rounding, which leaving a pass out would draw anew
+    const bool always = sizeof(T) == 4;
+    if (K == 0)
+    {
+        sub();
+        norm();
+    }
+    else if (always && K <= 64 && !gs_plain())
+    {
+        dots(alpha != nullptr);
+        reduce();
+        if constexpr (sizeof(T) == 4)
+        {
+            if (K > 32)
+                hipLaunchKernelGGL((gs_subdots_kernel<T, 64, 4>), grid, dim3(4 * kWave), 0,
+                                   op->stream, g, R, basis);
+            else if (K > 16)
+                hipLaunchKernelGGL((gs_subdots_kernel<T, 32, kWavesPerWG>), grid, wg, 0,
+                                   op->stream, g, R, basis);
+            else if (K > 8)
+                hipLaunchKernelGGL((gs_subdots_kernel<T, 16, kWavesPerWG>), grid, wg, 0,
+                                   op->stream, g, R, basis);
+            else
+                hipLaunchKernelGGL((gs_subdots_kernel<T, 8, kWavesPerWG>), grid, wg, 0,
+                                   op->stream, g, R, basis);
+        }
+        reduce();
+        sub();
+        norm();
+    }
+    else if (always || gs_plain())
+    {
+        dots(alpha != nullptr);
+        reduce();
+        sub();
+        dots(false);
+        reduce();
+        sub();
+        norm();
+    }
     else
     {
+        dots(alpha != nullptr);
+        reduce();
+        sub();
         hipLaunchKernelGGL(gs_again_kernel<T>, grid, wg, 0, op->stream, g, R, basis);
         hipLaunchKernelGGL((gs_sub_kernel<T, true>), grid, wg, 0, op->stream, g, R, basis);
     }
