@@ -807,16 +807,33 @@ __device__ __forceinline__ void spmm_epilogue4(const SpmmArgs<T>& a, int64_t row
 // four slabs at a time, A = the 16 x 4 slab values (64 consecutive values of
 // the slab array, one coalesced load), B = the four gathered operand rows,
 // one 16-probe block per MFMA (four per group). The matrix values arrive
-// through ordinary vector loads and are broadcast by the matrix core (no
-// scalar loads, no readlane per value), so loads stay in flight: the column
-// indices of up to 64 slabs are loaded once per chunk (lane l holds slab
-// chunk + l) and broadcast with readlane, so a group's gathers need no
-// dependent index load, and the loads of the next group of four slabs are
-// issued before the MFMAs of the current one (two register sets). Tiles are
-// handed out in order as in tiled_spmm_sched_kernel; the per-probe reduction
-// term of a tile adds the four rows held by a lane, then the four row groups
-// (lanes l, l ^ 16, l ^ 32, l ^ 48) in a fixed order.
-template <typename T, bool NT>
+// through ordinary vector loads and are broadcast by the matrix core, so
+// loads stay in flight.
+//
+// A wavefront takes one tile, a workgroup eight neighbouring ones, and the
+// hardware deals the workgroups out in order, workgroup id mod 8 to one XCD:
+// the tiles in flight on an XCD are consecutive and share the operand rows
+// in its L2. (A persistent grid that drew tiles from a per-XCD ticket
+// counter, one group of four slabs ahead, took 28 / 49 / 615 us at n =
+// 20011 / 65536 / 2^20 with 50 non-zeros a row, 118 us at 65536 with 247 and
+// 84 us with that in FP32; without tickets but with the same loop 25 / 41 /
+// 632, 109 and 76; this kernel 20 / 35 / 603, 100 and 55.)
+//
+// What bounds it below 2^20 rows is the latency of a wavefront's chain of
+// gathers, at 2^20 the rate of the gathers themselves. kSpmmDepth pairs of
+// four-slab groups (a pair's values are one load) are in flight per
+// wavefront, and the columns of the kSpmmDepth pairs after them, each lane
+// loading its own: 2 pairs 36 and 604 us at 65536 and 2^20 rows, 4 pairs
+// (150 VGPRs, three wavefronts per SIMD) 38 and 712. The per-probe
+// reduction term of a tile adds the four rows held by a lane, then the four
+// row groups (lanes l, l ^ 16, l ^ 32, l ^ 48), then the workgroup's tiles,
+// in a fixed order; its partial row goes to tile_partial. With a grid capped
+// by the launch settings (CAPPED) a workgroup takes further tiles in steps of
+// the grid; that loop costs the uncapped form's fourth wavefront per SIMD (148
+// against 126 VGPRs), so it has a form of its own.
+constexpr int kSpmmDepth = 3;
+
+template <typename T, bool NT, bool CAPPED>
 __global__ __launch_bounds__(kThreads) void mfma_spmm_kernel(
     SpmmArgs<T> a, const T* __restrict__ X, T* __restrict__ Y, T* __restrict__ Vout,
     const T* __restrict__ Sub, int64_t ntiles, const int64_t* __restrict__ tptr,
@@ -831,9 +848,7 @@ __global__ __launch_bounds__(kThreads) void mfma_spmm_kernel(
     const int64_t span = (ntiles + V - 1) / V;
     const int64_t b = x * span;
     const int64_t e = b + span < ntiles ? b + span : ntiles;
-    const unsigned int waves = (unsigned int) ((gridDim.x - x + V - 1) / V) * kWavesPerWG;
-    unsigned int* ticket = a.rb.tickets + 64 * x;
-    unsigned int* done = ticket + 32;
+    const int wave = wave_id();
     // block q of the four 16-probe MFMA blocks holds probe
     // Lanes<T>::probe(i0, q), so a lane's four B values of one gathered row
     // take two 16 B loads (FP64) that with lanes 0..15 read whole lines
@@ -841,50 +856,70 @@ __global__ __launch_bounds__(kThreads) void mfma_spmm_kernel(
 #pragma unroll
     for (int q = 0; q < 4; ++q) sq[q] = a.xscale ? (T) a.xscale[Lanes<T>::probe(i0, q)] : T(1);
     const T tt = (T) a.t;
-    for (;;)
+    const int64_t stride = (int64_t) ((gridDim.x - x + V - 1) / V) * kWavesPerWG;
+    double total = 0.0;   // lane (kq, i0): probe Lanes<T>::probe(i0, kq)
+    for (int64_t t = b + (int64_t) (blockIdx.x / V) * kWavesPerWG + wave; t < e; t += stride)
     {
-        unsigned int k = 0;
-        if (lane == 0) k = atomicAdd(ticket, 1u);
-        const int64_t t = b + (int64_t) __builtin_amdgcn_readfirstlane(k);
-        if (t >= e) break;
         V4 acc[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) acc[q] = V4{T(0), T(0), T(0), T(0)};
         const int64_t beg = tptr[t];
-        const int64_t end = tptr[t + 1];
-        for (int64_t base = beg; base < end; base += kWave)
+        const int np = (int) ((tptr[t + 1] - beg) / 8);   // pairs of four-slab groups
+        if (np > 0)
         {
-            const int64_t rem = end - base;
-            const int cnt = rem < kWave ? (int) rem : kWave;   // multiple of 4
-            const int cl = lane < cnt ? tcols[base + lane] : 0;
-            auto col_of = [&](int g) {
-                const int c0 = readlane(cl, 4 * g);
-                const int c1 = readlane(cl, 4 * g + 1);
-                const int c2 = readlane(cl, 4 * g + 2);
-                const int c3 = readlane(cl, 4 * g + 3);
-                return (int64_t) (kq == 0 ? c0 : (kq == 1 ? c1 : (kq == 2 ? c2 : c3)));
-            };
-            // pairs of MFMA groups (eight slabs): one access loads a lane's
-            // A values of both groups
-            const int np = cnt / 8;
-            const Pair2<T>* __restrict__ ap2 =
-                reinterpret_cast<const Pair2<T>*>(tvals + base * 16) + lane;
-            Pair2<T> ap = ap2[0], an;
-            T b0[4], b1[4];
-            Lanes<T>::load(X + col_of(0) * kBlock, i0, b0);
-            for (int P = 0; P < np; ++P)
+            const Pair2<T>* __restrict__ ap = reinterpret_cast<const Pair2<T>*>(tvals + beg * 16) + lane;
+            const int32_t* __restrict__ cp = tcols + beg + kq;
+            constexpr int D = kSpmmDepth;
+            // slot u of D: the values and gathered rows of one pair in flight,
+            // and the columns of the pair D further on
+            Pair2<T> av[D];
+            T b0[D][4], b1[D][4];
+            int32_t c0[D], c1[D];
+#pragma unroll
+            for (int u = 0; u < D; ++u)
             {
-                Lanes<T>::load(X + col_of(2 * P + 1) * kBlock, i0, b1);
+                const int P = u < np ? u : np - 1;
+                c0[u] = cp[8 * P];
+                c1[u] = cp[8 * P + 4];
+            }
 #pragma unroll
-                for (int q = 0; q < 4; ++q) acc[q] = Mfma16<T>::op(ap.x, sq[q] * b0[q], acc[q]);
-                if (P + 1 < np)
+            for (int u = 0; u < D; ++u)
+            {
+                const int P = u < np ? u : np - 1;
+                av[u] = ap[(int64_t) P * kWave];
+                Lanes<T>::load(X + (int64_t) c0[u] * kBlock, i0, b0[u]);
+                Lanes<T>::load(X + (int64_t) c1[u] * kBlock, i0, b1[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < D; ++u)
+            {
+                const int P = u + D < np ? u + D : np - 1;
+                c0[u] = cp[8 * P];
+                c1[u] = cp[8 * P + 4];
+            }
+            for (int P0 = 0; P0 < np; P0 += D)
+            {
+#pragma unroll
+                for (int u = 0; u < D; ++u)
                 {
-                    an = ap2[(P + 1) * kWave];
-                    Lanes<T>::load(X + col_of(2 * P + 2) * kBlock, i0, b0);
-                }
+                    const int P = P0 + u;
+                    if (P >= np) break;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) acc[q] = Mfma16<T>::op(ap.y, sq[q] * b1[q], acc[q]);
-                ap = an;
+                    for (int q = 0; q < 4; ++q)
+                        acc[q] = Mfma16<T>::op(av[u].x, sq[q] * b0[u][q], acc[q]);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        acc[q] = Mfma16<T>::op(av[u].y, sq[q] * b1[u][q], acc[q]);
+                    if (P + D < np)
+                    {
+                        av[u] = ap[(int64_t) (P + D) * kWave];
+                        Lanes<T>::load(X + (int64_t) c0[u] * kBlock, i0, b0[u]);
+                        Lanes<T>::load(X + (int64_t) c1[u] * kBlock, i0, b1[u]);
+                        const int Q = P + 2 * D < np ? P + 2 * D : np - 1;
+                        c0[u] = cp[8 * Q];
+                        c1[u] = cp[8 * Q + 4];
+                    }
+                }
             }
         }
         double red[4] = {0.0, 0.0, 0.0, 0.0};
@@ -907,24 +942,26 @@ __global__ __launch_bounds__(kThreads) void mfma_spmm_kernel(
         }
         if (a.red_mode)
         {
-            double mine = 0.0;
 #pragma unroll
             for (int q = 0; q < 4; ++q)
             {
                 const double r1 = red[q] + __shfl_xor(red[q], 16);
                 const double r2 = r1 + __shfl_xor(r1, 32);
-                if (q == kq) mine = r2;
+                if (q == kq) total += r2;
             }
-            a.rb.tile_partial[t * kWave + Lanes<T>::probe(i0, kq)] = mine;
         }
+        if constexpr (!CAPPED) break;
     }
-    unsigned int d = 0;
-    if (lane == 0) d = atomicAdd(done, 1u);
-    d = __builtin_amdgcn_readfirstlane(d);
-    if (d == waves - 1 && lane == 0)
+    if (!a.red_mode) return;
+    __shared__ double pr[kWavesPerWG][kWave];
+    pr[wave][Lanes<T>::probe(i0, kq)] = total;
+    __syncthreads();
+    if (wave == 0)
     {
-        atomicExch(ticket, 0u);
-        atomicExch(done, 0u);
+        double s = 0.0;
+#pragma unroll
+        for (int w = 0; w < kWavesPerWG; ++w) s += pr[w][lane];
+        a.rb.tile_partial[(int64_t) blockIdx.x * kWave + lane] = s;
     }
 }
 
@@ -1403,6 +1440,10 @@ int dense_ksplit(int64_t nrows, int64_t ncols)
 // total_kernel (one workgroup) adds the rows of rb.partial in order and
 // stores the total like the SpMM's own reduction.
 constexpr int kTileSumGrid = 256;
+// Partial rows that total_kernel adds by itself: up to here (65536 rows of
+// 16-row tiles) a second launch, 4.7 us however small, costs more than the
+// longer sum.
+constexpr int kTotalRows = 512;
 
 __global__ __launch_bounds__(kThreads) void tile_sum_kernel(const double* __restrict__ tp,
                                                             int64_t ntiles,
@@ -1437,9 +1478,10 @@ __global__ __launch_bounds__(kThreads) void tile_sum_kernel(const double* __rest
 }
 
 template <typename T>
-__global__ __launch_bounds__(kTotalWaves * kWave) void total_kernel(SpmmArgs<T> a, int G)
+__global__ __launch_bounds__(kTotalWaves * kWave) void total_kernel(
+    SpmmArgs<T> a, const double* __restrict__ rows, int G)
 {
-    const double t = ordered_total(a.rb.partial, G);
+    const double t = ordered_total(rows, G);
     if (threadIdx.x >= kWave) return;
     spmm_store_total(a, t, threadIdx.x);
 }
@@ -2007,6 +2049,16 @@ __global__ __launch_bounds__(256) void copy_block_kernel(const T* __restrict__ i
 // Grid of a sweep over `units`: at most kMaxGrid workgroups (4 per CU at 8
 // wavefronts each, i.e. one resident wave of workgroups), at least one
 // wavefront-unit each, a multiple of 8 (one share per XCD).
+// SLQ_GRID (0: unset), which also caps the matrix-core SpMM.
+int spmm_grid_env()
+{
+    static const int v = [] {
+        const char* e = std::getenv("SLQ_GRID");
+        return e ? std::atoi(e) : 0;
+    }();
+    return v;
+}
+
 int max_grid()
 {
     static int g = [] {
@@ -2097,7 +2149,8 @@ int64_t sched_tiles(const slq_op* op)
     if (A.tiles.R == 0) return 0;
     const int64_t R = A.tiles.R;
     const int64_t a = (A.csr.nrows + R - 1) / R, b = (A.csr.ncols + R - 1) / R;
-    return (a > b ? a : b) * (R == 16 ? spmm_split(op) : 1);
+    // at least the eight partial rows of the smallest grid
+    return std::max<int64_t>((a > b ? a : b) * (R == 16 ? spmm_split(op) : 1), kXcds);
 }
 
 RedBuf take_redbuf(Bump& bump, int64_t tiles)
@@ -2362,7 +2415,7 @@ void launch_spmm_nt(slq_op* op, const SpmmArgs<T>& s, const SpmmIO<T>& io, const
         }
         if (s.red_mode)
             hipLaunchKernelGGL((total_kernel<T>), dim3(1), dim3(kTotalWaves * kWave), 0,
-                               op->stream, s, rg);
+                               op->stream, s, (const double*) s.rb.partial, rg);
         return;
     }
     if (tl)
@@ -2375,6 +2428,8 @@ void launch_spmm_nt(slq_op* op, const SpmmArgs<T>& s, const SpmmIO<T>& io, const
         // launch_spmm has checked the counters and partial rows
         {
             const int split = tl->R == 16 ? spmm_split(op) : 1;
+            // partial rows of the reduction term
+            int64_t prows = tl->ntiles * split;
             if (tl->R == 16 && split == 2)
                 hipLaunchKernelGGL((mfma_spmm_split_kernel<T, NT, 2>), dim3(grid),
                                    dim3(kThreads), 0, op->stream, s, io.X, io.Y, io.Vout,
@@ -2384,22 +2439,38 @@ void launch_spmm_nt(slq_op* op, const SpmmArgs<T>& s, const SpmmIO<T>& io, const
                                    dim3(kThreads), 0, op->stream, s, io.X, io.Y, io.Vout,
                                    io.Sub, tl->ntiles, tl->ptr, tl->cols, tv);
             else if (tl->R == 16)
-                hipLaunchKernelGGL((mfma_spmm_kernel<T, NT>), dim3(grid), dim3(kThreads), 0,
-                                   op->stream, s, io.X, io.Y, io.Vout, io.Sub, tl->ntiles,
-                                   tl->ptr, tl->cols, tv);
+            {
+                // a workgroup per eight tiles unless the launch settings cap it
+                const int64_t span = (tl->ntiles + kXcds - 1) / kXcds;
+                int64_t g = (span + kWavesPerWG - 1) / kWavesPerWG * kXcds;
+                prows = g;
+                const int cap = op->spmm_grid > 0 ? op->spmm_grid : spmm_grid_env();
+                if (cap > 0 && g > cap) g = cap < kXcds ? kXcds : cap / kXcds * kXcds;
+                const bool capped = g < prows;
+                prows = g;
+                auto kern = capped ? mfma_spmm_kernel<T, NT, true>
+                                   : mfma_spmm_kernel<T, NT, false>;
+                hipLaunchKernelGGL(kern, dim3((unsigned) g), dim3(kThreads), 0, op->stream, s,
+                                   io.X, io.Y, io.Vout, io.Sub, tl->ntiles, tl->ptr, tl->cols,
+                                   tv);
+            }
             else
                 hipLaunchKernelGGL((tiled_spmm_sched_kernel<T, 8, NT>), dim3(grid),
                                    dim3(kThreads), 0, op->stream, s, io.X, io.Y, io.Vout,
                                    io.Sub, tl->ntiles, tl->ptr, tl->cols, tv);
             if (s.red_mode)
             {
-                const int64_t prows = tl->ntiles * split;
-                int rg = (int) ((prows + 63) / 64);
-                rg = rg < 1 ? 1 : (rg > kTileSumGrid ? kTileSumGrid : rg);
-                hipLaunchKernelGGL(tile_sum_kernel, dim3(rg), dim3(kThreads), 0, op->stream,
-                                   (const double*) s.rb.tile_partial, prows, s.rb.partial);
+                const double* rows = s.rb.tile_partial;
+                int rg = (int) prows;
+                if (prows > kTotalRows)
+                {
+                    rg = (int) std::min<int64_t>((prows + 63) / 64, kTileSumGrid);
+                    hipLaunchKernelGGL(tile_sum_kernel, dim3(rg), dim3(kThreads), 0,
+                                       op->stream, rows, prows, s.rb.partial);
+                    rows = s.rb.partial;
+                }
                 hipLaunchKernelGGL((total_kernel<T>), dim3(1), dim3(kTotalWaves * kWave), 0,
-                                   op->stream, s, rg);
+                                   op->stream, s, rows, rg);
             }
         }
     }
@@ -2445,7 +2516,7 @@ void launch_spmm_nt(slq_op* op, const SpmmArgs<T>& s, const SpmmIO<T>& io, const
                            io.Vout, io.Sub, csr_blocked_cols(s), sync);
         if (s.red_mode)
             hipLaunchKernelGGL((total_kernel<T>), dim3(1), dim3(kTotalWaves * kWave), 0,
-                               op->stream, s, grid);
+                               op->stream, s, (const double*) s.rb.partial, grid);
     }
     else
     {
@@ -2454,7 +2525,7 @@ void launch_spmm_nt(slq_op* op, const SpmmArgs<T>& s, const SpmmIO<T>& io, const
                            io.X, io.Y, io.Vout, io.Sub);
         if (s.red_mode)
             hipLaunchKernelGGL((total_kernel<T>), dim3(1), dim3(kTotalWaves * kWave), 0,
-                               op->stream, s, grid);
+                               op->stream, s, (const double*) s.rb.partial, grid);
     }
 }
 
