@@ -27,6 +27,12 @@ namespace slq {
 namespace {
 
 constexpr int kChunkWords = 64;   // words generated per thread after the jump
+// Chunks per wavefront, a power of two up to 64. What bounds generation is
+// the chain of GF(2) products before the words, about 1 us each: one per set
+// bit of the offset and one per lane but the first. 64 chunks took 61 us
+// for probes of a single word and 75 us at n = 2^20; with 8 (and no more lanes
+// than the probe has chunks) @@RNG@@.
+constexpr int kGroupChunks = 8;
 
 inline uint64_t rotl_h(uint64_t x, int k) { return (x << k) | (x >> (64 - k)); }
 
@@ -159,12 +165,13 @@ __device__ __forceinline__ void apply_wave(const uint64_t* __restrict__ M, const
 
 static_assert(kChunkWords == 64, "lane states are spaced by jump tables 6 + k");
 
-// One wavefront per (probe p, group g of 64 chunks): lane l generates words
-// [c L, min((c + 1) L, W)) of probe p, c = 64 g + l, i.e. stream words from
-// offset (first_sample + p) W + c L. The wavefront jumps the base state to
-// the group's first chunk with the matrices of the set bits of that offset,
-// then spreads it to its lanes by doubling (lanes s + 2^k take M^(2^k L) of
-// lane s, k = 0..5), every product computed by the whole wavefront.
+// One wavefront per (probe p, group g of kGroupChunks chunks): lane l
+// generates words [c L, min((c + 1) L, W)) of probe p, c = kGroupChunks g +
+// l, i.e. stream words from offset (first_sample + p) W + c L. The wavefront
+// jumps the base state to the group's first chunk with the matrices of the
+// set bits of that offset, then spreads it to the lanes that have a chunk by
+// doubling (lanes s + 2^k take M^(2^k L) of lane s), every product computed
+// by the whole wavefront.
 __global__ __launch_bounds__(256) void rng_words_kernel(
     const uint64_t* __restrict__ tables, uint64_t s0, uint64_t s1, uint64_t s2,
     uint64_t s3, int64_t W, int64_t first_sample, int32_t count, int64_t chunks,
@@ -176,15 +183,17 @@ __global__ __launch_bounds__(256) void rng_words_kernel(
     const int64_t g = wv - p * groups;
     if (p >= count) return;
     const uint64_t offset = (uint64_t) (first_sample + p) * (uint64_t) W +
-                            (uint64_t) (g * kWave * kChunkWords);
+                            (uint64_t) (g * kGroupChunks * kChunkWords);
     uint64_t x[4] = {s0, s1, s2, s3};
     for (int e = 0; e < 64; ++e)
         if ((offset >> e) & 1) apply_wave(tables + (size_t) e * 256 * 4, x, x, lane);
     uint64_t st[4] = {x[0], x[1], x[2], x[3]};
-    for (int k = 0; k < 6; ++k)
+    const int64_t left = chunks - g * kGroupChunks;
+    const int lanes = left < kGroupChunks ? (int) left : kGroupChunks;
+    for (int k = 0; (1 << k) < lanes; ++k)
     {
         const int half = 1 << k;
-        for (int src = 0; src < half; ++src)
+        for (int src = 0; src < half && src + half < lanes; ++src)
         {
             uint64_t v[4], r[4];
 #pragma unroll
@@ -197,8 +206,8 @@ __global__ __launch_bounds__(256) void rng_words_kernel(
             }
         }
     }
-    const int64_t c = g * kWave + lane;
-    if (c >= chunks) return;
+    const int64_t c = g * kGroupChunks + lane;
+    if (lane >= lanes) return;
     uint64_t x0 = st[0], x1 = st[1], x2 = st[2], x3 = st[3];
     uint64_t* out = words + p * W;
     const int64_t beg = c * kChunkWords;
@@ -300,7 +309,7 @@ int rng_words(hipStream_t s, const uint64_t base[4], int64_t W,
     }
     if (count <= 0) return SLQ_OK;
     const int64_t chunks = (W + kChunkWords - 1) / kChunkWords;
-    const int64_t groups = (chunks + kWave - 1) / kWave;
+    const int64_t groups = (chunks + kGroupChunks - 1) / kGroupChunks;
     const int64_t threads = groups * count * kWave;
     const int64_t grid = (threads + 255) / 256;
     hipLaunchKernelGGL(rng_words_kernel, dim3((unsigned) grid), dim3(256), 0, s,
