@@ -2578,7 +2578,11 @@ int estimate_loop(slq_op* op, const Plan& p, EstimateArgs a)
     // than min_num_samples processed by its end) the next block's probes
     // and recurrence are queued before the host waits for it. The kernels
     // and their inputs are those of the plain order, so results are equal.
-    const bool pipelined = p.pipeline && p.lanes == 0 && required == 1 && !a.krylov;
+    // A single block has nothing to overlap with: it keeps to one stream
+    // (the second one's creation, events and hand-over took 25 us, and 0.2 ms
+    // with its destruction for a handle used once).
+    const bool pipelined = p.pipeline && p.lanes == 0 && required == 1 && !a.krylov &&
+                           a.max_s > bs;
     if (pipelined && !op->aux_stream)
         SLQ_CHECK(hipStreamCreateWithFlags(&op->aux_stream, hipStreamNonBlocking));
     hipStream_t qstream = pipelined ? op->aux_stream : op->stream;

@@ -1997,16 +1997,23 @@ __global__ __launch_bounds__(kTotalWaves * kWave) void reduce_partials_kernel(
     if (threadIdx.x < kWave) out[k * kWave + threadIdx.x] = t;
 }
 
-// Block set-up: scale[p] = s0 for probes p < count (0 otherwise), sizes = 0.
-__global__ void init_block_kernel(double* scale, int32_t* sizes, int count,
-                                  double s0)
+// Set-up of a recurrence in one launch: scale = s0 and sizes = 0 for every
+// probe of the block, scale2 = s1 with sizes2 = 0 where given, and the
+// counters of its kernels cleared.
+__global__ __launch_bounds__(kThreads) void init_block_kernel(
+    double* scale, int32_t* sizes, double s0, double* scale2, int32_t* sizes2, double s1,
+    unsigned int* tickets, int ntickets, int* words, int nwords)
 {
     const int p = threadIdx.x;
     if (p < kBlock)
     {
-        scale[p] = p < count ? s0 : 0.0;
+        scale[p] = s0;
         sizes[p] = 0;
+        if (scale2) scale2[p] = s1;
+        if (sizes2) sizes2[p] = 0;
     }
+    for (int i = p; i < ntickets; i += kThreads) tickets[i] = 0u;
+    for (int i = p; i < nwords; i += kThreads) words[i] = 0;
 }
 
 __global__ void zero_u32_kernel(unsigned int* p, int n)
@@ -2022,18 +2029,13 @@ __global__ void convert_kernel(const S* __restrict__ in, D* __restrict__ out, in
     if (i < n) out[i] = (D) in[i];
 }
 
-// X[i][p] *= scale[p]; then scale[p] = 1 (second launch, after every reader).
+// X[i][p] *= scale[p].
 template <typename T>
 __global__ __launch_bounds__(256) void scale_rows_kernel(T* __restrict__ X, int64_t n,
                                                          const double* __restrict__ scale)
 {
     const int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n * kBlock) X[i] = (T) ((double) X[i] * scale[i % kBlock]);
-}
-
-__global__ void set_ones_kernel(double* s)
-{
-    if (threadIdx.x < kBlock) s[threadIdx.x] = 1.0;
 }
 
 template <typename T>
@@ -2168,13 +2170,18 @@ bool redbuf_ok(const RedBuf& rb)
     return rb.partial && rb.tickets;
 }
 
-void zero_counters(hipStream_t s, const RedBuf& rb, int* gs_words = nullptr, int n = 0)
+void zero_counters(hipStream_t s, const RedBuf& rb)
 {
     hipLaunchKernelGGL(zero_u32_kernel, dim3(kTicketWords / 64), dim3(64), 0, s, rb.tickets,
                        kTicketWords);
-    if (gs_words)
-        hipLaunchKernelGGL(zero_u32_kernel, dim3((n + 63) / 64), dim3(64), 0, s,
-                           (unsigned int*) gs_words, n);
+}
+
+void init_block(hipStream_t s, double* scale, int32_t* sizes, double s0, const RedBuf& rb,
+                double* scale2 = nullptr, int32_t* sizes2 = nullptr, double s1 = 0.0,
+                int* words = nullptr, int nwords = 0)
+{
+    hipLaunchKernelGGL(init_block_kernel, dim3(1), dim3(kThreads), 0, s, scale, sizes, s0,
+                       scale2, sizes2, s1, rb.tickets, kTicketWords, words, nwords);
 }
 
 size_t redbuf_bytes(int64_t tiles)
@@ -2692,13 +2699,14 @@ int reorthogonalize(slq_op* op, int64_t nrows, T* R, const T* basis, size_t slot
     return SLQ_OK;
 }
 
+// X[i][p] *= scale[p]: the stored basis of a re-orthogonalised Golub-Kahn
+// run is normalised, and read with unit scales.
 template <typename T>
-int normalize_in_place(slq_op* op, T* X, int64_t n, double* scale)
+int normalize_in_place(slq_op* op, T* X, int64_t n, const double* scale)
 {
     const int64_t g = (n * kBlock + 255) / 256;
     hipLaunchKernelGGL(scale_rows_kernel<T>, dim3((unsigned) g), dim3(256), 0,
-                       op->stream, X, n, (const double*) scale);
-    hipLaunchKernelGGL(set_ones_kernel, dim3(1), dim3(kBlock), 0, op->stream, scale);
+                       op->stream, X, n, scale);
     SLQ_CHECK(hipGetLastError());
     return SLQ_OK;
 }
@@ -2740,10 +2748,8 @@ int lanczos_ring(const RecurrenceArgs& ra, Bump& bump)
         set_error("internal: Lanczos workspace too small");
         return SLQ_E_OOM;
     }
-    zero_counters(op->stream, rb);
     const double s0 = 1.0 / std::sqrt((double) n);
-    hipLaunchKernelGGL(init_block_kernel, dim3(1), dim3(kBlock), 0, op->stream,
-                       S[0], ra.sizes, kBlock, s0);
+    init_block(op->stream, S[0], ra.sizes, s0, rb);
     SLQ_CHECK(hipGetLastError());
     const double tol_sqrt_n = ra.tol * std::sqrt((double) n);
     const DevTiles* tl = nullptr;
@@ -2838,13 +2844,10 @@ int lanczos(const RecurrenceArgs& ra, Bump& bump)
         set_error("internal: Lanczos workspace too small");
         return SLQ_E_OOM;
     }
-    zero_counters(op->stream, rb, again, kGsWords);
-    hipLaunchKernelGGL(set_ones_kernel, dim3(1), dim3(kBlock), 0, op->stream, ones);
     const bool beta_in_spmm = spmm_beta_enabled();
     // initial_beta = |probe| = sqrt(n) exactly for a Rademacher probe
     const double s0 = 1.0 / std::sqrt((double) n);
-    hipLaunchKernelGGL(init_block_kernel, dim3(1), dim3(kBlock), 0, op->stream,
-                       scale, ra.sizes, kBlock, s0);
+    init_block(op->stream, scale, ra.sizes, s0, rb, ones, nullptr, 1.0, again, kGsWords);
     SLQ_CHECK(hipGetLastError());
     const double tol_sqrt_n = ra.tol * std::sqrt((double) n);
     const DevTiles* tl = nullptr;
@@ -2935,28 +2938,27 @@ int golub_kahn(const RecurrenceArgs& ra, Bump& bump)
     double* sv = bump.take<double>((size_t) (m + 1) * kBlock);   // 1/beta_{j-1}
     const RedBuf rb = take_redbuf(bump, sched_tiles(op));
     int32_t* usizes = bump.take<int32_t>(kBlock);
+    double* ones = nullptr;   // scales of the normalised basis
     double* h = nullptr;
     int* again = nullptr;
     double* partial_k = nullptr;
     if (reorth)
     {
+        ones = bump.take<double>(kBlock);
         h = bump.take<double>((size_t) (m + 1) * kBlock);
         again = bump.take<int>(kGsWords);
         partial_k = bump.take<double>((size_t) kMaxGrid * (m + 1) * kBlock);
     }
     if (!U || !V || !su || !sv || !redbuf_ok(rb) || !usizes ||
-        (reorth && (!h || !again || !partial_k)))
+        (reorth && (!ones || !h || !again || !partial_k)))
     {
         set_error("internal: Golub-Kahn workspace too small");
         return SLQ_E_OOM;
     }
-    zero_counters(op->stream, rb, again, kGsWords);
     // v_0 = probe / |probe|, |probe| = sqrt(ncols) exactly
     const double s0 = 1.0 / std::sqrt((double) nc);
-    hipLaunchKernelGGL(init_block_kernel, dim3(1), dim3(kBlock), 0, op->stream,
-                       sv, ra.sizes, kBlock, s0);
-    hipLaunchKernelGGL(init_block_kernel, dim3(1), dim3(kBlock), 0, op->stream,
-                       su, usizes, kBlock, 0.0);
+    init_block(op->stream, sv, ra.sizes, s0, rb, ones, usizes, 1.0, again,
+               again ? kGsWords : 0);
     SLQ_CHECK(hipGetLastError());
     auto uslot = [&](int j) { return U + (size_t) (reorth ? j : j % 3) * ust; };
     auto vslot = [&](int j) { return V + (size_t) (reorth ? j : j % 3) * vst; };
@@ -2985,7 +2987,7 @@ int golub_kahn(const RecurrenceArgs& ra, Bump& bump)
         s.shift_mode = mode_a;
         s.shift_len = shift_len;
         s.t = ra.t;
-        s.xscale = sv + (size_t) j * kBlock;
+        s.xscale = reorth ? ones : sv + (size_t) j * kBlock;
         SpmmIO<T> io;
         io.X = vslot(j);
         io.Y = uslot(j);
@@ -2993,7 +2995,7 @@ int golub_kahn(const RecurrenceArgs& ra, Bump& bump)
         {
             io.Sub = uslot(j - 1);
             s.sub_coef = ra.beta + (size_t) (j - 1) * kBlock;
-            s.sub_scale = su + (size_t) (j - 1) * kBlock;
+            s.sub_scale = reorth ? ones : su + (size_t) (j - 1) * kBlock;
         }
         s.red_mode = reorth ? 0 : 2;
         s.finish_sqrt = 1;
@@ -3020,13 +3022,13 @@ int golub_kahn(const RecurrenceArgs& ra, Bump& bump)
         t.shift_mode = mode_t;
         t.shift_len = shift_len;
         t.t = ra.t;
-        t.xscale = su + (size_t) j * kBlock;
+        t.xscale = reorth ? ones : su + (size_t) j * kBlock;
         SpmmIO<T> io2;
         io2.X = uslot(j);
         io2.Y = vslot(j + 1);
         io2.Sub = vslot(j);
         t.sub_coef = ra.alpha + (size_t) j * kBlock;
-        t.sub_scale = sv + (size_t) j * kBlock;
+        t.sub_scale = reorth ? ones : sv + (size_t) j * kBlock;
         t.red_mode = reorth ? 0 : 2;
         t.finish_sqrt = 1;
         t.rb = rb;
@@ -3086,6 +3088,7 @@ size_t recurrence_scratch_bytes(const slq_op* op, int gram, int m, int ortho,
         add(sizeof(double) * (m + 1) * kBlock);
         add(sizeof(double) * (m + 1) * kBlock);
         add(sizeof(int32_t) * kBlock);
+        if (reorth) add(sizeof(double) * kBlock);
     }
     b += redbuf_bytes(sched_tiles(op));
     if (reorth)
