@@ -1747,12 +1747,16 @@ int slq_op_create_csr(int64_t nrows, int64_t ncols, int64_t nnz,
     // here rather than let a kernel read outside its buffers. The columns are
     // looked over on the device; on the host only where that is not done, or
     // to name the column it found.
+    int64_t max_row = 0;
     for (int64_t r = 0; r < nrows; ++r)
+    {
         if (indptr[r + 1] < indptr[r])
         {
             set_error("slq_op_create_csr: indptr decreases at row %lld", (long long) r);
             return SLQ_E_ARG;
         }
+        max_row = std::max(max_row, indptr[r + 1] - indptr[r]);
+    }
     auto check_columns = [&]() -> int {
         for (int64_t k = 0; k < nnz; ++k)
             if (indices[k] < 0 || (int64_t) indices[k] >= ncols)
@@ -1783,6 +1787,7 @@ int slq_op_create_csr(int64_t nrows, int64_t ncols, int64_t nnz,
     c.ncols = ncols;
     c.nnz = nnz;
     c.dtype = dtype;
+    c.max_row = max_row;
     const size_t vb = dtype == SLQ_F64 ? 8 : 4;
     auto fail = [&](int code) {
         if (op->stream) (void) hipStreamDestroy(op->stream);
@@ -1978,6 +1983,7 @@ int slq_op_create_sparse_gaussian(int64_t nrows, int64_t ncols, int32_t per_row,
     c.nrows = nrows;
     c.ncols = ncols;
     c.nnz = nrows * per_row;
+    c.max_row = per_row;
     c.dtype = dtype;
     c.sorted = c.strict = true;   // one entry per column stratum, strata in order
     const size_t vb = dtype == SLQ_F64 ? 8 : 4;
@@ -3139,6 +3145,7 @@ int slq_op_set_launch(slq_op* op, int32_t spmm_grid, int32_t stream_grid,
     op->stream_grid = stream_grid;
     op->spmm_split = spmm_split;
     op->tile_mode = tile_mode;
+    op->user_launch = spmm_grid || stream_grid || spmm_split || tile_mode;
     return SLQ_OK;
 }
 

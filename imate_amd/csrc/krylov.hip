@@ -3102,6 +3102,7 @@ size_t recurrence_scratch_bytes(const slq_op* op, int gram, int m, int ortho,
 
 int run_recurrence(const RecurrenceArgs& ra, void* scratch, size_t scratch_bytes)
 {
+    if (resident_fits(ra.op, ra.gram, ra.ortho)) return run_resident(ra);
     Bump bump{(char*) scratch, scratch_bytes};
     const bool f32 = ra.precision == SLQ_PREC_MIXED || ra.op->A->csr.dtype == SLQ_F32;
     if (ra.gram && !ra.op->A->has_trans && !ra.op->A->dn.trans)

@@ -36,6 +36,7 @@
 #include "slq_internal.hpp"
 #include "ql.hpp"
 #include "dc.hpp"
+#include "lanes.hpp"
 
 namespace slq {
 
@@ -47,46 +48,18 @@ constexpr int kDcMaxRows = 1024;
 // Inquiries up to which the threads share the nodes of one inquiry.
 constexpr int kFewInquiries = 8;
 
-// Lane l's value from the lane that Ctrl names (row operations within 16
-// lanes; every lane of the row is read, so all of its lanes must be active).
-template <int Ctrl>
-__device__ __forceinline__ int dpp(int x)
-{
-    return __builtin_amdgcn_update_dpp(0, x, Ctrl, 0xf, 0xf, true);
-}
-
-template <int Ctrl>
-__device__ __forceinline__ double dpp(double x)
-{
-    const uint64_t u = __builtin_bit_cast(uint64_t, x);
-    const uint32_t lo = (uint32_t) dpp<Ctrl>((int) (uint32_t) u);
-    const uint32_t hi = (uint32_t) dpp<Ctrl>((int) (uint32_t) (u >> 32));
-    return __builtin_bit_cast(double, ((uint64_t) hi << 32) | lo);
-}
-
 struct Workgroup {
     int tid, nt;
     __device__ __forceinline__ void sync() const { __syncthreads(); }
-    // Sum / product over P = 1, 2, 4, 8 or 16 neighbouring lanes, the same
-    // value in each: lane ^ 1, ^ 2 (quad permutes), then the mirrored half
-    // row and row, whose lanes already agree within quads and halves.
     template <int P, typename T>
     __device__ __forceinline__ T sum(T x) const
     {
-        if constexpr (P > 1) x += dpp<0xB1>(x);
-        if constexpr (P > 2) x += dpp<0x4E>(x);
-        if constexpr (P > 4) x += dpp<0x141>(x);
-        if constexpr (P > 8) x += dpp<0x140>(x);
-        return x;
+        return lanes_sum<P>(x);
     }
     template <int P>
     __device__ __forceinline__ double prod(double x) const
     {
-        if constexpr (P > 1) x *= dpp<0xB1>(x);
-        if constexpr (P > 2) x *= dpp<0x4E>(x);
-        if constexpr (P > 4) x *= dpp<0x141>(x);
-        if constexpr (P > 8) x *= dpp<0x140>(x);
-        return x;
+        return lanes_product<P>(x);
     }
 };
 

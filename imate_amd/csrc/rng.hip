@@ -31,7 +31,7 @@ constexpr int kChunkWords = 64;   // words generated per thread after the jump
 // the chain of GF(2) products before the words, about 1 us each: one per set
 // bit of the offset and one per lane but the first. 64 chunks took 61 us
 // for probes of a single word and 75 us at n = 2^20; with 8 (and no more lanes
-// than the probe has chunks) @@RNG@@.
+// than the probe has chunks) 13 us at n = 1003, 27 at 4099, 66 at 2^20.
 constexpr int kGroupChunks = 8;
 
 inline uint64_t rotl_h(uint64_t x, int k) { return (x << k) | (x >> (64 - k)); }

@@ -64,6 +64,7 @@ struct DevCSR {
     void* data = nullptr;
     bool sorted = false;   // column indices non-decreasing within every row
     bool strict = false;   // sorted, and no row repeats a column
+    int64_t max_row = 0;   // entries of the longest row (matrices given by the caller)
 };
 
 // Row-tiled "column slab" form of a CSR matrix for the SpMM. Rows are grouped
@@ -250,6 +251,9 @@ struct slq_op {
     // 1 the CSR rows (tuned: 0 = not tuned, else mode + 1)
     int tile_mode = 0;
     int tuned_tile_mode = 0;
+    // launch settings were given (slq_op_set_launch): estimates keep to the
+    // block kernels they are about
+    bool user_launch = false;
     // rocBLAS handle of the block Krylov form's eigensolver (first use)
     void* rocblas = nullptr;
 };
@@ -281,6 +285,10 @@ struct RecurrenceArgs {
     int32_t* sizes = nullptr;   // device [kBlock]
 };
 int run_recurrence(const RecurrenceArgs& a, void* scratch, size_t scratch_bytes);
+// Lanczos of a small matrix in one launch (resident.hip), and whether a
+// recurrence on `op` takes it.
+bool resident_fits(const slq_op* op, int gram, int ortho);
+int run_resident(const RecurrenceArgs& a);
 size_t recurrence_scratch_bytes(const slq_op* op, int gram, int m, int ortho,
                                 int value_bytes);
 
