@@ -16,6 +16,12 @@ __device__ __forceinline__ int dpp(int x)
 }
 
 template <int Ctrl>
+__device__ __forceinline__ float dpp(float x)
+{
+    return __builtin_bit_cast(float, dpp<Ctrl>(__builtin_bit_cast(int, x)));
+}
+
+template <int Ctrl>
 __device__ __forceinline__ double dpp(double x)
 {
     const uint64_t u = __builtin_bit_cast(uint64_t, x);

@@ -17,6 +17,7 @@
 #include <cstring>
 #include <vector>
 
+#include "lanes.hpp"
 #include "slq_internal.hpp"
 
 namespace slq {
@@ -42,174 +43,303 @@ __device__ __forceinline__ float dsilu(float z)
 
 // ---------------------------------------------------------------- training
 
-// One workgroup of H threads per sample: z1, z2 (pre-activations) and y.
-__global__ __launch_bounds__(H) void mlp_forward_kernel(const float* __restrict__ P,
-                                                        const float* __restrict__ x, int B,
-                                                        float* __restrict__ z1,
-                                                        float* __restrict__ z2,
-                                                        float* __restrict__ y)
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f32x4 mfma(float a, float b, f32x4 c)
 {
-    __shared__ float h1[H];
-    __shared__ float red[H];
-    const int b = blockIdx.x;
-    const int j = threadIdx.x;
-    if (b >= B) return;
-    const float x0 = x[2 * b], x1 = x[2 * b + 1];
-    const float a1 = P[kW1 + 2 * j] * x0 + P[kW1 + 2 * j + 1] * x1 + P[kB1 + j];
-    z1[(size_t) b * H + j] = a1;
-    h1[j] = silu(a1);
-    __syncthreads();
-    float a2 = P[kB2 + j];
-    const float* w = P + kW2 + (size_t) j * H;
-    for (int k = 0; k < H; ++k) a2 += w[k] * h1[k];
-    z2[(size_t) b * H + j] = a2;
-    red[j] = P[kW3 + j] * silu(a2);
-    __syncthreads();
-    for (int s = H / 2; s > 0; s >>= 1)
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+constexpr int kTrainThreads = 512;           // 8 wavefronts, 16 hidden units each
+constexpr int kTrainWaves = kTrainThreads / 64;
+constexpr int kTrainTiles = 1;               // 16-sample tiles a workgroup holds
+constexpr int kTrainSamples = 16 * kTrainTiles;
+constexpr int kTrainGroups = 256;            // most workgroups (partial gradients)
+constexpr int kFirst = kTrainSamples * H / kTrainThreads;   // first-layer values per thread
+constexpr int kPad = H + 4;                  // LDS row stride, see below
+static_assert(kTrainWaves * 16 == H && kTrainSamples <= 64, "wavefront split");
+
+// Samples per workgroup for a batch of B: one tile each up to half a
+// workgroup per CU, then at least two (half the partial gradients to write
+// and add: 96 steps at B = 4000 took 2.79 against 2.91 ms), and no more
+// workgroups than CUs (64000 samples: 9.9 ms, 16.5 ms on half of the CUs).
+inline int train_chunk(int B)
+{
+    const int tiles = (B + kTrainSamples - 1) / kTrainSamples;
+    if (tiles <= kTrainGroups / 2) return kTrainSamples;
+    const int per = (tiles + kTrainGroups - 1) / kTrainGroups;
+    return (per > 2 ? per : 2) * kTrainSamples;
+}
+
+inline int train_groups(int B)
+{
+    const int chunk = train_chunk(B);
+    return (B + chunk - 1) / chunk;
+}
+
+// Loss and gradient of a chunk of samples in one launch: forward,
+// back-propagation and the sums over the chunk, the three 128 x 128 products
+// on the FP32 matrix instruction (v_mfma_f32_16x16x4_f32: lane l holds
+// A[l % 16][l / 16] and B[l / 16][l % 16], and D[4 (l / 16) + i][l % 16]).
+//
+// Wavefront w owns hidden units 16 w .. 16 w + 15 (columns of z2 and z1, rows
+// of dW2). Its rows and its columns of W2 stay in registers; activations
+// cross between wavefronts through LDS. The order of the reduction index
+// within an operand is free as long as both operands agree: lane group g
+// takes indices 4 g .. 4 g + 3 of each 16, which makes the reads of h1 and d2
+// by row 16 bytes wide, and the row stride of 132 words keeps them, and the
+// reads by column of the gradient's product, on distinct LDS banks.
+//
+// What bounds it: latency, not the 98 kFLOP per sample (0.2 GFLOP, 1.3 us at
+// the matrix rate, for B = 2000): the loads of W2, a chain of 32 matrix
+// instructions per product, four exchanges through LDS, and the 68 KB of
+// sums per workgroup. 14.9 us at B = 2000 with 16 samples per workgroup
+// (17.2 with 32, 25.2 with 64); a workgroup per sample for the forward pass
+// and the back-propagation and a thread per parameter for the sums, which
+// this replaces, took 27.2 us together and 36.8 us.
+//
+// A chunk's sums go to partial[chunk]; mlp_update_kernel adds the chunks in
+// order, so results do not depend on scheduling. step, if given, is advanced
+// here: the update of the previous step has read it, the next has not.
+__global__ __launch_bounds__(kTrainThreads) void mlp_train_kernel(
+    const float* __restrict__ P, const float* __restrict__ x,
+    const float* __restrict__ target, int B, int chunk, float* __restrict__ partial,
+    float* __restrict__ loss_partial, int* __restrict__ step)
+{
+    __shared__ __align__(16) float h1[kTrainSamples][kPad];
+    __shared__ __align__(16) float d2[kTrainSamples][kPad];
+    __shared__ float xs[kTrainSamples][2];
+    __shared__ float ys[kTrainWaves][kTrainSamples];
+    __shared__ float d3[kTrainSamples];
+    const int lane = threadIdx.x % 64;
+    const int w = threadIdx.x / 64;
+    const int col = lane % 16, g = lane / 16;
+    const int unit = 16 * w + col;
+    const int b0 = blockIdx.x * chunk;
+    const int b1 = b0 + chunk < B ? b0 + chunk : B;
+    if (step && blockIdx.x == 0 && threadIdx.x == 0) *step += 1;
+
+    // loads in the order of their use: a wait for one waits for all before it
+    const int j1 = threadIdx.x % H;          // unit of the thread's first layer
+    const int s1 = threadIdx.x / H;          // its samples: s1, s1 + kTrainThreads / H, ...
+    float xin[kFirst][2], tin;
+    const auto load_samples = [&](int b) {
+        const int n = b1 - b;
+#pragma unroll
+        for (int i = 0; i < kFirst; ++i)
+        {
+            const int s = s1 + i * (kTrainThreads / H);
+            xin[i][0] = s < n ? x[2 * (b + s)] : 0.f;
+            xin[i][1] = s < n ? x[2 * (b + s) + 1] : 0.f;
+        }
+        const int s = threadIdx.x;
+        tin = s < kTrainSamples && s < n ? target[b + s] : 0.f;
+    };
+    load_samples(b0);
+    const float v1x = P[kW1 + 2 * j1], v1y = P[kW1 + 2 * j1 + 1], c1 = P[kB1 + j1];
+    const float w1x = P[kW1 + 2 * unit], w1y = P[kW1 + 2 * unit + 1], bias1 = P[kB1 + unit];
+    const float bias2 = P[kB2 + unit], w3 = P[kW3 + unit], bias3 = P[kB3];
+    f32x4 wrow[H / 16];             // W2[unit][16 k + 4 g + 0..3]
+    float wcol[H / 16][4];          // W2[16 k + 4 g + 0..3][unit]
+#pragma unroll
+    for (int k = 0; k < H / 16; ++k)
+        wrow[k] = *(const f32x4*) (P + kW2 + unit * H + 16 * k + 4 * g);
+#pragma unroll
+    for (int k = 0; k < H / 16; ++k)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) wcol[k][t] = P[kW2 + (16 * k + 4 * g + t) * H + unit];
+
+    f32x4 gw2[H / 16] = {};
+    float gw1x = 0.f, gw1y = 0.f, gb1 = 0.f, gb2 = 0.f, gw3 = 0.f, gb3 = 0.f, loss = 0.f;
+    for (int b = b0; b < b1; b += kTrainSamples)
     {
-        if (j < s) red[j] += red[j + s];
+        // samples past the chunk's end count as zero in every sum
+        const int n = b1 - b;
+#pragma unroll
+        for (int i = 0; i < kFirst; ++i)
+        {
+            const int s = s1 + i * (kTrainThreads / H);
+            h1[s][j1] = s < n ? silu(v1x * xin[i][0] + v1y * xin[i][1] + c1) : 0.f;
+            if (j1 < 2) xs[s][j1] = j1 ? xin[i][1] : xin[i][0];
+        }
+        const float tnow = tin;
+        load_samples(b + kTrainSamples);
+        __syncthreads();
+        f32x4 z[kTrainTiles], sz[kTrainTiles], dz[kTrainTiles];
+#pragma unroll
+        for (int m = 0; m < kTrainTiles; ++m) z[m] = f32x4{bias2, bias2, bias2, bias2};
+#pragma unroll
+        for (int k = 0; k < H / 16; ++k)
+#pragma unroll
+            for (int m = 0; m < kTrainTiles; ++m)
+            {
+                const f32x4 a = *(const f32x4*) &h1[16 * m + col][16 * k + 4 * g];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) z[m] = mfma(a[t], wrow[k][t], z[m]);
+            }
+#pragma unroll
+        for (int m = 0; m < kTrainTiles; ++m)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+            {
+                const float s = sigm(z[m][i]);
+                sz[m][i] = z[m][i] * s;
+                dz[m][i] = s + z[m][i] * s * (1.0f - s);
+                const float y = lanes_sum<16>(w3 * sz[m][i]);
+                if (col == 0) ys[w][16 * m + 4 * g + i] = y;
+            }
+        __syncthreads();
+        if (threadIdx.x < kTrainSamples)
+        {
+            const int s = threadIdx.x;
+            float y = 0.f;
+#pragma unroll
+            for (int q = 0; q < kTrainWaves; ++q) y += ys[q][s];
+            const float e = s < n ? y + bias3 - tnow : 0.f;
+            loss += e * e;
+            const float d = 2.0f * e / (float) B;
+            gb3 += d;
+            d3[s] = d;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < kTrainTiles; ++m)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+            {
+                const int s = 16 * m + 4 * g + i;
+                const float d = d3[s];
+                const float v = s < n ? d * w3 * dz[m][i] : 0.f;
+                d2[s][unit] = v;
+                gb2 += v;
+                gw3 += s < n ? d * sz[m][i] : 0.f;
+            }
+        __syncthreads();
+        f32x4 d1[kTrainTiles] = {};
+#pragma unroll
+        for (int k = 0; k < H / 16; ++k)
+#pragma unroll
+            for (int m = 0; m < kTrainTiles; ++m)
+            {
+                const f32x4 a = *(const f32x4*) &d2[16 * m + col][16 * k + 4 * g];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) d1[m] = mfma(a[t], wcol[k][t], d1[m]);
+            }
+#pragma unroll
+        for (int m = 0; m < kTrainTiles; ++m)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+            {
+                const int s = 16 * m + 4 * g + i;
+                const float x0 = xs[s][0], x1 = xs[s][1];
+                const float v =
+                    s < n ? d1[m][i] * dsilu(w1x * x0 + w1y * x1 + bias1) : 0.f;
+                gb1 += v;
+                gw1x += v * x0;
+                gw1y += v * x1;
+            }
+#pragma unroll
+        for (int m = 0; m < kTrainTiles; ++m)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+            {
+                const int s = 16 * m + 4 * g + t;
+                const float a = d2[s][unit];
+#pragma unroll
+                for (int k = 0; k < H / 16; ++k) gw2[k] = mfma(a, h1[s][16 * k + col], gw2[k]);
+            }
         __syncthreads();
     }
-    if (j == 0) y[b] = red[0] + P[kB3];
+
+    float* out = partial + (size_t) blockIdx.x * kMlpParams;
+#pragma unroll
+    for (int k = 0; k < H / 16; ++k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            out[kW2 + (16 * w + 4 * g + i) * H + 16 * k + col] = gw2[k][i];
+    // the sums over samples of one unit are spread over the four lane groups
+    float* sums[5] = {&gw1x, &gw1y, &gb1, &gb2, &gw3};
+#pragma unroll
+    for (int q = 0; q < 5; ++q)
+    {
+        *sums[q] += __shfl_xor(*sums[q], 16);
+        *sums[q] += __shfl_xor(*sums[q], 32);
+    }
+    if (g == 0)
+    {
+        out[kW1 + 2 * unit] = gw1x;
+        out[kW1 + 2 * unit + 1] = gw1y;
+        out[kB1 + unit] = gb1;
+        out[kB2 + unit] = gb2;
+        out[kW3 + unit] = gw3;
+    }
+    if (w == 0)
+    {
+        gb3 = lanes_sum<64>(gb3);
+        loss = lanes_sum<64>(loss);
+        if (lane == 0)
+        {
+            out[kB3] = gb3;
+            loss_partial[blockIdx.x] = loss;
+        }
+    }
 }
 
-// Per-sample back-propagation: d3 = dL/dy, d2 = dL/dz2, d1 = dL/dz1.
-__global__ __launch_bounds__(H) void mlp_backward_kernel(
-    const float* __restrict__ P, const float* __restrict__ target, int B,
-    const float* __restrict__ z1, const float* __restrict__ z2,
-    const float* __restrict__ y, float* __restrict__ d1, float* __restrict__ d2,
-    float* __restrict__ d3)
+constexpr int kGraphSteps = 16;
+constexpr int kUpdateParams = 64;            // parameters per workgroup
+constexpr int kUpdateParts = 4;              // wavefronts that share the chunks
+
+// Sum of the chunks' gradients and, with ADAM, the step of Adam (Kingma & Ba
+// 2015, bias correction) and the step's loss; the step counter lives in
+// device memory so that a captured step can be replayed. Without ADAM the
+// gradient goes to grad and the loss to losses[0]. A wavefront adds its part
+// of the chunks for 64 parameters, eight loads in flight; the parts are added
+// in order. 5.3 us at 125 chunks (8.5 MB); the sum, Adam and the counter were
+// three launches of 7.9, 4.8 and 4.2 us.
+template <bool ADAM>
+__global__ __launch_bounds__(kUpdateParams* kUpdateParts) void mlp_update_kernel(
+    const float* __restrict__ partial, const float* __restrict__ loss_partial, int groups,
+    int B, float* __restrict__ grad, float* __restrict__ P, float* __restrict__ m1,
+    float* __restrict__ m2, const int* __restrict__ step, float lr, float beta1,
+    float beta2, float eps, float* __restrict__ losses, int max_steps)
 {
-    __shared__ float s2[H];
-    const int b = blockIdx.x;
-    const int j = threadIdx.x;
-    if (b >= B) return;
-    const float g3 = 2.0f * (y[b] - target[b]) / (float) B;
-    if (j == 0) d3[b] = g3;
-    const float g2 = g3 * P[kW3 + j] * dsilu(z2[(size_t) b * H + j]);
-    d2[(size_t) b * H + j] = g2;
-    s2[j] = g2;
+    __shared__ float part[kUpdateParts][kUpdateParams];
+    const int lane = threadIdx.x % kUpdateParams;
+    const int w = threadIdx.x / kUpdateParams;
+    const int p = blockIdx.x * kUpdateParams + lane;
+    const int q = p < kMlpParams ? p : kMlpParams - 1;
+    const int per = (groups + kUpdateParts - 1) / kUpdateParts;
+    const int c1 = (w + 1) * per < groups ? (w + 1) * per : groups;
+    float s = 0.0f;
+#pragma unroll 8
+    for (int c = w * per; c < c1; ++c) s += partial[(size_t) c * kMlpParams + q];
+    part[w][lane] = s;
     __syncthreads();
-    // d1_k = dsilu(z1_k) sum_j W2[j][k] d2_j (thread k reads column k)
-    float acc = 0.0f;
-    for (int jj = 0; jj < H; ++jj) acc += P[kW2 + (size_t) jj * H + j] * s2[jj];
-    d1[(size_t) b * H + j] = acc * dsilu(z1[(size_t) b * H + j]);
-}
-
-// Gradient of every parameter: one thread per (parameter, batch chunk),
-// each summing its chunk of samples in order into partial[chunk][p]; the
-// chunks are then added in order by mlp_reduce_kernel (deterministic, and
-// the batch loop is split over blockIdx.y so that a small network still
-// fills the GPU). The last parameter's thread of each chunk also writes the
-// chunk's sum of squared errors.
-__global__ __launch_bounds__(256) void mlp_grad_kernel(
-    const float* __restrict__ x, const float* __restrict__ target, int B, int chunk,
-    const float* __restrict__ z1, const float* __restrict__ z2,
-    const float* __restrict__ y, const float* __restrict__ d1,
-    const float* __restrict__ d2, const float* __restrict__ d3,
-    float* __restrict__ partial, float* __restrict__ loss_partial)
-{
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (w != 0) return;
+    float g = part[0][lane];
+    for (int i = 1; i < kUpdateParts; ++i) g += part[i][lane];
+    if (blockIdx.x == 0)
+    {
+        float l = 0.0f;
+        for (int c = lane; c < groups; c += 64) l += loss_partial[c];
+        l = lanes_sum<64>(l) / (float) B;
+        const int at = ADAM ? *step - 1 : 0;
+        if (lane == 0 && losses && at < max_steps) losses[at] = l;
+    }
     if (p >= kMlpParams) return;
-    const int c = blockIdx.y;
-    const int b0 = c * chunk;
-    const int b1 = b0 + chunk < B ? b0 + chunk : B;
-    float g = 0.0f;
-    if (p < kB1)
+    if constexpr (ADAM)
     {
-        const int j = p / 2, i = p % 2;
-        for (int b = b0; b < b1; ++b) g += d1[(size_t) b * H + j] * x[2 * b + i];
-    }
-    else if (p < kW2)
-    {
-        const int j = p - kB1;
-        for (int b = b0; b < b1; ++b) g += d1[(size_t) b * H + j];
-    }
-    else if (p < kB2)
-    {
-        const int j = (p - kW2) / H, k = (p - kW2) % H;
-        for (int b = b0; b < b1; ++b)
-            g += d2[(size_t) b * H + j] * silu(z1[(size_t) b * H + k]);
-    }
-    else if (p < kW3)
-    {
-        const int j = p - kB2;
-        for (int b = b0; b < b1; ++b) g += d2[(size_t) b * H + j];
-    }
-    else if (p < kB3)
-    {
-        const int j = p - kW3;
-        for (int b = b0; b < b1; ++b) g += d3[b] * silu(z2[(size_t) b * H + j]);
+        const float t = (float) *step;
+        const float a = beta1 * m1[p] + (1.0f - beta1) * g;
+        const float v = beta2 * m2[p] + (1.0f - beta2) * g * g;
+        m1[p] = a;
+        m2[p] = v;
+        const float ah = a / (1.0f - powf(beta1, t));
+        const float vh = v / (1.0f - powf(beta2, t));
+        P[p] -= lr * ah / (sqrtf(vh) + eps);
     }
     else
-    {
-        for (int b = b0; b < b1; ++b) g += d3[b];
-        float l = 0.0f;
-        for (int b = b0; b < b1; ++b)
-        {
-            const float e = y[b] - target[b];
-            l += e * e;
-        }
-        loss_partial[c] = l;
-    }
-    partial[(size_t) c * kMlpParams + p] = g;
-}
-
-__global__ __launch_bounds__(256) void mlp_reduce_kernel(const float* __restrict__ partial,
-                                                         const float* __restrict__ loss_partial,
-                                                         int chunks, int B,
-                                                         float* __restrict__ grad,
-                                                         float* __restrict__ loss_out)
-{
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= kMlpParams) return;
-    float g = 0.0f;
-    for (int c = 0; c < chunks; ++c) g += partial[(size_t) c * kMlpParams + p];
-    grad[p] = g;
-    if (p == kMlpParams - 1 && loss_out)
-    {
-        float l = 0.0f;
-        for (int c = 0; c < chunks; ++c) l += loss_partial[c];
-        *loss_out = l / (float) B;
-    }
-}
-
-// Batch chunks of the gradient kernel: about 64 samples each, at most 32.
-inline int grad_chunks(int B)
-{
-    const int c = (B + 63) / 64;
-    return c < 32 ? c : 32;
-}
-
-// Adam (Kingma & Ba 2015) with bias correction; the step counter lives in
-// device memory so that a captured step can be replayed.
-__global__ __launch_bounds__(256) void mlp_adam_kernel(
-    float* __restrict__ P, const float* __restrict__ grad, float* __restrict__ m1,
-    float* __restrict__ m2, const int* __restrict__ step, float lr, float beta1,
-    float beta2, float eps)
-{
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= kMlpParams) return;
-    const int t = *step + 1;
-    const float g = grad[p];
-    const float a = beta1 * m1[p] + (1.0f - beta1) * g;
-    const float v = beta2 * m2[p] + (1.0f - beta2) * g * g;
-    m1[p] = a;
-    m2[p] = v;
-    const float ah = a / (1.0f - powf(beta1, (float) t));
-    const float vh = v / (1.0f - powf(beta2, (float) t));
-    P[p] -= lr * ah / (sqrtf(vh) + eps);
-}
-
-// Advances the step counter and records the loss of the step just taken.
-__global__ void mlp_step_kernel(int* step, const float* loss, float* losses, int max_steps)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0)
-    {
-        const int t = *step;
-        if (t < max_steps) losses[t] = *loss;
-        *step = t + 1;
-    }
+        grad[p] = g;
 }
 
 __global__ void zero_i32_kernel(int* p) { *p = 0; }
@@ -229,7 +359,6 @@ __global__ void zero_f32_kernel(float* p, int n)
 // A[l % 16][4 (l / 16) + 0..3] and B[4 (l / 16) + 0..3][l % 16]; the result
 // lane l holds D[4 (l / 16) + 0..3][l % 16].
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ short to_bf16(float f)
 {
@@ -363,38 +492,27 @@ int slq_mlp_grad(const float* params, const float* x, const float* target, int32
         set_error("slq_mlp_grad: invalid argument");
         return SLQ_E_ARG;
     }
-    DevBuf dp, dx, dt, dz1, dz2, dy, dd1, dd2, dd3, dg, dl, dpart, dlpart;
-    const int C = grad_chunks(B);
-    const int chunk = (B + C - 1) / C;
+    DevBuf dp, dx, dt, dg, dl, dpart, dlpart;
+    const int C = train_groups(B);
     SLQ_CHECK(hipMalloc(&dpart.p, sizeof(float) * kMlpParams * C));
     SLQ_CHECK(hipMalloc(&dlpart.p, sizeof(float) * C));
     SLQ_CHECK(hipMalloc(&dp.p, sizeof(float) * kMlpParams));
     SLQ_CHECK(hipMalloc(&dx.p, sizeof(float) * 2 * B));
     SLQ_CHECK(hipMalloc(&dt.p, sizeof(float) * B));
-    SLQ_CHECK(hipMalloc(&dz1.p, sizeof(float) * H * B));
-    SLQ_CHECK(hipMalloc(&dz2.p, sizeof(float) * H * B));
-    SLQ_CHECK(hipMalloc(&dy.p, sizeof(float) * B));
-    SLQ_CHECK(hipMalloc(&dd1.p, sizeof(float) * H * B));
-    SLQ_CHECK(hipMalloc(&dd2.p, sizeof(float) * H * B));
-    SLQ_CHECK(hipMalloc(&dd3.p, sizeof(float) * B));
     SLQ_CHECK(hipMalloc(&dg.p, sizeof(float) * kMlpParams));
     SLQ_CHECK(hipMalloc(&dl.p, sizeof(float)));
     SLQ_CHECK(hipMemcpy(dp.p, params, sizeof(float) * kMlpParams, hipMemcpyHostToDevice));
     SLQ_CHECK(hipMemcpy(dx.p, x, sizeof(float) * 2 * B, hipMemcpyHostToDevice));
     SLQ_CHECK(hipMemcpy(dt.p, target, sizeof(float) * B, hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(mlp_forward_kernel, dim3(B), dim3(H), 0, 0, (const float*) dp.p,
-                       (const float*) dx.p, B, (float*) dz1.p, (float*) dz2.p, (float*) dy.p);
-    hipLaunchKernelGGL(mlp_backward_kernel, dim3(B), dim3(H), 0, 0, (const float*) dp.p,
-                       (const float*) dt.p, B, (const float*) dz1.p, (const float*) dz2.p,
-                       (const float*) dy.p, (float*) dd1.p, (float*) dd2.p, (float*) dd3.p);
-    hipLaunchKernelGGL(mlp_grad_kernel, dim3((kMlpParams + 255) / 256, C), dim3(256), 0, 0,
-                       (const float*) dx.p, (const float*) dt.p, B, chunk,
-                       (const float*) dz1.p, (const float*) dz2.p, (const float*) dy.p,
-                       (const float*) dd1.p, (const float*) dd2.p, (const float*) dd3.p,
-                       (float*) dpart.p, (float*) dlpart.p);
-    hipLaunchKernelGGL(mlp_reduce_kernel, dim3((kMlpParams + 255) / 256), dim3(256), 0, 0,
-                       (const float*) dpart.p, (const float*) dlpart.p, C, B, (float*) dg.p,
-                       (float*) dl.p);
+    hipLaunchKernelGGL(mlp_train_kernel, dim3(C), dim3(kTrainThreads), 0, 0,
+                       (const float*) dp.p, (const float*) dx.p, (const float*) dt.p, B,
+                       train_chunk(B), (float*) dpart.p, (float*) dlpart.p, (int*) nullptr);
+    hipLaunchKernelGGL(mlp_update_kernel<false>,
+                       dim3((kMlpParams + kUpdateParams - 1) / kUpdateParams),
+                       dim3(kUpdateParams * kUpdateParts), 0, 0, (const float*) dpart.p,
+                       (const float*) dlpart.p, C, B, (float*) dg.p, (float*) nullptr,
+                       (float*) nullptr, (float*) nullptr, (const int*) nullptr, 0.f, 0.f,
+                       0.f, 0.f, (float*) dl.p, 1);
     SLQ_CHECK(hipGetLastError());
     SLQ_CHECK(hipDeviceSynchronize());
     SLQ_CHECK(hipMemcpy(grad, dg.p, sizeof(float) * kMlpParams, hipMemcpyDeviceToHost));
@@ -410,23 +528,13 @@ int slq_mlp_train(float* params, const float* x, const float* target, int32_t B,
         set_error("slq_mlp_train: invalid argument");
         return SLQ_E_ARG;
     }
-    DevBuf dp, dx, dt, dz1, dz2, dy, dd1, dd2, dd3, dg, dl, dm1, dm2, dstep, dlosses, dpart,
-        dlpart;
-    const int C = grad_chunks(B);
-    const int chunk = (B + C - 1) / C;
+    DevBuf dp, dx, dt, dm1, dm2, dstep, dlosses, dpart, dlpart;
+    const int C = train_groups(B);
     SLQ_CHECK(hipMalloc(&dpart.p, sizeof(float) * kMlpParams * C));
     SLQ_CHECK(hipMalloc(&dlpart.p, sizeof(float) * C));
     SLQ_CHECK(hipMalloc(&dp.p, sizeof(float) * kMlpParams));
     SLQ_CHECK(hipMalloc(&dx.p, sizeof(float) * 2 * B));
     SLQ_CHECK(hipMalloc(&dt.p, sizeof(float) * B));
-    SLQ_CHECK(hipMalloc(&dz1.p, sizeof(float) * H * B));
-    SLQ_CHECK(hipMalloc(&dz2.p, sizeof(float) * H * B));
-    SLQ_CHECK(hipMalloc(&dy.p, sizeof(float) * B));
-    SLQ_CHECK(hipMalloc(&dd1.p, sizeof(float) * H * B));
-    SLQ_CHECK(hipMalloc(&dd2.p, sizeof(float) * H * B));
-    SLQ_CHECK(hipMalloc(&dd3.p, sizeof(float) * B));
-    SLQ_CHECK(hipMalloc(&dg.p, sizeof(float) * kMlpParams));
-    SLQ_CHECK(hipMalloc(&dl.p, sizeof(float)));
     SLQ_CHECK(hipMalloc(&dm1.p, sizeof(float) * kMlpParams));
     SLQ_CHECK(hipMalloc(&dm2.p, sizeof(float) * kMlpParams));
     SLQ_CHECK(hipMalloc(&dstep.p, sizeof(int)));
@@ -440,37 +548,43 @@ int slq_mlp_train(float* params, const float* x, const float* target, int32_t B,
     hipLaunchKernelGGL(zero_f32_kernel, dim3(pg), dim3(256), 0, s, (float*) dm1.p, kMlpParams);
     hipLaunchKernelGGL(zero_f32_kernel, dim3(pg), dim3(256), 0, s, (float*) dm2.p, kMlpParams);
     hipLaunchKernelGGL(zero_i32_kernel, dim3(1), dim3(1), 0, s, (int*) dstep.p);
-    // one training step, captured once and replayed `steps` times
+    const auto one_step = [&] {
+        hipLaunchKernelGGL(mlp_train_kernel, dim3(C), dim3(kTrainThreads), 0, s,
+                           (const float*) dp.p, (const float*) dx.p, (const float*) dt.p, B,
+                           train_chunk(B), (float*) dpart.p, (float*) dlpart.p,
+                           (int*) dstep.p);
+        hipLaunchKernelGGL(mlp_update_kernel<true>,
+                           dim3((kMlpParams + kUpdateParams - 1) / kUpdateParams),
+                           dim3(kUpdateParams * kUpdateParts), 0, s, (const float*) dpart.p,
+                           (const float*) dlpart.p, C, B, (float*) nullptr, (float*) dp.p,
+                           (float*) dm1.p, (float*) dm2.p, (const int*) dstep.p, lr, 0.9f,
+                           0.999f, 1e-8f, (float*) dlosses.p, steps);
+    };
+    // kGraphSteps training steps, captured once and replayed; the steps
+    // left over are launched one by one (so are all of a few, where the
+    // capture costs more than its launches save)
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     int r = SLQ_OK;
-    hipError_t e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
-    if (e == hipSuccess)
+    int done = 0;
+    hipError_t e = hipSuccess;
+    if (steps >= 2 * kGraphSteps)
     {
-        hipLaunchKernelGGL(mlp_forward_kernel, dim3(B), dim3(H), 0, s, (const float*) dp.p,
-                           (const float*) dx.p, B, (float*) dz1.p, (float*) dz2.p,
-                           (float*) dy.p);
-        hipLaunchKernelGGL(mlp_backward_kernel, dim3(B), dim3(H), 0, s, (const float*) dp.p,
-                           (const float*) dt.p, B, (const float*) dz1.p, (const float*) dz2.p,
-                           (const float*) dy.p, (float*) dd1.p, (float*) dd2.p,
-                           (float*) dd3.p);
-        hipLaunchKernelGGL(mlp_grad_kernel, dim3(pg, C), dim3(256), 0, s, (const float*) dx.p,
-                           (const float*) dt.p, B, chunk, (const float*) dz1.p,
-                           (const float*) dz2.p, (const float*) dy.p, (const float*) dd1.p,
-                           (const float*) dd2.p, (const float*) dd3.p, (float*) dpart.p,
-                           (float*) dlpart.p);
-        hipLaunchKernelGGL(mlp_reduce_kernel, dim3(pg), dim3(256), 0, s,
-                           (const float*) dpart.p, (const float*) dlpart.p, C, B,
-                           (float*) dg.p, (float*) dl.p);
-        hipLaunchKernelGGL(mlp_adam_kernel, dim3(pg), dim3(256), 0, s, (float*) dp.p,
-                           (const float*) dg.p, (float*) dm1.p, (float*) dm2.p,
-                           (const int*) dstep.p, lr, 0.9f, 0.999f, 1e-8f);
-        hipLaunchKernelGGL(mlp_step_kernel, dim3(1), dim3(1), 0, s, (int*) dstep.p,
-                           (const float*) dl.p, (float*) dlosses.p, steps);
-        e = hipStreamEndCapture(s, &graph);
+        e = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
+        if (e == hipSuccess)
+        {
+            for (int i = 0; i < kGraphSteps; ++i) one_step();
+            e = hipStreamEndCapture(s, &graph);
+        }
+        if (e == hipSuccess) e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+        for (; e == hipSuccess && steps - done >= kGraphSteps; done += kGraphSteps)
+            e = hipGraphLaunch(exec, s);
     }
-    if (e == hipSuccess) e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-    for (int i = 0; e == hipSuccess && i < steps; ++i) e = hipGraphLaunch(exec, s);
+    for (; e == hipSuccess && done < steps; ++done)
+    {
+        one_step();
+        e = hipGetLastError();
+    }
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) r = hip_status(e, "slq_mlp_train", __FILE__, __LINE__);
     if (exec) (void) hipGraphExecDestroy(exec);
