@@ -1180,12 +1180,6 @@ void mfma_spmm_split_kernel(
 // matrix cores (78.6 TFLOP/s is 4.9 TB/s of A) as much as HBM.
 constexpr int kDenseKC = 64;
 
-template <typename T>
-__device__ __forceinline__ void load_vals4(const T* __restrict__ p, T (&v)[4])
-{
-    load_row4(p, v);
-}
-
 // Per-probe reduction terms of a workgroup's rows (red[q] of lane (kq, i0)
 // holds probe Lanes<T>::probe(i0, q) over that lane's rows) into its
 // partial row.
@@ -1300,6 +1294,11 @@ __global__ __launch_bounds__(kThreads) void dense_spmm_kernel(SpmmArgs<T> a,
             for (int c = 0; c < 4; ++c) load_row4(arow + c0 * kDenseKC + 16 * c, av[c]);
             xstore(xv, 0);
         }
+        // s_waitcnt vmcnt(0): the first chunk has arrived. Left in flight
+        // into the loop, its waits there also held every later chunk's MFMAs
+        // until the chunk after it had arrived (n = 6001 in FP64: 106 us a
+        // product, 96 without).
+        __builtin_amdgcn_s_waitcnt(0x0f70);
         __syncthreads();
         for (int64_t ci = c0; ci < c1; ++ci)
         {
