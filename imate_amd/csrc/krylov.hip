@@ -817,24 +817,25 @@ __device__ __forceinline__ void spmm_epilogue4(const SpmmArgs<T>& a, int64_t row
 // counter, one group of four slabs ahead, took 28 / 49 / 615 us at n =
 // 20011 / 65536 / 2^20 with 50 non-zeros a row, 118 us at 65536 with 247 and
 // 84 us with that in FP32; without tickets but with the same loop 25 / 41 /
-// 632, 109 and 76; this kernel 20 / 35 / 603, 100 and 55.)
+// 632, 109 and 76; this kernel 19 / 34 / 598, 99 and 55.)
 //
 // What bounds it below 2^20 rows is the latency of a wavefront's chain of
 // gathers, at 2^20 the rate of the gathers themselves. kSpmmDepth pairs of
 // four-slab groups (a pair's values are one load) are in flight per
 // wavefront, and the columns of the kSpmmDepth pairs after them, each lane
 // loading its own: 2 pairs 36 and 604 us at 65536 and 2^20 rows, 4 pairs
-// (150 VGPRs, three wavefronts per SIMD) 38 and 712. The per-probe
+// (150 VGPRs, three wavefronts per SIMD) 38 and 712, 3 pairs 35 and 603. The per-probe
 // reduction term of a tile adds the four rows held by a lane, then the four
 // row groups (lanes l, l ^ 16, l ^ 32, l ^ 48), then the workgroup's tiles,
 // in a fixed order; its partial row goes to tile_partial. With a grid capped
 // by the launch settings (CAPPED) a workgroup takes further tiles in steps of
 // the grid; that loop costs the uncapped form's fourth wavefront per SIMD (148
-// against 126 VGPRs), so it has a form of its own.
+// against 127 VGPRs), so it has a form of its own.
 constexpr int kSpmmDepth = 3;
 
 template <typename T, bool NT, bool CAPPED>
-__global__ __launch_bounds__(kThreads) void mfma_spmm_kernel(
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(CAPPED ? 3 : 4))) void mfma_spmm_kernel(
     SpmmArgs<T> a, const T* __restrict__ X, T* __restrict__ Y, T* __restrict__ Vout,
     const T* __restrict__ Sub, int64_t ntiles, const int64_t* __restrict__ tptr,
     const int32_t* __restrict__ tcols, const T* __restrict__ tvals)
@@ -882,43 +883,54 @@ __global__ __launch_bounds__(kThreads) void mfma_spmm_kernel(
                 c0[u] = cp[8 * P];
                 c1[u] = cp[8 * P + 4];
             }
-#pragma unroll
-            for (int u = 0; u < D; ++u)
-            {
-                const int P = u < np ? u : np - 1;
-                av[u] = ap[(int64_t) P * kWave];
+            // pair P into slot u, and the columns of pair P + D
+            const auto fetch = [&](int u, int P) {
+                av[u] = ap[(int64_t) (P < np ? P : np - 1) * kWave];
                 Lanes<T>::load(X + (int64_t) c0[u] * kBlock, i0, b0[u]);
                 Lanes<T>::load(X + (int64_t) c1[u] * kBlock, i0, b1[u]);
-            }
+                const int Q = P + D < np ? P + D : np - 1;
+                c0[u] = cp[8 * Q];
+                c1[u] = cp[8 * Q + 4];
+            };
+            const auto multiply = [&](int u) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    acc[q] = Mfma16<T>::op(av[u].x, sq[q] * b0[u][q], acc[q]);
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    acc[q] = Mfma16<T>::op(av[u].y, sq[q] * b1[u][q], acc[q]);
+            };
 #pragma unroll
             for (int u = 0; u < D; ++u)
             {
-                const int P = u + D < np ? u + D : np - 1;
-                c0[u] = cp[8 * P];
-                c1[u] = cp[8 * P + 4];
+                fetch(u, u);
+                // keeps the slots' loads in order
+                __builtin_amdgcn_sched_barrier(0);
             }
-            for (int P0 = 0; P0 < np; P0 += D)
+            // No load in the first loop is conditional: the loads in flight
+            // are then known at every wait, which waits for its own slot
+            // only (the second loop's first wait is for all of them). With
+            // one conditional loop 603 / 34.8 us at n = 2^20 / 65536, so 598
+            // / 34.2. The second takes the last D to 2 D - 1 pairs.
+            int P0 = 0;
+            for (; P0 + 2 * D <= np; P0 += D)
             {
 #pragma unroll
                 for (int u = 0; u < D; ++u)
                 {
-                    const int P = P0 + u;
-                    if (P >= np) break;
+                    multiply(u);
+                    fetch(u, P0 + u + D);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            for (; P0 < np; P0 += D)
+            {
 #pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        acc[q] = Mfma16<T>::op(av[u].x, sq[q] * b0[u][q], acc[q]);
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        acc[q] = Mfma16<T>::op(av[u].y, sq[q] * b1[u][q], acc[q]);
-                    if (P + D < np)
-                    {
-                        av[u] = ap[(int64_t) (P + D) * kWave];
-                        Lanes<T>::load(X + (int64_t) c0[u] * kBlock, i0, b0[u]);
-                        Lanes<T>::load(X + (int64_t) c1[u] * kBlock, i0, b1[u]);
-                        const int Q = P + 2 * D < np ? P + 2 * D : np - 1;
-                        c0[u] = cp[8 * Q];
-                        c1[u] = cp[8 * Q + 4];
-                    }
+                for (int u = 0; u < D; ++u)
+                {
+                    if (P0 + u >= np) break;
+                    multiply(u);
+                    if (P0 + u + D < np) fetch(u, P0 + u + D);
                 }
             }
         }
