@@ -260,7 +260,8 @@ int slq_autotune(slq_op* op, int32_t precision, int32_t* spmm_grid,
  * matrix-core SpMM (1, 2 or 4) and the SpMM's operand form (tile_mode 0:
  * the row tiles where they were built, 1: the CSR rows); 0 keeps the
  * library default (environment SLQ_GRID / SLQ_STREAM_GRID / SLQ_SPMM_SPLIT,
- * else the built-in). Every setting gives results within rounding of every
+ * else the built-in). With any of them set, small matrices too run their
+ * recurrence in a launch per kernel instead of one in all. Every setting gives results within rounding of every
  * other; for a fixed setting they are reproducible bit for bit (the
  * reduction order follows the grid, the split and the form). No reference
  * counterpart (imate has no tunable kernels). */
