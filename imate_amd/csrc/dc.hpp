@@ -36,6 +36,12 @@ namespace slq {
 constexpr int kDcDoubles = 11;
 constexpr int kDcInts = 1;
 
+// Couplings below this fraction of the norm count as zero: an eigenvalue moves
+// by no more than the coupling, and the squares of what is left (of a rotation's
+// coupling, of the reciprocal gaps of a merge) stay in range. Kept, one of
+// 1e-163 between equal diagonal entries gave a rotation of e / 0.
+constexpr double kDcLeast = 0x1p-400;
+
 struct DcWork {
     double *d, *e, *f;                 // diagonal -> eigenvalues, couplings, first row
     double *l, *ds, *zs, *fs, *ls;     // last row; a pair's rows in order
@@ -233,7 +239,11 @@ SLQ_DC bool dc_first_row(const G& g, const DcWork& w, int K)
     for (int i = g.tid; i < K; i += g.nt)
     {
         w.ds[i] = ldexp(w.d[i], -ex);
-        if (i + 1 < K) w.e[i] = ldexp(w.e[i], -ex);
+        if (i + 1 < K)
+        {
+            const double ei = ldexp(w.e[i], -ex);
+            w.e[i] = fabs(ei) < kDcLeast ? 0.0 : ei;
+        }
     }
     g.sync();
     // 2 x 2 blocks by one Jacobi rotation, torn from their neighbours

@@ -109,3 +109,16 @@ def test_scaled_zero_and_non_finite():
     assert abs(samples[1, 0] - 1e150) < 1e136
     assert samples[2, 0] == 0.0
     assert numpy.isnan(samples[3, 0]) and numpy.isnan(samples[4, 0])
+
+
+@pytest.mark.parametrize('coupling', [1e-161, 1e-163, 1e-300])
+def test_couplings_whose_squares_underflow(coupling):
+    # equal diagonals, as a Lanczos run on a multiple of the identity gives
+    for m in (2, 3, 20):
+        alpha = numpy.full((1, m), 2.0)
+        beta = numpy.full((1, m), coupling)
+        samples, theta, tau = _run(alpha, beta, [0])
+        assert numpy.all(theta == 2.0)
+        tol = 8 * EPS * (8 + numpy.sqrt(m))
+        assert abs(numpy.sum(tau**2) - 1.0) <= tol
+        assert abs(samples[0, 0] - 2.0) <= 2.0 * tol

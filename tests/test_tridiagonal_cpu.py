@@ -1,0 +1,80 @@
+"""The device's tridiagonal eigensolver (imate_amd/csrc/dc.hpp) built for the
+host, one thread, against numpy's dense eigensolver."""
+
+import ctypes
+import os
+import subprocess
+
+import numpy
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+EPS = numpy.finfo(float).eps
+
+
+@pytest.fixture(scope='module')
+def solve(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp('host') / 'tridiagonal.so')
+    subprocess.check_call([
+        'g++', '-O2', '-std=c++17', '-fPIC', '-shared',
+        '-I' + os.path.join(ROOT, 'imate_amd', 'csrc'),
+        '-I' + os.path.join(ROOT, 'include'), '-o', out,
+        os.path.join(HERE, 'tridiagonal_host.cpp')])
+    lib = ctypes.CDLL(out)
+
+    def run(d, e):
+        K = len(d)
+        d = numpy.ascontiguousarray(d, dtype=float)
+        e = numpy.ascontiguousarray(e, dtype=float)
+        theta, first = numpy.zeros(K), numpy.zeros(K)
+        args = [x.ctypes.data_as(ctypes.c_void_p) for x in (d, e)]
+        outs = [x.ctypes.data_as(ctypes.c_void_p) for x in (theta, first)]
+        return bool(lib.divide_and_conquer(*args, K, *outs)), theta, first
+    return run
+
+
+def _check(solve, d, e):
+    """Eigenvalues and weighted moments to a few eps of the norm (weights of
+    close nodes are shared arbitrarily)."""
+    K = len(d)
+    scale = max(numpy.max(numpy.abs(d)), numpy.max(numpy.abs(e[:K - 1]),
+                                                   initial=0.0))
+    a, b = d / scale, e[:K - 1] / scale
+    w, U = numpy.linalg.eigh(numpy.diag(a) + numpy.diag(b, 1) +
+                             numpy.diag(b, -1))
+    ok, theta, first = solve(d, e)
+    assert ok
+    t = theta / scale
+    tol = 8 * EPS * (8 + numpy.sqrt(K))
+    assert numpy.max(numpy.abs(numpy.sort(t) - w)) <= tol
+    for p in range(4):
+        got, want = numpy.sum(first**2 * t**p), numpy.sum(U[0]**2 * w**p)
+        assert abs(got - want) <= tol * 3.0**p
+
+
+@pytest.mark.parametrize('coupling', [
+    1e-100, 1e-150, 1e-161, 1e-163, 1e-200, 1e-300, 5e-324])
+def test_negligible_couplings(solve, coupling):
+    # equal diagonals: the rotation of a 2 x 2 block is coupling / |coupling|
+    for d in ([1.0, 1.0], [1e-3, 1e-3], [1.0] * 5,
+              [0.0, 0.0, 0.0, 0.0, 1.0, 2.0]):
+        K = len(d)
+        _check(solve, numpy.array(d), numpy.full(K, coupling))
+        # merges of blocks of mixed sizes
+        e = numpy.where(numpy.arange(K) % 2, 0.5, coupling)
+        _check(solve, numpy.array(d), e)
+        _check(solve, numpy.array(d), e[::-1].copy())
+
+
+@pytest.mark.parametrize('lowest', [-5, -100, -160, -200, -320])
+def test_random_magnitudes(solve, lowest):
+    rng = numpy.random.default_rng(-lowest)
+    for _ in range(300):
+        K = int(rng.integers(2, 34))
+        d, e = (10.0**rng.uniform(lowest, 0, K) * rng.choice([-1, 1], K)
+                for _ in range(2))
+        d[rng.random(K) < 0.3] = 0.0
+        d[0] = 1.0
+        e[rng.random(K) < 0.3] = 0.0
+        _check(solve, d, e)
