@@ -227,13 +227,25 @@ template <int P, typename G>
 SLQ_DC bool dc_first_row(const G& g, const DcWork& w, int K)
 {
     // scale by a power of two (exact) so that squares neither overflow nor
-    // underflow; a sum of the moduli is not finite if an entry is not
-    double sum = 0.0;
+    // underflow; a sum of the moduli is not finite if an entry is not. The
+    // terms are scaled down so that finite entries (at most 2 K) do not
+    // overflow it, and up again where that would lose them
+    auto moduli = [&](double by) {
+        double sum = 0.0;
 #pragma unroll 4
-    for (int i = 0; i < K; ++i) sum += fabs(w.d[i]) + (i + 1 < K ? fabs(w.e[i]) : 0.0);
+        for (int i = 0; i < K; ++i)
+            sum += by * fabs(w.d[i]) + (i + 1 < K ? by * fabs(w.e[i]) : 0.0);
+        return sum;
+    };
+    double sum = moduli(0x1p-12);
     if (!(sum <= DBL_MAX)) return false;
-    int ex = 0;
-    if (sum > 0.0) ex = ilogb(sum);
+    int ex = 12;
+    if (sum < 0x1p-900)
+    {
+        sum = moduli(0x1p100);
+        ex = -100;
+    }
+    ex = sum > 0.0 ? ex + ilogb(sum) : 0;
     const int sub = g.tid % P, row0 = g.tid / P, rows = g.nt / P;
     g.sync();
     for (int i = g.tid; i < K; i += g.nt)

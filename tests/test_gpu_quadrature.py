@@ -122,3 +122,14 @@ def test_couplings_whose_squares_underflow(coupling):
         tol = 8 * EPS * (8 + numpy.sqrt(m))
         assert abs(numpy.sum(tau**2) - 1.0) <= tol
         assert abs(samples[0, 0] - 2.0) <= 2.0 * tol
+
+
+def test_finite_entries_whose_sum_overflows():
+    m = 20
+    alpha = numpy.full((1, m), 1.5e308)
+    beta = numpy.full((1, m), 1e307)
+    w, z = _dense(numpy.full(m, 1.5), numpy.full(m, 0.1), 0)
+    _, theta, tau = _run(alpha, beta, [0])
+    tol = 8 * EPS * (8 + numpy.sqrt(m))
+    assert numpy.max(numpy.abs(numpy.sort(theta[0]) / 1e308 - w)) <= 2 * tol
+    assert abs(numpy.sum(tau**2) - 1.0) <= tol

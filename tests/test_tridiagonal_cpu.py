@@ -78,3 +78,21 @@ def test_random_magnitudes(solve, lowest):
         d[0] = 1.0
         e[rng.random(K) < 0.3] = 0.0
         _check(solve, d, e)
+
+
+def test_largest_and_smallest_magnitudes(solve):
+    # finite entries whose moduli sum to more than the largest double, and
+    # entries near the smallest
+    for K in (2, 3, 5, 20, 33):
+        for scale in (8e307, 1e-280):
+            _check(solve, numpy.full(K, scale), numpy.full(K, 0.5 * scale))
+            d = numpy.full(K, 1.5 * scale)
+            d[::2] = -scale
+            _check(solve, d, numpy.full(K, 0.1 * scale))
+    for bad in (numpy.nan, numpy.inf, -numpy.inf):
+        for at in (0, 2, 4):
+            d = numpy.ones(5)
+            d[at] = bad
+            assert not solve(d, numpy.ones(5))[0]
+            if at < 4:
+                assert not solve(numpy.ones(5), d)[0]
