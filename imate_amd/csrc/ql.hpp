@@ -67,6 +67,15 @@ SLQ_HD inline double ffunc(int func, const double* fp, double x)
     }
 }
 
+// A node's term tau^2 f(theta^p) of the quadrature. A node of zero weight adds
+// nothing, whatever f is there: it belongs to a part of the matrix that the
+// first row does not reach (past a negligible coupling), where f of a
+// singular or indefinite remainder may be infinite or NaN.
+SLQ_HD inline double node_term(const QuadArgs& a, double theta, double tau)
+{
+    return tau == 0.0 ? 0.0 : tau * tau * ffunc(a.func, a.fp, fpow(theta, a.exponent));
+}
+
 // Implicit QL on (d, e) of size K (e[i] couples i and i+1, e[K-1] = 0),
 // tracking z = first row of the eigenvector matrix. Arrays are strided by S.
 SLQ_HD inline int ql_first_row(double* __restrict__ d, double* __restrict__ e,
@@ -215,8 +224,7 @@ SLQ_HD inline void quadrature_one(const QuadArgs& a, const double* alpha,
         {
             double th = d[i * S];
             if (a.shift) th = (th - t0) + tj;
-            const double tau = z[i * S];
-            sum += tau * tau * ffunc(a.func, a.fp, fpow(th, a.exponent));
+            sum += node_term(a, th, z[i * S]);
         }
         const int col = a.shift ? j : a.j_out;
         out[col] = info == 0 ? a.n * sum : NAN;

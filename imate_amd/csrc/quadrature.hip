@@ -124,10 +124,7 @@ __global__ __launch_bounds__(NT) void quadrature_dc_kernel(QuadArgs a)
     const double t0 = a.shift ? a.params[0] : 0.0;
     double* out = a.samples + (size_t) p * a.q_stride;
     auto term = [&](int i, double tj) {
-        const double x = a.shift ? (th[i] - t0) + tj : th[i];
-        // a node of zero weight adds nothing, whatever f is there
-        const double t = tau[i];
-        return t == 0.0 ? 0.0 : t * t * ffunc(a.func, a.fp, fpow(x, a.exponent));
+        return node_term(a, a.shift ? (th[i] - t0) + tj : th[i], tau[i]);
     };
     if (jn > kFewInquiries)
     {

@@ -133,3 +133,14 @@ def test_finite_entries_whose_sum_overflows():
     tol = 8 * EPS * (8 + numpy.sqrt(m))
     assert numpy.max(numpy.abs(numpy.sort(theta[0]) / 1e308 - w)) <= 2 * tol
     assert abs(numpy.sum(tau**2) - 1.0) <= tol
+
+
+@pytest.mark.parametrize('gram,m', [(0, 3), (0, 1025), (1, 3), (1, 513)])
+def test_nodes_of_zero_weight(gram, m):
+    # past the first entry a singular part out of the probe's reach, in both
+    # solvers
+    alpha = numpy.full((1, m), 2.0)
+    alpha[0, 1::2] = 0.0
+    beta = numpy.zeros((1, m))
+    samples, _, _ = _run(alpha, beta, [0], gram, _lib.FUNC_LOG)
+    assert abs(samples[0, 0] - numpy.log(4.0 if gram else 2.0)) <= 4 * EPS

@@ -1,5 +1,6 @@
 """The device's tridiagonal eigensolver (imate_amd/csrc/dc.hpp) built for the
-host, one thread, against numpy's dense eigensolver."""
+host, one thread, against numpy's dense eigensolver; the host path's
+quadrature (imate_amd/csrc/ql.hpp) of nodes of zero weight."""
 
 import ctypes
 import os
@@ -8,21 +9,26 @@ import subprocess
 import numpy
 import pytest
 
+from imate_amd import _lib
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 EPS = numpy.finfo(float).eps
 
 
 @pytest.fixture(scope='module')
-def solve(tmp_path_factory):
+def host(tmp_path_factory):
     out = str(tmp_path_factory.mktemp('host') / 'tridiagonal.so')
     subprocess.check_call([
         'g++', '-O2', '-std=c++17', '-fPIC', '-shared',
         '-I' + os.path.join(ROOT, 'imate_amd', 'csrc'),
         '-I' + os.path.join(ROOT, 'include'), '-o', out,
         os.path.join(HERE, 'tridiagonal_host.cpp')])
-    lib = ctypes.CDLL(out)
+    return ctypes.CDLL(out)
 
+
+@pytest.fixture
+def solve(host):
     def run(d, e):
         K = len(d)
         d = numpy.ascontiguousarray(d, dtype=float)
@@ -30,7 +36,7 @@ def solve(tmp_path_factory):
         theta, first = numpy.zeros(K), numpy.zeros(K)
         args = [x.ctypes.data_as(ctypes.c_void_p) for x in (d, e)]
         outs = [x.ctypes.data_as(ctypes.c_void_p) for x in (theta, first)]
-        return bool(lib.divide_and_conquer(*args, K, *outs)), theta, first
+        return bool(host.divide_and_conquer(*args, K, *outs)), theta, first
     return run
 
 
@@ -96,3 +102,15 @@ def test_largest_and_smallest_magnitudes(solve):
             assert not solve(d, numpy.ones(5))[0]
             if at < 4:
                 assert not solve(numpy.ones(5), d)[0]
+
+
+@pytest.mark.parametrize('gram', [0, 1])
+@pytest.mark.parametrize('func,want', [(_lib.FUNC_LOG, numpy.log),
+                                       (_lib.FUNC_INV, lambda x: 1.0 / x)])
+def test_nodes_of_zero_weight(host, gram, func, want):
+    # the second entry is out of the probe's reach and singular
+    alpha, beta = numpy.array([2.0, 0.0, 3.0]), numpy.zeros(3)
+    host.quadrature.restype = ctypes.c_double
+    got = host.quadrature(alpha.ctypes.data_as(ctypes.c_void_p),
+                          beta.ctypes.data_as(ctypes.c_void_p), 3, gram, func)
+    assert abs(got - want(4.0 if gram else 2.0)) <= 4 * EPS

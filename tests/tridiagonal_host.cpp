@@ -1,4 +1,4 @@
-// Host build of the tridiagonal eigensolvers (one thread), for
+// Host build of the tridiagonal eigensolvers and quadrature (one thread), for
 // test_tridiagonal_cpu.py.
 #include <cstdint>
 #include <vector>
@@ -44,4 +44,20 @@ extern "C" int divide_and_conquer(const double* d, const double* e, int K, doubl
         first[i] = w.f[i];
     }
     return 1;
+}
+
+// The host path's quadrature of one tridiagonal (gram: bidiagonal).
+extern "C" double quadrature(const double* alpha, const double* beta, int m, int gram, int func)
+{
+    slq::QuadArgs a = {};
+    double out = 0.0;
+    std::vector<double> work((size_t) 6 * m);
+    a.m = m;
+    a.gram = gram;
+    a.func = func;
+    a.exponent = 1.0;
+    a.n = 1.0;
+    slq::quadrature_one(a, alpha, beta, 1, 0, work.data(), work.data() + 2 * m,
+                        work.data() + 4 * m, 1, &out, nullptr, nullptr);
+    return out;
 }
