@@ -1350,6 +1350,25 @@ struct TuneValue {
 std::mutex g_tune_mu;
 std::map<TuneKey, TuneValue> g_tune_cache;
 
+// Puts a tuning result into the handle and reports its caps; where a launch
+// is left uncapped (0), the grid that it has on this handle.
+void set_tuned(slq_op* op, const TuneValue& v, int32_t* spmm_grid, int32_t* stream_grid)
+{
+    op->tuned = true;
+    op->tuned_spmm_grid = v.spmm_grid;
+    op->tuned_stream_grid = v.stream_grid;
+    op->tuned_spmm_split = v.spmm_split;
+    op->tuned_tile_mode = v.tile_mode;
+    const int64_t rows = op->A->csr.nrows;
+    const bool tiles = op->A->tiles.R == 16 && v.tile_mode <= 1 && v.spmm_split <= 1;
+    if (spmm_grid)
+        *spmm_grid = v.spmm_grid > 0 ? v.spmm_grid
+                     : tiles         ? (int32_t) tile_grid(op->A->tiles.ntiles)
+                                     : grid_for(rows, kMaxGrid);
+    if (stream_grid)
+        *stream_grid = v.stream_grid > 0 ? v.stream_grid : grid_for(rows, kMaxGrid);
+}
+
 }  // namespace
 
 extern "C" int slq_autotune(slq_op* op, int32_t precision, int32_t* spmm_grid,
@@ -1374,67 +1393,58 @@ extern "C" int slq_autotune(slq_op* op, int32_t precision, int32_t* spmm_grid,
         auto it = g_tune_cache.find(key);
         if (it != g_tune_cache.end())
         {
-            op->tuned_spmm_grid = it->second.spmm_grid;
-            op->tuned_stream_grid = it->second.stream_grid;
-            op->tuned_spmm_split = it->second.spmm_split;
-            op->tuned_tile_mode = it->second.tile_mode;
-            if (spmm_grid) *spmm_grid = op->tuned_spmm_grid;
-            if (stream_grid) *stream_grid = op->tuned_stream_grid;
+            set_tuned(op, it->second, spmm_grid, stream_grid);
             return SLQ_OK;
         }
     }
-    // candidate caps (multiples of 8 up to the natural grid of the problem),
-    // timed on the handle's own grid fields, which are restored afterwards
-    const int cands[] = {8, 16, 32, 64, 128, 256, 512, 1024};
+    // candidate caps (no cap, then multiples of 8 up to the natural grid of
+    // the problem), timed on the handle's own grid fields, which are restored
+    // afterwards. The uncapped SpMM is a kernel of its own (mfma_spmm_kernel),
+    // faster than any grid of the looping one; a cap has to beat it by more
+    // than two timings differ. user_launch: the block kernels are what the
+    // settings are about, also where the resident kernel would run
+    const int cands[] = {0, 8, 16, 32, 64, 128, 256, 512, 1024};
+    const double margin = 0.97;
     const int steps = 4;
     const int keep_s = op->spmm_grid, keep_u = op->stream_grid;
+    const bool keep_user = op->user_launch;
     int best_s = 0, best_u = 0;
-    double best_t = 1e300;
     int r = SLQ_OK;
+    op->user_launch = true;
+    auto best_cap = [&](int& field) {
+        int best = 0;
+        double best_t = 1e300;
+        for (int cap : cands)
+        {
+            if (cap > grid_for(c.nrows, kMaxGrid)) break;
+            field = cap;
+            double t = time_block(op, steps, precision);
+            // the first timing may see the clocks of an idle GPU
+            if (cap == 0 && t >= 0) t = std::min(t, time_block(op, steps, precision));
+            if (t < 0)
+            {
+                r = SLQ_E_HIP;
+                break;
+            }
+            if (cap == 0 || t < best_t)
+            {
+                best_t = cap == 0 ? t * margin : t;
+                best = cap;
+            }
+        }
+        field = best;
+        return best;
+    };
     op->stream_grid = 0;
-    for (int cap : cands)
-    {
-        if (cap > grid_for(c.nrows, kMaxGrid)) break;
-        op->spmm_grid = cap;
-        const double t = time_block(op, steps, precision);
-        if (t < 0)
-        {
-            r = SLQ_E_HIP;
-            break;
-        }
-        if (t < best_t)
-        {
-            best_t = t;
-            best_s = cap;
-        }
-    }
-    op->spmm_grid = best_s;
-    best_t = 1e300;
-    for (int cap : cands)
-    {
-        if (r != SLQ_OK || cap > grid_for(c.nrows, kMaxGrid)) break;
-        op->stream_grid = cap;
-        const double t = time_block(op, steps, precision);
-        if (t < 0)
-        {
-            r = SLQ_E_HIP;
-            break;
-        }
-        if (t < best_t)
-        {
-            best_t = t;
-            best_u = cap;
-        }
-    }
+    best_s = best_cap(op->spmm_grid);
+    if (r == SLQ_OK) best_u = best_cap(op->stream_grid);
+    double best_t = 1e300;
     // operand form at the chosen caps: the 16-row tiles with 1, 2 or 4
     // wavefronts per tile, or the CSR rows
     int best_k = 0, best_m = 0;
     const int keep_k = op->spmm_split, keep_m = op->tile_mode;
     if (r == SLQ_OK && op->A->tiles.R > 0)
     {
-        op->spmm_grid = best_s;
-        op->stream_grid = best_u;
-        best_t = 1e300;
         struct Form {
             int mode, split;
         };
@@ -1465,17 +1475,12 @@ extern "C" int slq_autotune(slq_op* op, int32_t precision, int32_t* spmm_grid,
     op->stream_grid = keep_u;
     op->spmm_split = keep_k;
     op->tile_mode = keep_m;
+    op->user_launch = keep_user;
     if (r != SLQ_OK) return r;
-    op->tuned_spmm_grid = best_s;
-    op->tuned_stream_grid = best_u;
-    op->tuned_spmm_split = best_k;
-    op->tuned_tile_mode = best_m;
-    {
-        std::lock_guard<std::mutex> lock(g_tune_mu);
-        g_tune_cache[key] = {best_s, best_u, best_k, best_m};
-    }
-    if (spmm_grid) *spmm_grid = best_s;
-    if (stream_grid) *stream_grid = best_u;
+    const TuneValue v{best_s, best_u, best_k, best_m};
+    set_tuned(op, v, spmm_grid, stream_grid);
+    std::lock_guard<std::mutex> lock(g_tune_mu);
+    g_tune_cache[key] = v;
     return SLQ_OK;
 }
 
@@ -1495,8 +1500,11 @@ struct TunedLaunch {
         {
             slq_op* op = ops[i];
             saved[i] = {op->spmm_grid, op->stream_grid, op->spmm_split, op->tile_mode};
-            if (op->tuned_spmm_grid > 0) op->spmm_grid = op->tuned_spmm_grid;
-            if (op->tuned_stream_grid > 0) op->stream_grid = op->tuned_stream_grid;
+            if (op->tuned)
+            {
+                op->spmm_grid = op->tuned_spmm_grid;
+                op->stream_grid = op->tuned_stream_grid;
+            }
             if (op->tuned_spmm_split > 0) op->spmm_split = op->tuned_spmm_split;
             if (op->tuned_tile_mode > 0) op->tile_mode = op->tuned_tile_mode - 1;
         }

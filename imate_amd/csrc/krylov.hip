@@ -2085,6 +2085,12 @@ int max_grid()
 
 }  // namespace
 
+int64_t tile_grid(int64_t ntiles)
+{
+    const int64_t span = (ntiles + kXcds - 1) / kXcds;
+    return (span + kWavesPerWG - 1) / kWavesPerWG * kXcds;
+}
+
 int grid_for(int64_t units, int cap)
 {
     // reduction buffers hold kMaxGrid partial rows: never exceed it
@@ -2459,8 +2465,7 @@ void launch_spmm_nt(slq_op* op, const SpmmArgs<T>& s, const SpmmIO<T>& io, const
             else if (tl->R == 16)
             {
                 // a workgroup per eight tiles unless the launch settings cap it
-                const int64_t span = (tl->ntiles + kXcds - 1) / kXcds;
-                int64_t g = (span + kWavesPerWG - 1) / kWavesPerWG * kXcds;
+                int64_t g = tile_grid(tl->ntiles);
                 prows = g;
                 const int cap = op->spmm_grid > 0 ? op->spmm_grid : spmm_grid_env();
                 if (cap > 0 && g > cap) g = cap < kXcds ? kXcds : cap / kXcds * kXcds;

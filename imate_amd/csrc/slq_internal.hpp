@@ -239,9 +239,11 @@ struct slq_op {
     // launch-grid caps of the kernels (0 = library default)
     int spmm_grid = 0;
     int stream_grid = 0;
-    // caps chosen by the autotuner (0 = not tuned); slq_estimate_batch runs
-    // with them, every other entry point with the caps above, so a tuned
-    // handle gives slq_estimate the same reduction order as before
+    // caps chosen by the autotuner (0 = no cap), where it has run;
+    // slq_estimate_batch runs with them, every other entry point with the
+    // caps above, so a tuned handle gives slq_estimate the same reduction
+    // order as before
+    bool tuned = false;
     int tuned_spmm_grid = 0;
     int tuned_stream_grid = 0;
     // wavefronts per tile of the matrix-core SpMM (1, 2, 4; 0 = default)
@@ -377,5 +379,7 @@ int copy_bandwidth(int64_t bytes, int iters, double* ms);
 // Grid of a launch over `units` work units with an optional cap (0 = the
 // library default cap).
 int grid_for(int64_t units, int cap = 0);
+// Uncapped grid of the matrix-core SpMM over 16-row tiles.
+int64_t tile_grid(int64_t ntiles);
 
 }  // namespace slq

@@ -242,15 +242,16 @@ int slq_estimate_batch(slq_op** ops, int32_t count, int32_t func,
                        int32_t use_graph, double* trace, double* error,
                        double* samples, double* run_time, double* setup_time);
 
-/* Autotuner: times one 64-probe block of Lanczos steps over candidate launch
- * grids for the SpMM and for the streaming kernels, then over the SpMM's
- * operand form (the 16-row tiles with 1, 2 or 4 wavefronts per tile, or the
- * CSR rows), keeps the fastest in the handle for slq_estimate_batch and
- * caches it per (rows, non-zeros per row, value type, tile rows). Outputs
- * the chosen caps when non-NULL. The other
- * entry points keep the library's default grids on a tuned handle, so their
- * reduction order, and with it every result bit, does not depend on tuning.
- * Square matrix or A + tI handles only (Lanczos is what is timed).
+/* Autotuner: times one 64-probe block of Lanczos steps, in the kernels that
+ * take launch settings, without caps and over candidate launch grids for the
+ * SpMM and for the streaming kernels, then over the SpMM's operand form (the
+ * 16-row tiles with 1, 2 or 4 wavefronts per tile, or the CSR rows), keeps
+ * the fastest in the handle for slq_estimate_batch and caches it per (rows,
+ * non-zeros per row, value type, tile rows). Outputs the chosen caps when
+ * non-NULL, or the whole grid of this handle where no cap is the fastest.
+ * The other entry points keep the library's default grids on a tuned handle,
+ * so their reduction order, and with it every result bit, does not depend on
+ * tuning. Square matrix or A + tI handles only (Lanczos is what is timed).
  * No reference counterpart (imate has no tunable kernels). */
 int slq_autotune(slq_op* op, int32_t precision, int32_t* spmm_grid,
                  int32_t* stream_grid);

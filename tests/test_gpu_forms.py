@@ -127,6 +127,54 @@ def test_batch_autotune_leaves_handles_untouched():
         assert rel.max() < 1e-10
 
 
+def _autotune(M):
+    import ctypes
+    from imate_amd import _lib
+    sg, ug = ctypes.c_int32(0), ctypes.c_int32(0)
+    _lib.check(_lib.load().slq_autotune(
+        M.get_linear_operator(gpu=True).handle, 0, ctypes.byref(sg),
+        ctypes.byref(ug)), 'slq_autotune')
+    return sg.value, ug.value
+
+
+def test_autotune_keeps_the_uncapped_spmm():
+    # past 131072 rows every cap the autotuner tries selects the looping
+    # SpMM; the uncapped one (a workgroup per eight 16-row tiles) is faster
+    n = 1 << 18
+    A = scipy.sparse.diags([4.0] + [-0.1] * 48, list(range(0, 25)) +
+                           list(range(-24, 0)), shape=(n, n), format='csr')
+    M = imate_amd.Matrix(A)
+    want = (n // 16) // 8
+    assert _autotune(M)[0] == want
+    # a matrix of the same cache key gets its own uncapped grid
+    n2 = n + 4096
+    A2 = scipy.sparse.diags([4.0] + [-0.1] * 48, list(range(0, 25)) +
+                            list(range(-24, 0)), shape=(n2, n2), format='csr')
+    M2 = imate_amd.Matrix(A2)
+    assert _autotune(M2)[0] == (n2 // 16) // 8
+
+
+def test_autotune_of_small_matrices_times_the_block_kernels():
+    # matrices that plain estimates run in one resident launch: the caps are
+    # for the block kernels (orthogonalize != 0), for which eight or sixteen
+    # workgroups are the slowest. Ten cache keys (non-zeros per row)
+    Ms = []
+    for k in range(10):
+        n = 1900
+        A = scipy.sparse.diags([4.0] + [-0.01] * (2 * k + 2),
+                               list(range(0, k + 2)) +
+                               list(range(-k - 1, 0)), shape=(n, n),
+                               format='csr')
+        M = imate_amd.Matrix(A)
+        assert _autotune(M)[1] >= 32
+        Ms.append(M)
+    kw = dict(func='log', lanczos_degree=12, num_samples=64, seed=3,
+              orthogonalize=-1, use_graph=False)
+    a, ia = slq_batch(Ms, autotune=True, **kw)
+    b, ib = slq_batch(Ms, autotune=False, **kw)
+    assert numpy.max(numpy.abs(a - b) / numpy.abs(b)) < 1e-11
+
+
 def test_batch_gram_rectangular_matches_oracle():
     rng = numpy.random.default_rng(11)
     mats = []
