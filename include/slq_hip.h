@@ -353,8 +353,9 @@ int slq_recurrences(slq_op* op, double t, int32_t gram, int64_t seed,
  * or of the bidiagonal's squared singular values (gram != 0), then
  * samples[count][q] = n * sum_i tau_i^2 f((theta_i - params[0] + params[j])^p)
  * (shift only when shift != 0; else one inquiry). Outputs theta/tau
- * [count][m] when non-NULL. A node of zero weight adds nothing, whatever f is
- * there (likewise in every estimate, on the device and on the host).
+ * [count][m] when non-NULL. A node whose weight is zero to rounding (tau up
+ * to 64 eps) adds nothing where f is infinite or NaN (likewise in every
+ * estimate, on the device and on the host).
  * Replaces Diagonalization::eigh_tridiagonal / svd_bidiagonal (LAPACK ?stev /
  * ?bdsdc, imate/_c_trace_estimator/diagonalization.cpp:88-118,189-231) and the
  * quadrature of cu_trace_estimator.cu:~555-630. */

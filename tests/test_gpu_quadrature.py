@@ -144,3 +144,13 @@ def test_nodes_of_zero_weight(gram, m):
     beta = numpy.zeros((1, m))
     samples, _, _ = _run(alpha, beta, [0], gram, _lib.FUNC_LOG)
     assert abs(samples[0, 0] - numpy.log(4.0 if gram else 2.0)) <= 4 * EPS
+
+
+def test_weights_at_the_rounding_level():
+    # node -beta^2 with tau = beta: log of it is NaN. A weight of 3e-16
+    # squared is rounding, one of 1e-6 squared is not
+    alpha = numpy.array([[1.0, 0.0], [1.0, 0.0]])
+    beta = numpy.array([[3e-16, 0.0], [1e-6, 0.0]])
+    samples, _, _ = _run(alpha, beta, [0, 0], 0, _lib.FUNC_LOG)
+    assert abs(samples[0, 0]) <= 4 * EPS
+    assert numpy.isnan(samples[1, 0])

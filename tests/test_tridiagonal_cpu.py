@@ -1,6 +1,6 @@
 """The device's tridiagonal eigensolver (imate_amd/csrc/dc.hpp) built for the
 host, one thread, against numpy's dense eigensolver; the host path's
-quadrature (imate_amd/csrc/ql.hpp) of nodes of zero weight."""
+quadrature (imate_amd/csrc/ql.hpp) of nodes without weight."""
 
 import ctypes
 import os
@@ -114,3 +114,17 @@ def test_nodes_of_zero_weight(host, gram, func, want):
     got = host.quadrature(alpha.ctypes.data_as(ctypes.c_void_p),
                           beta.ctypes.data_as(ctypes.c_void_p), 3, gram, func)
     assert abs(got - want(4.0 if gram else 2.0)) <= 4 * EPS
+
+
+def _host_logdet(host, alpha, beta):
+    host.quadrature.restype = ctypes.c_double
+    args = [numpy.ascontiguousarray(x, dtype=float) for x in (alpha, beta)]
+    return host.quadrature(*[x.ctypes.data_as(ctypes.c_void_p) for x in args],
+                           len(alpha), 0, _lib.FUNC_LOG)
+
+
+def test_weights_at_the_rounding_level(host):
+    # the second node is -9e-32 with tau = 3e-16: log of it is NaN
+    assert _host_logdet(host, [1.0, 0.0], [3e-16, 0.0]) == 0.0
+    # a node of real weight keeps its NaN
+    assert numpy.isnan(_host_logdet(host, [1.0, 0.0], [1e-6, 0.0]))
