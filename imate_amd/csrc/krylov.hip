@@ -1639,24 +1639,29 @@ __global__ __launch_bounds__(kTotalWaves * kWave) void norm_total_kernel(
 
 // Classical Gram-Schmidt against the K newest basis vectors of each probe
 // (basis layout [slot][row][64]; vector k of a pass is slot last - k), a
-// second time where the first cancelled: h = V^T r, r -= V h, |r|, and again
-// when |h| is not small against |r| for some probe of the block
-// (gs_norm_kernel). "Twice is enough" (Parlett & Kahan; Daniel, Gragg,
-// Kaufman & Stewart, Math. Comp. 30, 1976): one pass leaves V^T r at the
-// rounding level unless the subtraction cancels most of r, and after the
-// three-term recurrence it does so only near a breakdown. The second pass's
-// kernels are queued either way; its product kernel also decides, and the
-// other returns at once when there is nothing to do. (An empty launch costs
-// 4-5 us, as much as a pass over a few thousand rows: so the second pass is
-// two launches, whose totals the last workgroup to finish adds up.)
+// second time where the first cancels: h = V^T r and |r|^2, r -= V h, and
+// again when |h| is not small against what is left for some probe of the
+// block. "Twice is enough" (Parlett & Kahan; Daniel, Gragg, Kaufman &
+// Stewart, Math. Comp. 30, 1976): one pass leaves V^T r at the rounding level
+// unless the subtraction cancels most of r, and after the three-term
+// recurrence it does so only near a breakdown. The second pass is known
+// before the first subtraction, which then forms the next products in the
+// same pass over the basis (gs_first_kernel). Its totals and its subtraction
+// are queued either way; without a second pass the former finish the norm and
+// the latter returns at once. (An empty launch costs 4-5 us, as much as a
+// pass over a few thousand rows, so there is one.)
 // Every probe has its own basis, so each product is a GEMV per probe (0.5
 // flop per byte): the kernels are HBM streams, written for loads in flight:
 // a wavefront takes one row per iteration and issues the loads of kGsChunk
 // basis vectors at once. Two
 // passes over the basis a step instead of the three of a pass that always
 // runs twice (the middle two fused, as FP32 vectors still take them):
-// n = 65536, m = 60, 128 probes 98.5 -> 67.4 ms; the passes run at 5.1
-// (products) and 4.9 TB/s (subtractions). Sweeping the subtraction's rows
+// n = 65536, m = 60, 128 probes 98.5 -> 64.5 ms; the passes run at 5.1
+// (products) and 4.9 TB/s (subtractions). Where every step cancels
+// (Golub-Kahn on 11 distinct values, n = 2000, m = 60) it takes 6.9 ms, as
+// long as two passes in every step; deciding after the first subtraction,
+// with a pass of its own for the second products, their totals in one
+// workgroup and a fence before the norm's, took 48.5. Sweeping the subtraction's rows
 // backwards, to meet what the product pass left in the Infinity Cache, was
 // 7 % faster in FP32 and 7 % slower in FP64, and is not done.
 constexpr int kGsChunk = 32;     // basis vectors per pass over the rows
@@ -1672,14 +1677,14 @@ struct GsArgs {
     int last;                // slot of the newest vector; vector k is slot last - k
     int K;
     const double* h;         // [K][64] coefficients (gs_sub_kernel)
-    double* partial_k;       // [G][K][64] (gs_dots_kernel)
+    double* partial_k;       // [G][rows][64] (gs_dots_kernel)
+    int rows;                // K, in FP64 with |r|^2 as row K one more
     // gs_dots_kernel with UPD: r = w - alpha v (v the newest vector) first
     const double* alpha;
     // the second pass (gs_again_kernel, gs_sub_kernel<T, true>)
+    bool always;             // it runs whatever the first cancels
     int* again;              // 1 where it runs
     unsigned int* ticket;    // workgroups done, zero between launches
-    double* h_out;           // h, to be replaced by the second pass's
-    int first_rows;          // partial rows of the first pass's |r|^2
     int j;
     double tol_sqrt_n;
     double* norm_out;
@@ -1693,10 +1698,11 @@ struct GsArgs {
 // again as the last (a cache hit), so every load is unconditional and all C
 // are in flight at once; chunks are cut to C = 8, 16 or 32 to keep the
 // repeats few.
-template <typename T, int C, bool UPD>
+// With LEN the sum of r^2 too.
+template <typename T, int C, bool UPD, bool LEN>
 __device__ __forceinline__ void dots_rows(const T* __restrict__ base, T* __restrict__ R,
                                           int64_t stride, int kn, const Sweep& sw, int lane,
-                                          double al, double (&acc)[kGsChunk])
+                                          double al, double (&acc)[kGsChunk], double& len)
 {
     for (int64_t row = sw.first; row < sw.end; row += sw.stride)
     {
@@ -1712,6 +1718,7 @@ __device__ __forceinline__ void dots_rows(const T* __restrict__ base, T* __restr
             R[o] = rt;
         }
         const double r = (double) rt;
+        if constexpr (LEN) len += r * r;
 #pragma unroll
         for (int g = 0; g < C; ++g) acc[g] += r * (double) v[g];
     }
@@ -1741,17 +1748,19 @@ __device__ __forceinline__ double sub_rows(const T* __restrict__ base, T* __rest
 }
 
 // partial_k[g][k] = sum over the rows of workgroup g of basis_k * r, with
-// UPD after the update r = w - alpha v_j.
-template <typename T, bool UPD>
+// UPD after the update r = w - alpha v_j; with LEN row K that of r^2.
+template <typename T, bool UPD, bool LEN>
 __device__ __forceinline__ void gs_dots(const GsArgs& a, T* __restrict__ R,
                                         const T* __restrict__ basis)
 {
     __shared__ double red[kWavesPerWG][8][kWave];
+    __shared__ double rlen[LEN ? kWavesPerWG : 1][kWave];
     const int lane = threadIdx.x % kWave;
     const int wave = wave_id();
     const Sweep sw = sweep_linear(a.nrows, wave);
     const int64_t stride = a.slot;
     const double al = UPD ? a.alpha[lane] : 0.0;
+    double len = 0.0;
     for (int k0 = 0; k0 < a.K; k0 += kGsChunk)
     {
         const int kn = (a.K - k0) < kGsChunk ? (a.K - k0) : kGsChunk;
@@ -1759,17 +1768,20 @@ __device__ __forceinline__ void gs_dots(const GsArgs& a, T* __restrict__ R,
         double acc[kGsChunk];
 #pragma unroll
         for (int g = 0; g < kGsChunk; ++g) acc[g] = 0.0;
-        if (UPD && k0 == 0)
+        if ((UPD || LEN) && k0 == 0)
         {
-            if (kn > 16) dots_rows<T, 32, UPD>(base, R, stride, kn, sw, lane, al, acc);
-            else if (kn > 8) dots_rows<T, 16, UPD>(base, R, stride, kn, sw, lane, al, acc);
-            else dots_rows<T, 8, UPD>(base, R, stride, kn, sw, lane, al, acc);
+            if (kn > 16) dots_rows<T, 32, UPD, LEN>(base, R, stride, kn, sw, lane, al, acc, len);
+            else if (kn > 8)
+                dots_rows<T, 16, UPD, LEN>(base, R, stride, kn, sw, lane, al, acc, len);
+            else dots_rows<T, 8, UPD, LEN>(base, R, stride, kn, sw, lane, al, acc, len);
         }
         else
         {
-            if (kn > 16) dots_rows<T, 32, false>(base, R, stride, kn, sw, lane, al, acc);
-            else if (kn > 8) dots_rows<T, 16, false>(base, R, stride, kn, sw, lane, al, acc);
-            else dots_rows<T, 8, false>(base, R, stride, kn, sw, lane, al, acc);
+            if (kn > 16)
+                dots_rows<T, 32, false, false>(base, R, stride, kn, sw, lane, al, acc, len);
+            else if (kn > 8)
+                dots_rows<T, 16, false, false>(base, R, stride, kn, sw, lane, al, acc, len);
+            else dots_rows<T, 8, false, false>(base, R, stride, kn, sw, lane, al, acc, len);
         }
         // workgroup sums, eight vectors at a time through LDS
 #pragma unroll
@@ -1778,13 +1790,21 @@ __device__ __forceinline__ void gs_dots(const GsArgs& a, T* __restrict__ R,
             if (g0 >= kn) break;
 #pragma unroll
             for (int g = 0; g < 8; ++g) red[wave][g][lane] = acc[g0 + g];
+            if (LEN && k0 + g0 == 0) rlen[wave][lane] = len;
             __syncthreads();
             if (wave < 8 && g0 + wave < kn)
             {
                 double t = 0.0;
 #pragma unroll
                 for (int w = 0; w < kWavesPerWG; ++w) t += red[w][wave][lane];
-                a.partial_k[((int64_t) blockIdx.x * a.K + k0 + g0 + wave) * kWave + lane] = t;
+                a.partial_k[((int64_t) blockIdx.x * a.rows + k0 + g0 + wave) * kWave + lane] = t;
+            }
+            if (LEN && k0 + g0 == 0 && wave == kWavesPerWG - 1)
+            {
+                double t = 0.0;
+#pragma unroll
+                for (int w = 0; w < kWavesPerWG; ++w) t += rlen[w][lane];
+                a.partial_k[((int64_t) blockIdx.x * a.rows + a.K) * kWave + lane] = t;
             }
             __syncthreads();
         }
@@ -1795,46 +1815,15 @@ template <typename T, bool UPD>
 __global__ __launch_bounds__(kThreads) void gs_dots_kernel(GsArgs a, T* __restrict__ R,
                                                            const T* __restrict__ basis)
 {
-    gs_dots<T, UPD>(a, R, basis);
+    gs_dots<T, UPD, sizeof(T) == 8>(a, R, basis);
 }
 
-// True in every thread of the last workgroup of the grid to get here, whose
-// later reads see what the others wrote before (the counter is then zero
-// again).
-__device__ __forceinline__ bool last_workgroup(unsigned int* ticket)
-{
-    __shared__ bool last;
-    __threadfence();
-    __syncthreads();
-    if (threadIdx.x == 0)
-    {
-        last = atomicAdd(ticket, 1u) == gridDim.x - 1;
-        if (last) atomicExch(ticket, 0u);
-    }
-    __syncthreads();
-    __threadfence();
-    return last;
-}
-
-// Sum of rows[g][lane] over g in [0, G) by the workgroup's wavefronts, in a
-// fixed order, the same in every wavefront.
-__device__ __forceinline__ double wg_total(const double* __restrict__ rows, int G, int lane,
-                                           int wave)
+// The sum of x over the workgroup's threads of a lane, in wavefront 0.
+__device__ __forceinline__ double wg_sum(double x, int lane, int wave)
 {
     __shared__ double red[kWavesPerWG][kWave];
-    double s = 0.0;
-    int g = wave;
-    for (; g + 7 * kWavesPerWG < G; g += 8 * kWavesPerWG)
-    {
-        double v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = rows[(int64_t) (g + u * kWavesPerWG) * kWave + lane];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) s += v[u];
-    }
-    for (; g < G; g += kWavesPerWG) s += rows[(int64_t) g * kWave + lane];
     __syncthreads();
-    red[wave][lane] = s;
+    red[wave][lane] = x;
     __syncthreads();
     double t = 0.0;
 #pragma unroll
@@ -1842,56 +1831,59 @@ __device__ __forceinline__ double wg_total(const double* __restrict__ rows, int 
     return t;
 }
 
-// After the first pass: |r|^2 from its partial rows, by every workgroup.
-// Unless |h| > 0.1 |r| for some probe (below that r lost at most 0.5 % of its
-// length; a NaN asks for nothing, it would stay one) the norm is final and
-// *again = 0; else *again = 1 and this is the second pass's product h = V^T r,
-// whose totals the last workgroup stores.
-constexpr double kCancelSquared = 1e-2;
-
-template <typename T>
-__global__ __launch_bounds__(kThreads) void gs_again_kernel(GsArgs a, T* __restrict__ R,
-                                                            const T* __restrict__ basis)
+// Total of x over the grid, in a fixed order: true in every thread of the
+// last workgroup to get here, whose wavefront 0 then has the total (and the
+// counter is zero again). The workgroups hand their rows over by agent-scope
+// stores, which go through the caches, and the counter is advanced when those
+// of the wavefront are done. (A fence in their place writes back the XCD's
+// whole L2 in every workgroup: the second subtraction took 63 us with it at n
+// = 2000 and 60 vectors, 9 us without a total.)
+__device__ __forceinline__ bool grid_total(double x, double* rows, unsigned int* ticket, int lane,
+                                           int wave, double& total)
 {
-    const int lane = threadIdx.x % kWave;
-    const int wave = wave_id();
-    __shared__ double hs[kWavesPerWG][kWave];
-    double hh = 0.0;
-    for (int k = wave; k < a.K; k += kWavesPerWG)
+    __shared__ bool last;
+    const double t = wg_sum(x, lane, wave);
+    if (wave == 0)
     {
-        const double v = a.h[(int64_t) k * kWave + lane];
-        hh += v * v;
+        __hip_atomic_store(rows + (int64_t) blockIdx.x * kWave + lane, t, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): the row is in memory
+        asm volatile("" ::: "memory");
+        if (lane == 0)
+        {
+            last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+            if (last)
+                __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
     }
-    hs[wave][lane] = hh;
-    const double t = wg_total(a.rb.partial, a.first_rows, lane, wave);
-    double sum = 0.0;
-#pragma unroll
-    for (int w = 0; w < kWavesPerWG; ++w) sum += hs[w][lane];
-    const bool more = __any(sum > kCancelSquared * t);
-    if (blockIdx.x == 0 && wave == 0)
-    {
-        if (lane == 0) *a.again = more ? 1 : 0;
-        if (!more) finish_norm(t, lane, a.j, a.tol_sqrt_n, a.norm_out, a.scale_out, a.sizes);
-    }
-    if (!more) return;
-    gs_dots<T, false>(a, R, basis);
-    if (!last_workgroup(a.ticket)) return;
+    __syncthreads();
+    if (!last) return false;
     const int G = gridDim.x;
-    for (int k = wave; k < a.K; k += kWavesPerWG)
+    double s = 0.0;
+    for (int g0 = wave; g0 < G; g0 += 16 * kWavesPerWG)
     {
-        double s = 0.0;
-        for (int g = 0; g < G; ++g) s += a.partial_k[((int64_t) g * a.K + k) * kWave + lane];
-        a.h_out[(int64_t) k * kWave + lane] = s;
+        double v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+        {
+            const int g = g0 + u * kWavesPerWG;
+            v[u] = __hip_atomic_load(rows + (int64_t) (g < G ? g : G - 1) * kWave + lane,
+                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+#pragma unroll
+        for (int u = 0; u < 16; ++u) s += g0 + u * kWavesPerWG < G ? v[u] : 0.0;
     }
+    total = wg_sum(s, lane, wave);
+    return true;
 }
 
-// r -= sum_k h_k basis_k, with the partial rows of |r|^2; in the second pass
-// (SECOND) where that runs, and the last workgroup finishes the norm.
-template <typename T, bool SECOND>
-__global__ __launch_bounds__(kThreads) void gs_sub_kernel(GsArgs a, T* __restrict__ R,
-                                                          const T* __restrict__ basis)
+// r -= sum_k h_k basis_k (in k order); this thread's part of |r|^2.
+template <typename T>
+__device__ __forceinline__ double gs_sub(const GsArgs& a, T* __restrict__ R,
+                                         const T* __restrict__ basis)
 {
-    if (SECOND && *a.again == 0) return;
     __shared__ double hs[kGsChunk][kWave];
     const int lane = threadIdx.x % kWave;
     const int wave = wave_id();
@@ -1920,28 +1912,47 @@ __global__ __launch_bounds__(kThreads) void gs_sub_kernel(GsArgs a, T* __restric
         else if (kn > 8) red = sub_rows<T, 16>(base, R, stride, kn, sw, lane, hs, norm);
         else red = sub_rows<T, 8>(base, R, stride, kn, sw, lane, hs, norm);
     }
-    wg_partial(red, a.rb);
-    if constexpr (SECOND)
-    {
-        if (!last_workgroup(a.ticket)) return;
-        const double t = wg_total(a.rb.partial, gridDim.x, lane, wave);
-        if (wave == 0)
-            finish_norm(t, lane, a.j, a.tol_sqrt_n, a.norm_out, a.scale_out, a.sizes);
-    }
+    return red;
 }
 
-// The first subtraction and the second product of the classical form that
-// always runs twice, in one pass over the basis: per row r' = r - sum_k h1_k v_k (k order, all K <= C vectors held
-// in registers), stored, and partial_k[g][k] = sum over the rows of
-// workgroup g of v_k r'. Per row this is the arithmetic of gs_sub_kernel
+// The subtraction with the partial rows of |r|^2; in the second pass (SECOND)
+// where that runs, and the last workgroup finishes the norm.
+template <typename T, bool SECOND>
+__global__ __launch_bounds__(kThreads) void gs_sub_kernel(GsArgs a, T* __restrict__ R,
+                                                          const T* __restrict__ basis)
+{
+    if (SECOND && *a.again == 0) return;
+    const double red = gs_sub<T>(a, R, basis);
+    if constexpr (SECOND)
+    {
+        const int lane = threadIdx.x % kWave;
+        const int wave = wave_id();
+        double t;
+        if (grid_total(red, a.rb.partial, a.ticket, lane, wave, t) && wave == 0)
+            finish_norm(t, lane, a.j, a.tol_sqrt_n, a.norm_out, a.scale_out, a.sizes);
+    }
+    else
+        wg_partial(red, a.rb);
+}
+
+// A second pass where |h| > 0.1 of what the first leaves of r (below that r
+// lost at most 0.5 % of its length), whose square is |r|^2 - |h|^2.
+constexpr double kCancelSquared = 1e-2;
+
+// The first subtraction, r' = r - sum_k h_k v_k (k order, all K <= C vectors
+// of a row held in registers), and from the same read of the basis either
+// |r'|^2 or, where the second pass runs, its products partial_k[g][k] = sum
+// over the rows of workgroup g of v_k r'. It runs in FP64 where the first
+// cancels for some probe of the block (a NaN asks for nothing, it would stay
+// one), in FP32 always. Per row this is the arithmetic of gs_sub_kernel
 // followed by gs_dots_kernel (for K > kGsChunk without the rounding of r to
 // T between chunks), with one read of the basis instead of two.
 // C <= 32 runs in 512-thread workgroups (two wavefronts per SIMD: at C =
 // 32 the values, the sums and the addresses take 252 VGPRs); C = 64 in
 // 256-thread workgroups, one wavefront per SIMD with up to 512 VGPRs.
 template <typename T, int C, int WPG>
-__global__ __launch_bounds__(WPG * kWave) void gs_subdots_kernel(GsArgs a, T* __restrict__ R,
-                                                                 const T* __restrict__ basis)
+__global__ __launch_bounds__(WPG * kWave) void gs_first_kernel(GsArgs a, T* __restrict__ R,
+                                                               const T* __restrict__ basis)
 {
     __shared__ double hs[C][kWave];
     __shared__ double red[WPG][8][kWave];
@@ -1953,11 +1964,21 @@ __global__ __launch_bounds__(WPG * kWave) void gs_subdots_kernel(GsArgs a, T* __
     sw.end = a.nrows;
     const int64_t stride = a.slot;
     const int kn = a.K;
+    const double rr = sizeof(T) == 8 ? a.h[kn * kWave + lane] : 0.0;
     for (int i = threadIdx.x; i < C * kWave; i += blockDim.x)
         hs[i / kWave][i % kWave] = i < kn * kWave ? a.h[i] : 0.0;
     __syncthreads();
+    bool more = true;
+    if constexpr (sizeof(T) == 8)
+    {
+        double hh = 0.0;
+#pragma unroll
+        for (int k = 0; k < C; ++k) hh += hs[k][lane] * hs[k][lane];
+        more = a.always || __any(hh > kCancelSquared * (rr - hh));
+        if (blockIdx.x == 0 && threadIdx.x == 0) *a.again = more ? 1 : 0;
+    }
     const T* __restrict__ base = basis + (int64_t) a.last * stride;
-    double acc[C];
+    double acc[C], len = 0.0;
 #pragma unroll
     for (int g = 0; g < C; ++g) acc[g] = 0.0;
 #pragma unroll 1
@@ -1976,8 +1997,26 @@ __global__ __launch_bounds__(WPG * kWave) void gs_subdots_kernel(GsArgs a, T* __
         const T rt = (T) r;
         R[o] = rt;
         const double rd = (double) rt;
+        if (more)
+        {
 #pragma unroll
-        for (int g = 0; g < C; ++g) acc[g] += rd * (double) v[g];
+            for (int g = 0; g < C; ++g) acc[g] += rd * (double) v[g];
+        }
+        else
+            len += rd * rd;
+    }
+    if (!more)
+    {
+        red[wave][0][lane] = len;
+        __syncthreads();
+        if (wave == 0)
+        {
+            double t = 0.0;
+#pragma unroll
+            for (int w = 0; w < WPG; ++w) t += red[w][0][lane];
+            a.rb.partial[(int64_t) blockIdx.x * kWave + lane] = t;
+        }
+        return;
     }
     // workgroup sums, eight vectors at a time through LDS
 #pragma unroll
@@ -1993,19 +2032,63 @@ __global__ __launch_bounds__(WPG * kWave) void gs_subdots_kernel(GsArgs a, T* __
                 double t = 0.0;
 #pragma unroll
                 for (int w = 0; w < WPG; ++w) t += red[w][q][lane];
-                a.partial_k[((int64_t) blockIdx.x * a.K + g0 + q) * kWave + lane] = t;
+                a.partial_k[((int64_t) blockIdx.x * a.rows + g0 + q) * kWave + lane] = t;
             }
         __syncthreads();
     }
 }
 
-// out[k][p] = sum_g partial[g][k][p] in a fixed order; one workgroup per k.
-__global__ __launch_bounds__(kTotalWaves * kWave) void reduce_partials_kernel(
-    const double* __restrict__ partial, int G, int K, double* __restrict__ out)
+// The same in FP64 for more than 64 vectors, in chunks: the subtraction, then
+// where the second pass runs its products over the same rows.
+__global__ __launch_bounds__(kThreads) void gs_first_chunks_kernel(GsArgs a,
+                                                                   double* __restrict__ R,
+                                                                   const double* __restrict__ basis)
+{
+    const int lane = threadIdx.x % kWave;
+    double hh = 0.0;
+#pragma unroll 8
+    for (int k = 0; k < a.K; ++k)
+    {
+        const double h = a.h[(int64_t) k * kWave + lane];
+        hh += h * h;
+    }
+    const bool more =
+        a.always || __any(hh > kCancelSquared * (a.h[(int64_t) a.K * kWave + lane] - hh));
+    if (blockIdx.x == 0 && threadIdx.x == 0) *a.again = more ? 1 : 0;
+    const double red = gs_sub<double>(a, R, basis);
+    if (more) gs_dots<double, false, false>(a, R, basis);
+    else wg_partial(red, a.rb);
+}
+
+// h[k][p] = sum_g partial_k[g][k][p] in a fixed order; one workgroup per k.
+__global__ __launch_bounds__(kTotalWaves * kWave) void gs_total_kernel(GsArgs a, int G, double* h)
 {
     const int k = blockIdx.x;
-    const double t = ordered_total(partial + (int64_t) k * kWave, G, (int64_t) K * kWave);
-    if (threadIdx.x < kWave) out[k * kWave + threadIdx.x] = t;
+    const double t = ordered_total(a.partial_k + (int64_t) k * kWave, G, (int64_t) a.rows * kWave);
+    if (threadIdx.x < kWave) h[k * kWave + threadIdx.x] = t;
+}
+
+// The same for the second pass's products; where that does not run, the norm
+// that gs_first_kernel left in partial rows.
+__global__ __launch_bounds__(kTotalWaves * kWave) void gs_again_kernel(GsArgs a, int G, double* h)
+{
+    const int k = blockIdx.x;
+    const bool more = *a.again != 0;
+    // (the norm's rows are on their way before the flag is here)
+    if (k == 0)
+    {
+        const double t = ordered_total(a.rb.partial, G);
+        if (!more)
+        {
+            if (threadIdx.x < kWave)
+                finish_norm(t, threadIdx.x, a.j, a.tol_sqrt_n, a.norm_out, a.scale_out, a.sizes);
+            return;
+        }
+        __syncthreads();
+    }
+    if (!more) return;
+    const double t = ordered_total(a.partial_k + (int64_t) k * kWave, G, (int64_t) a.rows * kWave);
+    if (threadIdx.x < kWave) h[k * kWave + threadIdx.x] = t;
 }
 
 // Set-up of a recurrence in one launch: scale = s0 and sizes = 0 for every
@@ -2604,12 +2687,12 @@ int gs_grid(int64_t rows, int cap) { return stream_grid(rows, cap); }
 constexpr int kGsTicket = 32;
 constexpr int kGsWords = 64;
 
-// SLQ_FUSED_GS=0: every product and subtraction of two passes by itself
-// (read per call, so a process can compare).
-bool gs_plain()
+// SLQ_FUSED_GS: 0 every product and subtraction of two passes by itself, 2 the
+// second pass in every step (read per call, so a process can compare).
+int gs_mode()
 {
     const char* e = std::getenv("SLQ_FUSED_GS");
-    return e && std::atoi(e) == 0;
+    return e ? std::atoi(e) : 1;
 }
 
 // Gram-Schmidt of r against the K newest basis vectors (slots last, last -
@@ -2629,14 +2712,15 @@ int reorthogonalize(slq_op* op, int64_t nrows, T* R, const T* basis, size_t slot
     g.slot = (int64_t) slot;
     g.last = last;
     g.K = K;
+    g.rows = K + (sizeof(T) == 8 ? 1 : 0);
     g.partial_k = partial_k;
     g.rb = rb;
     g.h = h;
-    g.h_out = h;
     g.alpha = alpha;
+    const int mode = gs_mode();
+    g.always = mode == 2;
     g.again = again;
     g.ticket = (unsigned int*) again + kGsTicket;
-    g.first_rows = G;
     g.j = j;
     g.tol_sqrt_n = tol_sqrt_n;
     g.norm_out = norm_out;
@@ -2650,9 +2734,27 @@ int reorthogonalize(slq_op* op, int64_t nrows, T* R, const T* basis, size_t slot
             hipLaunchKernelGGL((gs_dots_kernel<T, false>), grid, wg, 0, op->stream, g, R,
                                basis);
     };
-    auto reduce = [&]() {
-        hipLaunchKernelGGL(reduce_partials_kernel, dim3(K), tg, 0, op->stream,
-                           (const double*) partial_k, G, K, h);
+    auto reduce = [&](int rows) {
+        hipLaunchKernelGGL(gs_total_kernel, dim3(rows), tg, 0, op->stream, g, G, h);
+    };
+    auto first = [&]() {
+        if (K > 64)
+        {
+            if constexpr (sizeof(T) == 8)
+                hipLaunchKernelGGL(gs_first_chunks_kernel, grid, wg, 0, op->stream, g, R, basis);
+        }
+        else if (K > 32)
+            hipLaunchKernelGGL((gs_first_kernel<T, 64, 4>), grid, dim3(4 * kWave), 0,
+                               op->stream, g, R, basis);
+        else if (K > 16)
+            hipLaunchKernelGGL((gs_first_kernel<T, 32, kWavesPerWG>), grid, wg, 0, op->stream,
+                               g, R, basis);
+        else if (K > 8)
+            hipLaunchKernelGGL((gs_first_kernel<T, 16, kWavesPerWG>), grid, wg, 0, op->stream,
+                               g, R, basis);
+        else
+            hipLaunchKernelGGL((gs_first_kernel<T, 8, kWavesPerWG>), grid, wg, 0, op->stream,
+                               g, R, basis);
     };
     auto sub = [&]() {
         hipLaunchKernelGGL((gs_sub_kernel<T, false>), grid, wg, 0, op->stream, g, R, basis);
@@ -2662,53 +2764,37 @@ int reorthogonalize(slq_op* op, int64_t nrows, T* R, const T* basis, size_t slot
                            (const double*) rb.partial, G, j, tol_sqrt_n, norm_out, scale_out,
                            sizes);
     };
-    // FP32 vectors always take both passes: the error of their results is
-    // that of the vectors' rounding, which leaving a pass out would draw anew
-    const bool always = sizeof(T) == 4;
     if (K == 0)
     {
         sub();
         norm();
     }
-    else if (always && K <= 64 && !gs_plain())
+    else if (mode == 0 || (K > 64 && sizeof(T) == 4))
     {
         dots(alpha != nullptr);
-        reduce();
-        if constexpr (sizeof(T) == 4)
-        {
-            if (K > 32)
-                hipLaunchKernelGGL((gs_subdots_kernel<T, 64, 4>), grid, dim3(4 * kWave), 0,
-                                   op->stream, g, R, basis);
-            else if (K > 16)
-                hipLaunchKernelGGL((gs_subdots_kernel<T, 32, kWavesPerWG>), grid, wg, 0,
-                                   op->stream, g, R, basis);
-            else if (K > 8)
-                hipLaunchKernelGGL((gs_subdots_kernel<T, 16, kWavesPerWG>), grid, wg, 0,
-                                   op->stream, g, R, basis);
-            else
-                hipLaunchKernelGGL((gs_subdots_kernel<T, 8, kWavesPerWG>), grid, wg, 0,
-                                   op->stream, g, R, basis);
-        }
-        reduce();
+        reduce(K);
+        sub();
+        dots(false);
+        reduce(K);
         sub();
         norm();
     }
-    else if (always || gs_plain())
+    else if (sizeof(T) == 4)
     {
+        // FP32 vectors always take both passes
         dots(alpha != nullptr);
-        reduce();
-        sub();
-        dots(false);
-        reduce();
+        reduce(K);
+        first();
+        reduce(K);
         sub();
         norm();
     }
     else
     {
         dots(alpha != nullptr);
-        reduce();
-        sub();
-        hipLaunchKernelGGL(gs_again_kernel<T>, grid, wg, 0, op->stream, g, R, basis);
+        reduce(K + 1);
+        first();
+        hipLaunchKernelGGL(gs_again_kernel, dim3(K), tg, 0, op->stream, g, G, h);
         hipLaunchKernelGGL((gs_sub_kernel<T, true>), grid, wg, 0, op->stream, g, R, basis);
     }
     SLQ_CHECK(hipGetLastError());
