@@ -206,6 +206,9 @@ int build_tiles(int64_t nrows, int64_t ncols, const int64_t* indptr,
 // 0.12 ms for its launches, allocations and copies even of a tiny matrix.
 constexpr int64_t kHostTileNnz = 4096;
 
+// Least part of the slab entries that hold a non-zero in a tiled form.
+constexpr double kTileDensity = 0.25;
+
 // Tiled form of a device CSR whose column order is known (strict): on the
 // device, else on the host from a copy.
 static int tiles_of(hipStream_t s, const DevCSR& c, int R, DevTiles& out)
@@ -213,7 +216,7 @@ static int tiles_of(hipStream_t s, const DevCSR& c, int R, DevTiles& out)
     if (c.strict)
     {
         TileStatus st;
-        SLQ_TRY(device_tiles(s, c, nullptr, R, 0.25, out, nullptr, nullptr, st));
+        SLQ_TRY(device_tiles(s, c, nullptr, R, kTileDensity, out, nullptr, nullptr, st));
         if (st.built) return SLQ_OK;
     }
     const size_t vb = c.dtype == SLQ_F64 ? 8 : 4;
@@ -229,8 +232,8 @@ static int tiles_of(hipStream_t s, const DevCSR& c, int R, DevTiles& out)
                             hipMemcpyDeviceToHost));
         SLQ_CHECK(hipMemcpy(dv.data(), c.data, vb * c.nnz, hipMemcpyDeviceToHost));
     }
-    return build_tiles(c.nrows, c.ncols, ip.data(), ix.data(), dv.data(), c.dtype, R, 0.25,
-                       out);
+    return build_tiles(c.nrows, c.ncols, ip.data(), ix.data(), dv.data(), c.dtype, R,
+                       kTileDensity, out);
 }
 
 PairTiles::~PairTiles()
@@ -313,8 +316,8 @@ int host_pair_tiles(slq_op* op, const DevCSR& ca, const DevCSR& cb, int64_t n, i
     if (!union_pattern(n, ipa, ixa, ipb, ixb, ipu, ixu, ka, kb)) return SLQ_OK;
     std::vector<int32_t> src;
     DevTiles t;
-    SLQ_TRY(build_tiles(n, ca.ncols, ipu.data(), ixu.data(), nullptr, ca.dtype, R, 0.25, t,
-                        &src));
+    SLQ_TRY(build_tiles(n, ca.ncols, ipu.data(), ixu.data(), nullptr, ca.dtype, R, kTileDensity,
+                        t, &src));
     if (t.R == 0) return SLQ_OK;
     if (src.empty())
     {
@@ -378,8 +381,8 @@ int ensure_pair_tiles(slq_op* op, bool need_f32, bool trans)
         if (ca.strict && cb.strict)
         {
             TileStatus st;
-            SLQ_TRY(device_tiles(op->stream, ca, &cb, R, 0.25, ab.tiles, &ab.src_a, &ab.src_b,
-                                 st));
+            SLQ_TRY(device_tiles(op->stream, ca, &cb, R, kTileDensity, ab.tiles, &ab.src_a,
+                                 &ab.src_b, st));
             built = st.built;
         }
         if (!built) SLQ_TRY(host_pair_tiles(op, ca, cb, n, R, ab));
@@ -1755,16 +1758,12 @@ int slq_op_create_csr(int64_t nrows, int64_t ncols, int64_t nnz,
     // here rather than let a kernel read outside its buffers. The columns are
     // looked over on the device; on the host only where that is not done, or
     // to name the column it found.
-    int64_t max_row = 0;
     for (int64_t r = 0; r < nrows; ++r)
-    {
         if (indptr[r + 1] < indptr[r])
         {
             set_error("slq_op_create_csr: indptr decreases at row %lld", (long long) r);
             return SLQ_E_ARG;
         }
-        max_row = std::max(max_row, indptr[r + 1] - indptr[r]);
-    }
     auto check_columns = [&]() -> int {
         for (int64_t k = 0; k < nnz; ++k)
             if (indices[k] < 0 || (int64_t) indices[k] >= ncols)
@@ -1795,7 +1794,6 @@ int slq_op_create_csr(int64_t nrows, int64_t ncols, int64_t nnz,
     c.ncols = ncols;
     c.nnz = nnz;
     c.dtype = dtype;
-    c.max_row = max_row;
     const size_t vb = dtype == SLQ_F64 ? 8 : 4;
     auto fail = [&](int code) {
         if (op->stream) (void) hipStreamDestroy(op->stream);
@@ -1821,11 +1819,14 @@ int slq_op_create_csr(int64_t nrows, int64_t ncols, int64_t nnz,
         const char* env = std::getenv("SLQ_TILE_ROWS");
         const int R = env ? std::atoi(env) : 16;
         TileStatus st;
+        const TileShape shape = tile_shape(nrows, indptr, R == 8 ? 8 : 16);
+        c.max_row = shape.longest;
         st.want_tiles = R == 8 || R == 16;
+        st.rows_known = true;
         int r = SLQ_OK;
-        if (nnz > kHostTileNnz)
-            r = device_tiles(op->stream, c, nullptr, R, 0.25, op->A->tiles, nullptr, nullptr,
-                             st);
+        if (nnz > kHostTileNnz && !shape.long_row())
+            r = device_tiles(op->stream, c, nullptr, R, kTileDensity, op->A->tiles, nullptr,
+                             nullptr, st);
         if (r == SLQ_OK && (!st.checked || st.bad_column)) r = check_columns();
         if (r != SLQ_OK) return fail(r);
         if (st.checked)
@@ -1843,9 +1844,10 @@ int slq_op_create_csr(int64_t nrows, int64_t ncols, int64_t nnz,
                     if (indices[k] <= indices[k - 1]) c.strict = false;
                 }
         }
-        if (st.want_tiles && !st.built)
+        if (st.want_tiles && !st.built && !(c.strict && shape.none(R, kTileDensity)))
         {
-            r = build_tiles(nrows, ncols, indptr, indices, data, dtype, R, 0.25, op->A->tiles);
+            r = build_tiles(nrows, ncols, indptr, indices, data, dtype, R, kTileDensity,
+                            op->A->tiles);
             if (r != SLQ_OK) return fail(r);
         }
     }

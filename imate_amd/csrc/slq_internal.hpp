@@ -145,15 +145,37 @@ void free_tiles(DevTiles& t);
 // repeating the tile's last column) and the values are laid out as the
 // matrix-core SpMM's operands (tile_slot).
 //
+// What the row lengths alone tell of it (of the union of two patterns: their
+// longest rows and all entries).
+struct TileShape {
+    int64_t nnz = 0;
+    int64_t longest = 0;   // entries of the longest row
+    int64_t slabs = 0;     // at least, when no row repeats a column: a tile has
+                           // no fewer than its longest row
+    // too sparse, whatever the columns are
+    bool none(int R, double min_density) const
+    {
+        return (double) nnz < min_density * (double) slabs * R;
+    }
+    // Not for the device: a row takes one of its wavefronts 0.3 us per entry
+    // where others of the tile are searched for them, the host build about 5
+    // ns per entry of the matrix at best. One full row, the last of its tile,
+    // made the device build of 327,672 (5 M) entries 17.5 (302) ms against
+    // 1.5 (22) on the host. (256 entries: 80 us.)
+    __host__ __device__ bool long_row() const { return longest > 256 && longest > nnz / 64; }
+};
+TileShape tile_shape(int64_t nrows, const int64_t* indptr, int R);
+
 // device_tiles builds it on the device for matrices whose rows are sorted
-// without repeats and of at most 2^31 - 1 entries: of `a`, or with `b` of
-// the union of both patterns (values left zero; *src_a and *src_b receive
-// the slot -> CSR position maps of the two in place of out.src). st.checked
-// tells whether the columns were looked at and st.built whether the form was
-// decided; otherwise (unsorted rows, too many entries, no memory for the
-// temporaries) the caller builds on the host.
+// without repeats, with none that is long, and of at most 2^31 - 1 entries:
+// of `a`, or with `b` of the union of both patterns (values left zero; *src_a
+// and *src_b receive the slot -> CSR position maps of the two in place of
+// out.src). st.checked tells whether the columns were looked at and st.built
+// whether the form was decided; otherwise (unsorted rows, a long row, too
+// many entries, no memory for the temporaries) the caller builds on the host.
 struct TileStatus {
     bool want_tiles = true;    // false: only look the columns over
+    bool rows_known = false;   // the caller has looked for a long row
     bool checked = false;
     bool built = false;
     bool bad_column = false;   // a column index out of range
@@ -161,6 +183,7 @@ struct TileStatus {
 };
 int device_tiles(hipStream_t s, const DevCSR& a, const DevCSR* b, int R, double min_density,
                  DevTiles& out, int32_t** src_a, int32_t** src_b, TileStatus& st);
+
 // On the host, for rows in any order; repeated columns are summed.
 // `data` may be null (values left zero); `src_host`, when given, receives
 // the host copy of the slot -> CSR position map (empty if not kept).

@@ -10,7 +10,8 @@
 // over all of them.
 //
 // What bounds it: the latency of the searches (R rows x log2 row length L1
-// loads per entry). The host sort and scatter that this replaces
+// loads per entry), one wavefront to a row, so matrices of a few long rows
+// stay on the host (TileShape). The host sort and scatter that this replaces
 // (build_tiles, still used for rows that are unsorted or repeat a column and
 // for matrices of a few thousand entries) took about 27 ns per entry, 34 of
 // the 36 ms of a logdet of a new 20011-row matrix of 1 M entries; here
@@ -30,6 +31,7 @@ namespace {
 constexpr int kBadColumn = 1;   // column out of range
 constexpr int kDescending = 2;  // columns of a row not ascending
 constexpr int kRepeated = 4;    // a row repeats a column
+constexpr int kLongRow = 8;     // not done: a long row
 
 constexpr int32_t kOpens = INT32_MIN;   // flag bit of `pre`: the entry opens a slab
 
@@ -109,9 +111,14 @@ constexpr int kTileWaves = kTileThreads / kWave;
 template <int R>
 __global__ __launch_bounds__(kTileThreads) void tile_count_kernel(
     int64_t nrows, int64_t ncols, int64_t ntiles, RowSet s0, RowSet s1, int nsets,
-    int32_t* __restrict__ tile_cnt, int* __restrict__ status,
-    unsigned long long* __restrict__ overlap)
+    const TileShape* __restrict__ shape, int32_t* __restrict__ tile_cnt,
+    int* __restrict__ status, unsigned long long* __restrict__ overlap)
 {
+    if (shape && shape->long_row())
+    {
+        if (blockIdx.x == 0 && threadIdx.x == 0) *status = kLongRow;
+        return;
+    }
     __shared__ int cnt[kTileWaves];
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -249,6 +256,31 @@ __global__ __launch_bounds__(kTileThreads) void tile_fill_kernel(
     }
 }
 
+// The shape of one or two patterns (cleared before, with the entries set).
+template <int R>
+__global__ __launch_bounds__(256) void tile_shape_kernel(int64_t nrows, int64_t ntiles, RowSet s0,
+                                                         RowSet s1, int nsets, int64_t nnz,
+                                                         TileShape* __restrict__ shape)
+{
+    const int pad = R == 16 ? 8 : 1;
+    long long longest = 0, slabs = 0;
+    for (int64_t t = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; t < ntiles;
+         t += (int64_t) gridDim.x * blockDim.x)
+    {
+        long long most = 0;
+        for (int64_t r = t * R; r < (t + 1) * R && r < nrows; ++r)
+        {
+            most = max(most, (long long) (s0.indptr[r + 1] - s0.indptr[r]));
+            if (nsets > 1) most = max(most, (long long) (s1.indptr[r + 1] - s1.indptr[r]));
+        }
+        longest = max(longest, most);
+        slabs += (most + pad - 1) / pad * pad;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) shape->nnz = nnz;
+    if (longest) atomicMax((unsigned long long*) &shape->longest, (unsigned long long) longest);
+    if (slabs) atomicAdd((unsigned long long*) &shape->slabs, (unsigned long long) slabs);
+}
+
 struct Temp {
     void* p = nullptr;
     ~Temp()
@@ -279,6 +311,7 @@ int device_tiles_r(hipStream_t s, const DevCSR& a, const DevCSR* b, double min_d
     char* base = (char*) tmp.p;
     unsigned long long* overlap = (unsigned long long*) base;
     int* status = (int*) (base + 8);
+    TileShape* shape = (TileShape*) (base + 16);
     int32_t* cnt = (int32_t*) (base + 256);
     char* p = base + 256 + b_cnt;
     RowSet s0{a.indptr, a.indices, (int32_t*) (p + nsets * b_row), (int32_t*) p};
@@ -288,8 +321,13 @@ int device_tiles_r(hipStream_t s, const DevCSR& a, const DevCSR* b, double min_d
                     (int32_t*) (p + b_row)};
     const dim3 grid((unsigned) std::min<int64_t>(T, 1 << 20));
     SLQ_CHECK(hipMemsetAsync(base, 0, 256, s));
+    if (!st.rows_known)
+        hipLaunchKernelGGL(tile_shape_kernel<R>,
+                           dim3((unsigned) std::min<int64_t>((T + 255) / 256, 1024)), dim3(256), 0,
+                           s, n, T, s0, s1, nsets, a.nnz + (b ? b->nnz : 0), shape);
     hipLaunchKernelGGL(tile_count_kernel<R>, grid, dim3(kTileThreads), 0, s, n, a.ncols, T, s0,
-                       s1, nsets, cnt, status, overlap);
+                       s1, nsets, st.rows_known ? nullptr : (const TileShape*) shape, cnt, status,
+                       overlap);
     SLQ_CHECK(hipGetLastError());
     // status, overlap and the tile counts in one copy
     std::vector<char> host(256 + b_cnt);
@@ -299,6 +337,13 @@ int device_tiles_r(hipStream_t s, const DevCSR& a, const DevCSR* b, double min_d
     unsigned long long both;
     std::memcpy(&both, host.data(), sizeof(both));
     std::memcpy(&flags, host.data() + 8, sizeof(flags));
+    if (flags & kLongRow)
+    {
+        TileShape sh;
+        std::memcpy(&sh, host.data() + 16, sizeof(sh));
+        st.built = sh.none(R, min_density);
+        return SLQ_OK;
+    }
     st.checked = true;
     st.bad_column = (flags & kBadColumn) != 0;
     st.sorted = (flags & kDescending) == 0;
@@ -367,6 +412,22 @@ int device_tiles_r(hipStream_t s, const DevCSR& a, const DevCSR* b, double min_d
 }
 
 }  // namespace
+
+TileShape tile_shape(int64_t nrows, const int64_t* indptr, int R)
+{
+    TileShape sh;
+    sh.nnz = indptr[nrows];
+    const int64_t pad = R == 16 ? 8 : 1;
+    for (int64_t t = 0; t * R < nrows; ++t)
+    {
+        int64_t most = 0;
+        for (int64_t r = t * R; r < std::min<int64_t>((t + 1) * R, nrows); ++r)
+            most = std::max(most, indptr[r + 1] - indptr[r]);
+        sh.longest = std::max(sh.longest, most);
+        sh.slabs += (most + pad - 1) / pad * pad;
+    }
+    return sh;
+}
 
 int device_tiles(hipStream_t s, const DevCSR& a, const DevCSR* b, int R, double min_density,
                  DevTiles& out, int32_t** src_a, int32_t** src_b, TileStatus& st)

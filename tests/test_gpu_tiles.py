@@ -5,6 +5,7 @@ the layouts are the same, so products are equal bit for bit; and against
 numpy (1e-13 / 1e-5 of the largest entry)."""
 
 import ctypes
+import time
 
 import numpy
 import pytest
@@ -156,3 +157,67 @@ def test_bad_column_is_named(gpu_lib):
                                          ctypes.byref(h))
         assert code == _lib.SLQ_E_ARG
         assert 'column index %d out of range at 2' % bad in _lib.last_error()
+
+
+def _bordered(n, full, at, seed):
+    """Tridiagonal with `full` full rows from row `at` on."""
+    rng = numpy.random.default_rng(seed)
+    A = scipy.sparse.diags([4.0 + rng.random(n), rng.random(n - 1),
+                            rng.random(n - 1)], [0, 1, -1], format='lil')
+    for r in range(at, at + full):
+        A[r, :] = rng.standard_normal(n)
+    return A.tocsr()
+
+
+# a full row last in its tile and alone (no tiled form), a tile of full rows
+# (tiled); the transpose and the union take the rows' lengths from the device
+@pytest.mark.parametrize('n', [500, 2000])
+@pytest.mark.parametrize('full,at', [(1, 15), (16, 16), (16, 24)])
+def test_long_rows(gpu_lib, n, full, at):
+    A = _bordered(n, full, at, n)
+    B = _banded(n, n, 9, 3, numpy.float64)
+    h1 = _handle(gpu_lib, A.shape, A.indptr, A.indices, A.data)
+    h2 = _handle(gpu_lib, A.shape, *_shuffled(A, 1))
+    hb = _handle(gpu_lib, B.shape, B.indptr, B.indices, B.data)
+    hab = ctypes.c_void_p()
+    _lib.check(gpu_lib.slq_op_create_affine(h1, hb, ctypes.byref(hab)),
+               'slq_op_create_affine')
+    try:
+        X = numpy.random.default_rng(2).standard_normal((n, 64))
+        for trans, M in ((0, A), (1, A.T.tocsr())):
+            Y1 = _spmm(gpu_lib, h1, 0.0, X, n, trans)
+            Y2 = _spmm(gpu_lib, h2, 0.0, X, n, trans)
+            if _tiled(A, 16) and _tiled(M, 16):
+                assert numpy.array_equal(Y1, Y2)
+            ref = M @ X
+            assert numpy.max(numpy.abs(Y1 - ref)) <= \
+                1e-13 * numpy.max(numpy.abs(ref))
+            ref = ref + 0.75 * ((B.T if trans else B) @ X)
+            Y = _spmm(gpu_lib, hab, 0.75, X, n, trans)
+            assert numpy.max(numpy.abs(Y - ref)) <= \
+                1e-13 * numpy.max(numpy.abs(ref))
+    finally:
+        for h in (hab, h1, h2, hb):
+            gpu_lib.slq_op_destroy(h)
+
+
+def test_cost_of_a_long_row(gpu_lib):
+    # a full row last in its tile takes no longer than first in it: searched
+    # for in the fifteen others by one wavefront, it took 14 times as long
+    n = 65536
+
+    def best(row):
+        E = scipy.sparse.csr_matrix(
+            (numpy.full(n, 1e-6), (numpy.full(n, row), numpy.arange(n))),
+            shape=(n, n))
+        A = (scipy.sparse.diags([4.0, 0.5, 0.5], [0, 1, -1], shape=(n, n)) +
+             E).tocsr()
+        A.sort_indices()
+        times = []
+        for _ in range(5):
+            t0 = time.perf_counter()
+            h = _handle(gpu_lib, A.shape, A.indptr, A.indices, A.data)
+            times.append(time.perf_counter() - t0)
+            gpu_lib.slq_op_destroy(h)
+        return min(times)
+    assert best(15) <= 3.0 * best(0)
