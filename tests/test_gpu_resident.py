@@ -72,6 +72,9 @@ def test_coefficients_equal_block_kernels(gpu_lib, n, k, dtype):
         tol = 1e-11 if dtype == 'float64' else 2e-5
         scale = numpy.max(numpy.abs(a2))
         assert numpy.array_equal(s1, s2)
+        if dtype == 'float32' and n >= 63:
+            # two kernels: the resident one keeps FP64 vectors
+            assert not numpy.array_equal(a1, a2)
         for p in range(64):
             q = s1[p]
             assert numpy.max(numpy.abs(a1[p, :q] - a2[p, :q])) <= tol * scale

@@ -159,6 +159,32 @@ def test_bad_column_is_named(gpu_lib):
         assert 'column index %d out of range at 2' % bad in _lib.last_error()
 
 
+# past a few thousand entries the columns are looked over on the device, with
+# and without tiles to build, and the host names the one found
+@pytest.mark.parametrize('rows', [None, '8', '0'])
+@pytest.mark.parametrize('at', ['first', 'middle', 'last'])
+def test_bad_column_of_a_larger_matrix(gpu_lib, monkeypatch, rows, at):
+    if rows is None:
+        monkeypatch.delenv('SLQ_TILE_ROWS', raising=False)
+    else:
+        monkeypatch.setenv('SLQ_TILE_ROWS', rows)
+    n = 2000
+    A = scipy.sparse.diags([4.0, 0.5, 0.5], [0, 1, -1], shape=(n, n),
+                           format='csr')
+    k = {'first': 0, 'middle': A.nnz // 2, 'last': A.nnz - 1}[at]
+    ip = A.indptr.astype(numpy.int64)
+    for bad in (n, -1, 2**31 - 1):
+        ix = A.indices.astype(numpy.int32)
+        ix[k] = bad
+        h = ctypes.c_void_p()
+        code = gpu_lib.slq_op_create_csr(n, n, A.nnz, _lib.ptr(ip),
+                                         _lib.ptr(ix), _lib.ptr(A.data),
+                                         _lib.SLQ_F64, ctypes.byref(h))
+        assert code == _lib.SLQ_E_ARG
+        assert 'column index %d out of range at %d' % (bad, k) in \
+            _lib.last_error()
+
+
 def _bordered(n, full, at, seed):
     """Tridiagonal with `full` full rows from row `at` on."""
     rng = numpy.random.default_rng(seed)
