@@ -2347,16 +2347,15 @@ int nt_default()
 // which then serves the L2's misses) take blocks of 4 MiB: at 16384 rows of
 // 656 non-zeros over 65536 columns 388 us against 396 / 418 / 458 with 2, 1
 // and 0.5 MiB and 453 for the row kernel; larger ones 1024 columns.
-// SLQ_CSR_BLOCK_COLS sets the block (0 disables).
+// SLQ_CSR_BLOCK_COLS sets the block (0 disables; read per call, so a process
+// can compare).
 constexpr double kCachedOperand = 128.0 * (1 << 20);
 
 template <typename T>
 int csr_blocked_cols(const SpmmArgs<T>& s)
 {
-    static const int env = [] {
-        const char* e = std::getenv("SLQ_CSR_BLOCK_COLS");
-        return e ? std::atoi(e) : -1;
-    }();
+    const char* e = std::getenv("SLQ_CSR_BLOCK_COLS");
+    const int env = e ? std::atoi(e) : -1;
     if (env == 0 || !s.sorted || s.shift_mode == 2 || s.nrows <= 0) return 0;
     const double operand = (double) s.ncols * kBlock * sizeof(T);
     if (operand <= 16.0 * (1 << 20)) return 0;
@@ -2598,7 +2597,10 @@ void launch_spmm_nt(slq_op* op, const SpmmArgs<T>& s, const SpmmIO<T>& io, const
                               : (rw == 8 ? csr_blocked_kernel<T, NT, 8, 8>
                                          : csr_blocked_kernel<T, NT, 8, 4>);
         const int threads = wpg * kWave;
-        if (wpg == 16) grid = (int) std::max<int64_t>(kXcds, ((grid / 2) / kXcds) * kXcds);
+        // (rounded up: rounded down, the 3500 groups of 14000 rows left 44 to a
+        // second sweep of the columns: 1003 us a pair of products with 656
+        // entries a row against 707)
+        if (wpg == 16) grid = (grid / 2 + kXcds - 1) / kXcds * kXcds;
         // (the 8-row kernel holds the more registers)
         static const int resident = [&] {
             int per_cu = 0, cus = 0, dev = 0;

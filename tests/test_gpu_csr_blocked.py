@@ -8,7 +8,9 @@ import numpy
 import pytest
 import scipy.sparse
 
+import imate_amd
 from imate_amd import _lib
+from imate_amd.sample_matrices import sparse_gaussian_device
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +52,29 @@ def test_product(gpu_lib, nrows, dtype):
         assert numpy.all(numpy.abs(Y - ref) <= bound)
     finally:
         gpu_lib.slq_op_destroy(h)
+
+
+def _pair_us(lib, rows, cols, k):
+    """SpMM time of u = A v and v = A^T u together (us), sparse Gaussian A."""
+    D = sparse_gaussian_device(rows, cols, k / cols, seed=1)
+    h = D.gpu_Aop.handle
+    ms = [ctypes.c_double(0), ctypes.c_double(0)]
+    count = [ctypes.c_int64(0), ctypes.c_int64(0)]
+    best = numpy.inf
+    for _ in range(4):
+        _lib.check(lib.slq_profile_enable(h, 1), 'slq_profile_enable')
+        imate_amd.logdet(D, gram=True, method='slq', gpu=True,
+                         lanczos_degree=5, min_num_samples=64,
+                         max_num_samples=64, seed=1)
+        _lib.check(lib.slq_profile_read(
+            h, ctypes.byref(ms[0]), ctypes.byref(count[0]),
+            ctypes.byref(ms[1]), ctypes.byref(count[1])), 'slq_profile_read')
+        best = min(best, 2e3 * ms[0].value / count[0].value)
+    return best
+
+
+def test_a_round_nearly_full_of_rows(gpu_lib):
+    # 3500 groups of four rows, as many as are resident at once: per row as
+    # fast as 4096 groups (a grid rounded down took half as long again)
+    full = _pair_us(gpu_lib, 16384, 65536, 656) / 16384
+    assert _pair_us(gpu_lib, 14000, 65536, 656) / 14000 <= 1.25 * full
