@@ -2340,17 +2340,49 @@ int nt_default()
     return v;
 }
 
+// Rows per wavefront of the blocked CSR SpMM, 8 or 4, or 0 for the row
+// kernel. Every wavefront sweeps all columns once per group of rows, so the
+// groups should fill whole rounds of the resident wavefronts (16 on each of
+// 256 CUs): 16384 rows in groups of 8 left half of the CUs idle (881 us;
+// groups of 4: 458 us at the same block). When neither count fills 85 % of
+// its rounds the row kernel, whose rows are independent, is the faster one
+// while the operand stays in the Infinity Cache.
+constexpr double kCachedOperand = 128.0 * (1 << 20);
+constexpr int64_t kBlkResident = 256 * 16;
+
+template <typename T>
+int csr_blocked_rows(const SpmmArgs<T>& s)
+{
+    auto used = [&](int rows) {
+        const int64_t groups = (s.nrows + rows - 1) / rows;
+        const int64_t rounds = (groups + kBlkResident - 1) / kBlkResident;
+        return (double) groups / (double) (rounds * kBlkResident);
+    };
+    if (used(8) >= 0.85) return 8;
+    if (used(4) >= 0.85) return 4;
+    if ((double) s.ncols * kBlock * sizeof(T) <= kCachedOperand) return 0;
+    return used(8) >= used(4) ? 8 : 4;
+}
+
 // Column block of the blocked CSR SpMM, or 0 for the row-per-wavefront
 // kernel: blocked when the rows are sorted, long (>= 128 non-zeros on
 // average) and the gathered operand is well beyond the L2 (> 16 MiB), and
-// no second (B) stream. Operands up to 128 MiB (half the Infinity Cache,
-// which then serves the L2's misses) take blocks of 4 MiB: at 16384 rows of
-// 656 non-zeros over 65536 columns 388 us against 396 / 418 / 458 with 2, 1
-// and 0.5 MiB and 453 for the row kernel; larger ones 1024 columns.
+// no second (B) stream. A block should hold about ten entries of a row in
+// FP64 (20 in FP32): fewer, and the wavefronts step through blocks instead
+// of gathering; more, and they drift apart within a block, over the rounds
+// of a long sweep and an operand beyond 2^17 columns until the L2 holds no
+// block for all of them. us a pair of products (sparse Gaussian, FP64) by
+// block, and of the row kernel:
+//   rows x columns x a row      row    1024    4096    8192   16384   32768
+//   65536 x 2^18 x 1300        9475    7506    6493    6381    6881    8206
+//   2^18 x 2^18 x 656         22836   22279   14919   16529   16284   17867
+//   2^18 x 2^18 x 160          5686   11641    6938    4966    4634    4922
+//   65536 x 2^20 x 160         1660    4905    2590    2242    2104    1619
+//   2^18 x 2^21 x 160          6369   32398   13182   10195    8831    8308
+// and 2^20 x 2^18 x 2621 in all 6.36 s at 1024, 7.85 at 2048, 9.39 at 8192.
+// Two rounds of rows and operands of up to 2^17 columns take at least 8192.
 // SLQ_CSR_BLOCK_COLS sets the block (0 disables; read per call, so a process
 // can compare).
-constexpr double kCachedOperand = 128.0 * (1 << 20);
-
 template <typename T>
 int csr_blocked_cols(const SpmmArgs<T>& s)
 {
@@ -2361,29 +2393,17 @@ int csr_blocked_cols(const SpmmArgs<T>& s)
     if (operand <= 16.0 * (1 << 20)) return 0;
     if (s.avg_row_nnz < 128.0) return 0;
     if (env > 0) return env;
-    return operand <= kCachedOperand ? (4 << 20) / (int) (kBlock * sizeof(T)) : 1024;
-}
-
-// Rows per wavefront of the blocked CSR SpMM, 8 or 4, or 0 for the row
-// kernel. Every wavefront sweeps all columns once per group of rows, so the
-// groups should fill whole rounds of the resident wavefronts (16 on each of
-// 256 CUs): 16384 rows in groups of 8 left half of the CUs idle (881 us;
-// groups of 4: 458 us at the same block). When neither count fills 85 % of
-// its rounds the row kernel, whose rows are independent, is the faster one
-// while the operand stays in the Infinity Cache.
-template <typename T>
-int csr_blocked_rows(const SpmmArgs<T>& s)
-{
-    auto used = [&](int rows) {
-        const int64_t resident = 256 * 16;
-        const int64_t groups = (s.nrows + rows - 1) / rows;
-        const int64_t rounds = (groups + resident - 1) / resident;
-        return (double) groups / (double) (rounds * resident);
-    };
-    if (used(8) >= 0.85) return 8;
-    if (used(4) >= 0.85) return 4;
-    if ((double) s.ncols * kBlock * sizeof(T) <= kCachedOperand) return 0;
-    return used(8) >= used(4) ? 8 : 4;
+    const int rw = csr_blocked_rows(s);
+    if (rw == 0) return 0;
+    const int entries = sizeof(T) == 8 ? 10 : 20;
+    const int most = 32768;
+    // columns that hold so many entries of a row
+    const double want = entries * (double) s.ncols / s.avg_row_nnz;
+    if (want > (sizeof(T) == 8 ? 2.5 : 1.0) * most) return 0;
+    const int64_t groups = (s.nrows + rw - 1) / rw;
+    int cb = groups <= 2 * kBlkResident || s.ncols <= 1 << 17 ? 8192 : 1024;
+    while (cb < most && cb < 0.75 * want) cb *= 2;
+    return cb;
 }
 
 template <typename T>

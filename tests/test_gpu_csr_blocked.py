@@ -78,3 +78,18 @@ def test_a_round_nearly_full_of_rows(gpu_lib):
     # fast as 4096 groups (a grid rounded down took half as long again)
     full = _pair_us(gpu_lib, 16384, 65536, 656) / 16384
     assert _pair_us(gpu_lib, 14000, 65536, 656) / 14000 <= 1.25 * full
+
+
+def test_blocks_that_hold_few_entries(gpu_lib):
+    # 1024-column blocks of 2^20 columns held 0.16 of a row's 160 entries: four
+    # times the time that the same entries take over 2^17 columns
+    near = _pair_us(gpu_lib, 65536, 1 << 17, 160)
+    assert _pair_us(gpu_lib, 65536, 1 << 20, 160) <= 2.0 * near
+
+
+def test_blocks_that_hold_many_entries(gpu_lib):
+    # eight rounds of rows in 8192-column blocks of 40 entries drifted apart
+    # and took a quarter more per row than two
+    short = _pair_us(gpu_lib, 1 << 16, 1 << 18, 1300) / (1 << 16)
+    assert _pair_us(gpu_lib, 1 << 18, 1 << 18, 1300) / (1 << 18) <= \
+        1.15 * short
