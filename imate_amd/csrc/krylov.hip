@@ -1451,10 +1451,11 @@ int dense_ksplit(int64_t nrows, int64_t ncols)
 // total_kernel (one workgroup) adds the rows of rb.partial in order and
 // stores the total like the SpMM's own reduction.
 constexpr int kTileSumGrid = 256;
-// Partial rows that total_kernel adds by itself: up to here (65536 rows of
-// 16-row tiles) a second launch, 4.7 us however small, costs more than the
-// longer sum.
-constexpr int kTotalRows = 512;
+// Partial rows that total_kernel adds by itself: up to here a second launch,
+// 4.7 us however small, costs more than the longer sum (us a Lanczos step
+// with one launch and with two: 37.7 / 38.4 at 256 rows, 47.6 / 46.7 at 320,
+// 59.4 / 58.5 at 512, 216 / 201 at 2048; a row is 128 matrix rows).
+constexpr int kTotalRows = 256;
 
 __global__ __launch_bounds__(kThreads) void tile_sum_kernel(const double* __restrict__ tp,
                                                             int64_t ntiles,

@@ -44,3 +44,31 @@ def test_product(gpu_lib, c, dtype):
         assert numpy.array_equal(Y[0], Y[1])
     finally:
         gpu_lib.slq_op_destroy(h)
+
+
+# 256 partial rows of 128 matrix rows are added in one launch, more in two
+@pytest.mark.parametrize('n', [32640, 32768, 32770, 33800, 66000])
+def test_total_over_the_tiles(gpu_lib, n):
+    d = numpy.random.default_rng(n).random(n)
+    A = scipy.sparse.diags([2.0 + d] + [-0.1] * 16,
+                           list(range(0, 9)) + list(range(-8, 0)),
+                           shape=(n, n), format='csr')
+    h = ctypes.c_void_p()
+    ip = A.indptr.astype(numpy.int64)
+    _lib.check(gpu_lib.slq_op_create_csr(
+        n, n, A.nnz, _lib.ptr(ip), _lib.ptr(A.indices), _lib.ptr(A.data),
+        _lib.SLQ_F64, ctypes.byref(h)), 'create')
+    Z = numpy.empty((64, n))
+    _lib.check(gpu_lib.slq_rademacher(5, n, 0, 64, _lib.SLQ_F64, _lib.ptr(Z),
+                                      None), 'slq_rademacher')
+    alpha, beta = numpy.zeros((64, 1)), numpy.zeros((64, 1))
+    sizes = numpy.zeros(64, dtype=numpy.int32)
+    try:
+        _lib.check(gpu_lib.slq_recurrences(
+            h, 0.0, 0, 5, 0, 64, 1, 1e-14, 0, 0, _lib.ptr(alpha),
+            _lib.ptr(beta), _lib.ptr(sizes)), 'slq_recurrences')
+        want = numpy.einsum('pi,pi->p', Z, (A @ Z.T).T) / n
+        # sums of n terms of size 1/n, added in parts of 128 rows
+        assert numpy.max(numpy.abs(alpha[:, 0] - want)) <= 1e-13
+    finally:
+        gpu_lib.slq_op_destroy(h)
