@@ -2346,8 +2346,10 @@ int nt_default()
 // groups should fill whole rounds of the resident wavefronts (16 on each of
 // 256 CUs): 16384 rows in groups of 8 left half of the CUs idle (881 us;
 // groups of 4: 458 us at the same block). When neither count fills 85 % of
-// its rounds the row kernel, whose rows are independent, is the faster one
-// while the operand stays in the Infinity Cache.
+// its rounds the row kernel, whose rows are independent, is the faster one;
+// with operands beyond half the Infinity Cache below 70 % (400000 columns,
+// 300 entries a row, us a pair of products blocked and by rows: 862 / 803 at
+// 61 % of 20000 rows, 1543 / 1605 at 81 % of 40000).
 constexpr double kCachedOperand = 128.0 * (1 << 20);
 constexpr int64_t kBlkResident = 256 * 16;
 
@@ -2362,6 +2364,7 @@ int csr_blocked_rows(const SpmmArgs<T>& s)
     if (used(8) >= 0.85) return 8;
     if (used(4) >= 0.85) return 4;
     if ((double) s.ncols * kBlock * sizeof(T) <= kCachedOperand) return 0;
+    if (used(8) < 0.7 && used(4) < 0.7) return 0;
     return used(8) >= used(4) ? 8 : 4;
 }
 
