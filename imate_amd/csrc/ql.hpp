@@ -67,6 +67,13 @@ SLQ_HD inline double ffunc(int func, const double* fp, double x)
     }
 }
 
+// tau of a singular value from the first components of its eigenvectors for
+// +sigma and -sigma (of the 2 k x 2 k Golub-Kahan tridiagonal).
+SLQ_HD inline double pair_weight(double plus, double minus)
+{
+    return copysign(sqrt(plus * plus + minus * minus), plus);
+}
+
 // A node's term tau^2 f(theta^p) of the quadrature. tau, a component of a unit
 // vector, is known to a few eps. Up to kNoWeight it may be zero: the node then
 // belongs to a part of the matrix that the first row does not reach (past a
@@ -193,13 +200,16 @@ SLQ_HD inline void quadrature_one(const QuadArgs& a, const double* alpha,
 
     if (a.gram)
     {
-        // keep the k largest eigenvalues (selection by repeated maximum),
-        // compacted into the first k slots as theta = sigma^2, tau^2 = 2 z^2
-        for (int i = 0; i < k; ++i)
+        // the k largest eigenvalues and, from the most negative up, the k
+        // smallest (selection by repeated maximum and minimum). theta =
+        // sigma^2, and tau^2 is the weight of both: of +sigma and -sigma each
+        // has half, but a zero singular value's two share it arbitrarily
+        for (int i = 0; i < K; ++i)
         {
+            const bool top = i < k;
             int best = i;
             for (int r = i + 1; r < K; ++r)
-                if (d[r * S] > d[best * S]) best = r;
+                if (top ? d[r * S] > d[best * S] : d[r * S] < d[best * S]) best = r;
             const double db = d[best * S], zb = z[best * S];
             d[best * S] = d[i * S];
             z[best * S] = z[i * S];
@@ -210,7 +220,7 @@ SLQ_HD inline void quadrature_one(const QuadArgs& a, const double* alpha,
         {
             const double sg = d[i * S];
             d[i * S] = sg * sg;
-            z[i * S] = sqrt(2.0) * z[i * S];
+            z[i * S] = pair_weight(z[i * S], z[(k + i) * S]);
         }
     }
     if (theta_out)

@@ -16,8 +16,11 @@
 // eigenvectors of each block. The bidiagonal case is solved as the 2k x 2k
 // Golub-Kahan tridiagonal with zero diagonal and off-diagonal (alpha_0,
 // beta_0, alpha_1, ..., alpha_{k-1}), whose eigenvalues are +-sigma_i; the
-// eigenvector of +sigma_i is (v_0, u_0, v_1, u_1, ...)/sqrt(2), so tau_i^2 =
-// 2 z_0^2. The k largest eigenvalues are taken. Matrices past kDcMaxRows
+// eigenvectors of +sigma_i and -sigma_i are (v_0, +-u_0, v_1, +-u_1, ...) /
+// sqrt(2), so tau_i^2 is the sum of both z_0^2, the i-th largest eigenvalue
+// taken with the i-th smallest: for a zero singular value, whose two
+// eigenvectors are any pair of that plane, only the sum is the weight
+// (twice one of them was up to 0.3 off). Matrices past kDcMaxRows
 // rows (their work arrays would not fit the LDS) run the implicit QL of
 // ql.hpp, the host path's solver, one probe per workgroup.
 //
@@ -107,13 +110,16 @@ __global__ __launch_bounds__(NT) void quadrature_dc_kernel(QuadArgs a)
                 const double dj = w.d[j];
                 r += ((a.gram ? dj > di : dj < di) || (dj == di && j < i)) ? 1 : 0;
             }
-            if (r < k)
-            {
-                th[r] = a.gram ? di * di : di;
-                tau[r] = a.gram ? sqrt(2.0) * w.f[i] : w.f[i];
-            }
+            if (r < k) th[r] = a.gram ? di * di : di;
+            // with gram -sigma's behind +sigma's
+            tau[r < k ? r : k + (K - 1 - r)] = w.f[i];
         }
     g.sync();
+    if (ok && a.gram)
+    {
+        for (int i = g.tid; i < k; i += NT) tau[i] = pair_weight(tau[i], tau[k + i]);
+        g.sync();
+    }
     if (a.theta_out)
         for (int i = g.tid; i < a.m; i += NT)
         {

@@ -13,7 +13,7 @@ EPS = numpy.finfo(float).eps
 
 
 def _run(alpha, beta, sizes, gram=0, func=_lib.FUNC_IDENT, params=None,
-         n=1.0):
+         n=1.0, coefficients=None):
     lib = _lib.load()
     count, m = alpha.shape
     q = 1 if params is None else len(params)
@@ -23,7 +23,7 @@ def _run(alpha, beta, sizes, gram=0, func=_lib.FUNC_IDENT, params=None,
     sz = numpy.asarray(sizes, dtype=numpy.int32)
     _lib.check(lib.slq_quadrature(
         _lib.ptr(alpha), _lib.ptr(beta), _lib.ptr(sz), count, m, gram, func,
-        None, 1.0, n, _lib.ptr(params), q, 0 if params is None else 1,
+        _lib.ptr(coefficients), 1.0, n, _lib.ptr(params), q, 0 if params is None else 1,
         _lib.ptr(samples), _lib.ptr(theta), _lib.ptr(tau)), 'slq_quadrature')
     return samples, theta, tau
 
@@ -154,3 +154,21 @@ def test_weights_at_the_rounding_level():
     samples, _, _ = _run(alpha, beta, [0, 0], 0, _lib.FUNC_LOG)
     assert abs(samples[0, 0]) <= 4 * EPS
     assert numpy.isnan(samples[1, 0])
+
+
+# both solvers; a zero and a nearly zero singular value
+@pytest.mark.parametrize('k', [1, 2, 20, 33, 100, 512, 513])
+@pytest.mark.parametrize('low', [0.0, 1e-17, 1e-9])
+def test_zero_singular_values(k, low):
+    rng = numpy.random.default_rng(k)
+    alpha, beta = 1.0 + rng.random((3, k)), 0.3 + 0.5 * rng.random((3, k))
+    for p, at in enumerate((0, k // 2, k - 1)):
+        alpha[p, at] = low
+    samples, theta, tau = _run(alpha, beta, [0, 0, 0], 1, _lib.FUNC_EXP,
+                               coefficients=numpy.array([-1.0]))
+    tol = 8 * EPS * (8 + numpy.sqrt(2 * k))
+    for p in range(3):
+        w, z = _dense(alpha[p], beta[p], 1)
+        want = numpy.sum(z**2 * numpy.exp(-w))
+        assert abs(samples[p, 0] - want) <= tol * max(1.0, numpy.max(w))
+        assert abs(numpy.sum(tau[p]**2) - 1.0) <= tol

@@ -104,27 +104,44 @@ def test_largest_and_smallest_magnitudes(solve):
                 assert not solve(numpy.ones(5), d)[0]
 
 
+def _host_sum(host, alpha, beta, func, gram=0, coefficient=0.0):
+    host.quadrature.restype = ctypes.c_double
+    args = [numpy.ascontiguousarray(x, dtype=float) for x in (alpha, beta)]
+    return host.quadrature(*[x.ctypes.data_as(ctypes.c_void_p) for x in args],
+                           len(alpha), gram, func,
+                           ctypes.c_double(coefficient))
+
+
 @pytest.mark.parametrize('gram', [0, 1])
 @pytest.mark.parametrize('func,want', [(_lib.FUNC_LOG, numpy.log),
                                        (_lib.FUNC_INV, lambda x: 1.0 / x)])
 def test_nodes_of_zero_weight(host, gram, func, want):
     # the second entry is out of the probe's reach and singular
     alpha, beta = numpy.array([2.0, 0.0, 3.0]), numpy.zeros(3)
-    host.quadrature.restype = ctypes.c_double
-    got = host.quadrature(alpha.ctypes.data_as(ctypes.c_void_p),
-                          beta.ctypes.data_as(ctypes.c_void_p), 3, gram, func)
+    got = _host_sum(host, alpha, beta, func, gram)
     assert abs(got - want(4.0 if gram else 2.0)) <= 4 * EPS
-
-
-def _host_logdet(host, alpha, beta):
-    host.quadrature.restype = ctypes.c_double
-    args = [numpy.ascontiguousarray(x, dtype=float) for x in (alpha, beta)]
-    return host.quadrature(*[x.ctypes.data_as(ctypes.c_void_p) for x in args],
-                           len(alpha), 0, _lib.FUNC_LOG)
 
 
 def test_weights_at_the_rounding_level(host):
     # the second node is -9e-32 with tau = 3e-16: log of it is NaN
-    assert _host_logdet(host, [1.0, 0.0], [3e-16, 0.0]) == 0.0
+    assert _host_sum(host, [1.0, 0.0], [3e-16, 0.0], _lib.FUNC_LOG) == 0.0
     # a node of real weight keeps its NaN
-    assert numpy.isnan(_host_logdet(host, [1.0, 0.0], [1e-6, 0.0]))
+    assert numpy.isnan(_host_sum(host, [1.0, 0.0], [1e-6, 0.0],
+                                 _lib.FUNC_LOG))
+
+
+@pytest.mark.parametrize('k', [1, 2, 3, 8, 20, 33])
+@pytest.mark.parametrize('low', [0.0, 1e-17, 1e-9, 0.5])
+def test_zero_singular_values(host, k, low):
+    # exp(-sigma^2) is 1 at a zero singular value, whose weight the two
+    # eigenvectors of the Golub-Kahan tridiagonal share arbitrarily
+    rng = numpy.random.default_rng(k)
+    tol = 8 * EPS * (8 + numpy.sqrt(2 * k))
+    for at in {0, k // 2, k - 1}:
+        alpha, beta = 1.0 + rng.random(k), 0.3 + 0.5 * rng.random(k)
+        alpha[at] = low
+        _, s, vt = numpy.linalg.svd(numpy.diag(alpha) +
+                                    numpy.diag(beta[:k - 1], 1))
+        want = numpy.sum(vt[:, 0]**2 * numpy.exp(-s**2))
+        got = _host_sum(host, alpha, beta, _lib.FUNC_EXP, 1, -1.0)
+        assert abs(got - want) <= tol * max(1.0, s[0]**2)

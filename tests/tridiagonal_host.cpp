@@ -47,7 +47,8 @@ extern "C" int divide_and_conquer(const double* d, const double* e, int K, doubl
 }
 
 // The host path's quadrature of one tridiagonal (gram: bidiagonal).
-extern "C" double quadrature(const double* alpha, const double* beta, int m, int gram, int func)
+extern "C" double quadrature(const double* alpha, const double* beta, int m, int gram, int func,
+                             double coefficient)
 {
     slq::QuadArgs a = {};
     double out = 0.0;
@@ -55,6 +56,7 @@ extern "C" double quadrature(const double* alpha, const double* beta, int m, int
     a.m = m;
     a.gram = gram;
     a.func = func;
+    a.fp[0] = coefficient;
     a.exponent = 1.0;
     a.n = 1.0;
     slq::quadrature_one(a, alpha, beta, 1, 0, work.data(), work.data() + 2 * m,
