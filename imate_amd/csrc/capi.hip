@@ -1758,12 +1758,17 @@ int slq_op_create_csr(int64_t nrows, int64_t ncols, int64_t nnz,
     // here rather than let a kernel read outside its buffers. The columns are
     // looked over on the device; on the host only where that is not done, or
     // to name the column it found.
-    for (int64_t r = 0; r < nrows; ++r)
-        if (indptr[r + 1] < indptr[r])
-        {
-            set_error("slq_op_create_csr: indptr decreases at row %lld", (long long) r);
-            return SLQ_E_ARG;
-        }
+    // 16-row tiles (matrix-core SpMM) unless SLQ_TILE_ROWS asks for 8 or 0
+    // (CSR only)
+    const char* env = std::getenv("SLQ_TILE_ROWS");
+    const int R = env ? std::atoi(env) : 16;
+    int64_t decreasing;
+    const TileShape shape = tile_shape(nrows, indptr, R == 8 ? 8 : 16, decreasing);
+    if (decreasing >= 0)
+    {
+        set_error("slq_op_create_csr: indptr decreases at row %lld", (long long) decreasing);
+        return SLQ_E_ARG;
+    }
     auto check_columns = [&]() -> int {
         for (int64_t k = 0; k < nnz; ++k)
             if (indices[k] < 0 || (int64_t) indices[k] >= ncols)
@@ -1814,12 +1819,7 @@ int slq_op_create_csr(int64_t nrows, int64_t ncols, int64_t nnz,
         (nnz > 0 && (e = hipMemcpy(c.data, data, vb * nnz, hipMemcpyHostToDevice)) != hipSuccess))
         return fail(hip_status(e, "hipMemcpy", __FILE__, __LINE__));
     {
-        // 16-row tiles (matrix-core SpMM) unless SLQ_TILE_ROWS asks for 8 or
-        // 0 (CSR only)
-        const char* env = std::getenv("SLQ_TILE_ROWS");
-        const int R = env ? std::atoi(env) : 16;
         TileStatus st;
-        const TileShape shape = tile_shape(nrows, indptr, R == 8 ? 8 : 16);
         c.max_row = shape.longest;
         st.want_tiles = R == 8 || R == 16;
         st.rows_known = true;

@@ -22,13 +22,13 @@
 // (workgroups per XCD) x (wavefronts per workgroup) units at a time. Units
 // processed concurrently on an XCD are therefore neighbours; on a spatially
 // ordered matrix their gathered operand rows overlap and stay in that XCD's
-// 4 MB L2. The tiled SpMM hands each XCD's tiles out in order from a
-// per-XCD ticket counter instead, for the same locality with dynamic load
-// balance.
+// 4 MB L2. The matrix-core SpMM launches a workgroup per eight tiles, which
+// the hardware deals out in order; its split and 8-row forms draw tiles from
+// a per-XCD ticket counter instead, for the same locality.
 //
 // Reductions (alpha, beta, norms) are per-probe sums over all rows, computed
-// deterministically and without fences: each workgroup (or, in the tiled
-// SpMM, each row tile) writes one partial row, and a following launch of
+// deterministically and without fences: each workgroup (or, in the split and
+// 8-row SpMM, each row tile) writes one partial row, and a following launch of
 // one workgroup adds the rows in a fixed order and finishes the value (the
 // kernel boundary orders the two). The result is bitwise reproducible run
 // to run.
@@ -829,7 +829,7 @@ __device__ __forceinline__ void spmm_epilogue4(const SpmmArgs<T>& a, int64_t row
 // row groups (lanes l, l ^ 16, l ^ 32, l ^ 48), then the workgroup's tiles,
 // in a fixed order; its partial row goes to tile_partial. With a grid capped
 // by the launch settings (CAPPED) a workgroup takes further tiles in steps of
-// the grid; that loop costs the uncapped form's fourth wavefront per SIMD (148
+// the grid; that loop costs the uncapped form's fourth wavefront per SIMD (152
 // against 127 VGPRs), so it has a form of its own.
 constexpr int kSpmmDepth = 3;
 
@@ -2553,8 +2553,8 @@ void launch_spmm_nt(slq_op* op, const SpmmArgs<T>& s, const SpmmIO<T>& io, const
         const T* tv = (sizeof(T) == 4 && op->A->csr.dtype == SLQ_F64)
                           ? (const T*) tl->vals_f32 : (const T*) tl->vals;
         const int grid = grid_for(tl->ntiles, op->spmm_grid);
-        // tiles are handed out in order from the XCD's ticket counter (16-row
-        // tiles on the matrix cores, 8-row tiles on the vector ALUs);
+        // 16-row tiles on the matrix cores, a tile a wavefront; the split and
+        // 8-row forms draw tiles in order from the XCD's ticket counter.
         // launch_spmm has checked the counters and partial rows
         {
             const int split = tl->R == 16 ? spmm_split(op) : 1;

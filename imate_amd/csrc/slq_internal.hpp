@@ -164,7 +164,9 @@ struct TileShape {
     // 1.5 (22) on the host. (256 entries: 80 us.)
     __host__ __device__ bool long_row() const { return longest > 256 && longest > nnz / 64; }
 };
-TileShape tile_shape(int64_t nrows, const int64_t* indptr, int R);
+// From host row pointers (`slabs` only where a row is long); `decreasing`
+// receives the first row whose pointers decrease, or -1.
+TileShape tile_shape(int64_t nrows, const int64_t* indptr, int R, int64_t& decreasing);
 
 // device_tiles builds it on the device for matrices whose rows are sorted
 // without repeats, with none that is long, and of at most 2^31 - 1 entries:

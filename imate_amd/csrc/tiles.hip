@@ -413,17 +413,28 @@ int device_tiles_r(hipStream_t s, const DevCSR& a, const DevCSR* b, double min_d
 
 }  // namespace
 
-TileShape tile_shape(int64_t nrows, const int64_t* indptr, int R)
+TileShape tile_shape(int64_t nrows, const int64_t* indptr, int R, int64_t& decreasing)
 {
     TileShape sh;
     sh.nnz = indptr[nrows];
+    decreasing = -1;
+    for (int64_t r = 0; r < nrows; ++r)
+    {
+        const int64_t len = indptr[r + 1] - indptr[r];
+        if (len < 0)
+        {
+            decreasing = r;
+            return sh;
+        }
+        sh.longest = std::max(sh.longest, len);
+    }
+    if (!sh.long_row()) return sh;
     const int64_t pad = R == 16 ? 8 : 1;
     for (int64_t t = 0; t * R < nrows; ++t)
     {
         int64_t most = 0;
         for (int64_t r = t * R; r < std::min<int64_t>((t + 1) * R, nrows); ++r)
             most = std::max(most, indptr[r + 1] - indptr[r]);
-        sh.longest = std::max(sh.longest, most);
         sh.slabs += (most + pad - 1) / pad * pad;
     }
     return sh;
