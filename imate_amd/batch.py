@@ -4,7 +4,9 @@ imate estimates one operator per call; a user with many matrices loops over
 ``logdet(A_i, method='slq', gpu=True)``. ``slq_batch`` runs them together:
 every kernel of every problem is captured into one hipGraph (one branch per
 problem, so problems of uneven size run side by side) and launched once,
-after an autotuner has picked each problem's launch grid. ``use_graph=False``
+after an autotuner has picked each problem's launch grid. (In a process that had
+another HIP runtime loaded than the library was built for, torch's for
+instance, the problems are queued on streams of their own instead.) ``use_graph=False``
 runs the same kernels problem after problem (the per-problem launch loop it
 is compared against). Many t values of ``A + tI`` need no batching API: one
 ``logdet(AffineMatrixFunction(A), parameters=t, ...)`` call runs one Lanczos

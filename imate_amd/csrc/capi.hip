@@ -1524,6 +1524,22 @@ struct TunedLaunch {
     }
 };
 
+// Whether a batch may be one hipGraph launch: only on the HIP runtime that this
+// library was built for. Under another one of the same soname (torch brings
+// its own, and the one loaded first serves the process) a program that captured,
+// launched and destroyed such graphs over and over ended with a segmentation
+// fault on the host, which is not explained; there the problems are queued
+// on their own streams instead, with the same results. SLQ_BATCH_GRAPH=0 asks
+// for that too (read per call, so a process can compare).
+bool graph_batches()
+{
+    const char* e = std::getenv("SLQ_BATCH_GRAPH");
+    if (e && std::atoi(e) == 0) return false;
+    int version = 0;
+    return hipRuntimeGetVersion(&version) == hipSuccess &&
+           version / 100000 == HIP_VERSION / 100000;
+}
+
 // A valid matrix function: a known code, with coefficients where the code
 // takes them (a positive sigma for the Gaussian).
 bool func_ok(int func, const double* fp)
@@ -1612,7 +1628,24 @@ extern "C" int slq_estimate_batch(slq_op** ops, int32_t count, int32_t func,
     };
     auto enqueue = [&](int i) -> int { return enqueue_blocks(i); };
     double t_run = 0.0;
-    if (use_graph)
+    if (use_graph && !graph_batches())
+    {
+        if (setup_time)
+            *setup_time = std::chrono::duration<double>(std::chrono::steady_clock::now() - c0).count();
+        const auto t0 = std::chrono::steady_clock::now();
+        int r = SLQ_OK;
+        for (int i = 0; i < count && r == SLQ_OK; ++i) r = enqueue(i);
+        // whatever was queued ends before the handles are given back
+        for (int i = 0; i < count; ++i)
+        {
+            const hipError_t ee = hipStreamSynchronize(ops[i]->stream);
+            if (r == SLQ_OK && ee != hipSuccess)
+                r = hip_status(ee, "hipStreamSynchronize", __FILE__, __LINE__);
+        }
+        if (r != SLQ_OK) return r;
+        t_run = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+    }
+    else if (use_graph)
     {
         hipStream_t main = nullptr;
         SLQ_CHECK(hipStreamCreateWithFlags(&main, hipStreamNonBlocking));

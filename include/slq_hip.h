@@ -228,8 +228,10 @@ int slq_estimate_noalloc(slq_op* op, const double* params, int32_t num_inquiries
  * trace[i], error[i] (after the outlier pass) and samples[i][num_samples]
  * (may be NULL). use_graph != 0 captures every kernel of every problem into
  * one hipGraph (one branch per problem, so uneven problems run side by side)
- * and launches it once; use_graph == 0 runs the same kernels problem after
- * problem (a per-problem launch loop). *run_time is the launch-to-completion
+ * and launches it once, or, on another HIP runtime than the library was
+ * built for (one that the process had loaded before it), queues every problem
+ * on its own stream; use_graph == 0 runs the same kernels problem after
+ * problem (a per-problem launch loop). The results are the same bit for bit. *run_time is the launch-to-completion
  * time (s), *setup_time the preparation and capture time before it.
  * Replaces a Python loop of imate.logdet(..., method='slq', gpu=True) calls
  * over separate matrices; imate has no batched entry point. */

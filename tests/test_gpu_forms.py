@@ -42,6 +42,19 @@ def test_batch_graph_equals_loop():
     assert numpy.array_equal(ia['samples'], ib['samples'])
 
 
+@pytest.mark.parametrize('orthogonalize', [0, -1])
+def test_batch_on_streams_equals_graph(monkeypatch, orthogonalize):
+    # what a process gets whose HIP runtime the library was not built for
+    mats = _mats([1200, 400, 3000, 2000, 900])
+    kw = dict(func='log', lanczos_degree=12, num_samples=100, seed=2,
+              orthogonalize=orthogonalize, autotune=False)
+    a, ia = slq_batch(mats, **kw)
+    monkeypatch.setenv('SLQ_BATCH_GRAPH', '0')
+    b, ib = slq_batch(mats, **kw)
+    assert numpy.array_equal(ia['samples'], ib['samples'])
+    assert numpy.array_equal(a, b)
+
+
 def test_batch_float32_mixed():
     mats = _mats([1000, 2500], dtype='float32')
     tr, info = slq_batch(mats, func='log', lanczos_degree=12, num_samples=32,
